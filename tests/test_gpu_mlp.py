@@ -276,3 +276,17 @@ def test_gru_training_fits_a_delayed_sequence_task():
     err = pred.cpu().double().numpy()[1:] - Y[1:, :64]
     assert np.sqrt((err ** 2).mean()) < 0.4
     assert hT.shape == (64, 64)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (63, 15), (64, 16), (65, 17), (1024, 33), (1025, 512), (2048, 2080)])
+def test_bias_grad_over_row_and_column_remainders(M, N):
+    """Column sums at the edges of the 16-column, 64-row, 1024-row passes
+    against FP64; a pairwise FP32 sum of M terms is within M/64 + 6 roundings."""
+    g = torch.Generator().manual_seed(M + N)
+    dZ = torch.randn((M, N), generator=g).cuda()
+    db = torch.full((N + 1,), 7.0, device="cuda")
+    nat.check(nat.lib().dtb_mlp_bias_grad(M, N, dZ.data_ptr(), db.data_ptr(), ctypes_stream()))
+    torch.cuda.synchronize()
+    bound = (M / 64 + 6) * 2.0 ** -24 * dZ.double().abs().sum(0)
+    assert ((db[:N].double() - dZ.double().sum(0)).abs() <= bound).all()
+    assert float(db[N]) == 7.0
