@@ -85,82 +85,241 @@ static int bold_step(int64_t n, const double* par, T* s, T* q, T* v, T* f, const
 // K_ev = wd_ev(last)/c_v/(E-1); innov_ev = y_v + sqrt(sigma) xi_ev - w_ev(last)
 // w += rho innov_ev sum_e' K_e'v wd_e'vs + (1-rho) sum_e' A_ee' wd_e'vs,
 // A_ee' = sum_v innov_ev K_e'v / V.
-__global__ void enkf_mean_kernel(int32_t E, int32_t V, int32_t S, const double* __restrict__ w, double* __restrict__ mean)
+//
+// Two kernels, both bound by latency at the sizes of an assimilation window
+// (256 members, 90 voxels, 10 states: 1.8 MB and 0.13 GFLOP), so the work is
+// spread until no thread walks a long chain of dependent loads:
+//   enkf_voxel_kernel   one workgroup per voxel, one wavefront per state with
+//                       its lanes over the members: ensemble mean,
+//                       deviations, gain, innovation and the local term, all
+//                       sums of one voxel, with one barrier (the gains)
+//   enkf_update_kernel  one workgroup per 16 members x 64 CT states: its 16
+//                       rows of A from the innovations and gains, then the
+//                       global term A wd, both on the FP64 matrix cores
+// 256 x 90 x 10: 9.4 + 17 us.  (Six launches with a thread per output element,
+// each summing over the members or voxels by itself, took 394 us.)
+constexpr int kEnkfWaves = 16;        // wavefronts of the voxel kernel
+constexpr int kEnkfLdsMembers = 4096; // members whose gains stay in LDS (larger ensembles re-read them)
+constexpr int kEnkfRegs = 8;          // members per lane held in registers (up to 512 members)
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__device__ inline double wave_sum_f64(double v)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // (v, s)
-    if (x >= (int64_t)V * S) return;
-    double acc = 0.0;
-    for (int32_t e = 0; e < E; ++e) acc += w[(int64_t)e * V * S + x];
-    mean[x] = acc / E;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
 }
 
-__global__ void enkf_diff_kernel(int32_t E, int32_t V, int32_t S, const double* __restrict__ w,
-                                 const double* __restrict__ mean, double* __restrict__ wd)
+// HELD: at most kEnkfWaves states and 64 kEnkfRegs members, so each wavefront
+// keeps its one state's deviations in registers; else they are read again
+// from wd.  GLDS: the gains are exchanged through LDS, else through tempT.
+template <bool HELD, bool GLDS>
+__global__ __launch_bounds__(64 * kEnkfWaves) void enkf_voxel_kernel(int32_t E, int32_t V, int32_t S,
+                                                                     const double* __restrict__ w, double sigma,
+                                                                     const double* __restrict__ y,
+                                                                     const double* __restrict__ xi, double* wd,
+                                                                     double* tempT, double* __restrict__ innovT,
+                                                                     double* __restrict__ gsum)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= (int64_t)E * V * S) return;
-    wd[x] = w[x] - mean[x % ((int64_t)V * S)];
-}
-
-__global__ void enkf_gain_kernel(int32_t E, int32_t V, int32_t S, const double* __restrict__ w,
-                                 const double* __restrict__ wd, double sigma, const double* __restrict__ y,
-                                 const double* __restrict__ xi, double* __restrict__ temp, double* __restrict__ innov)
-{
-    const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    double c = 0.0;
-    for (int32_t e = 0; e < E; ++e) {
-        const double d = wd[((int64_t)e * V + v) * S + (S - 1)];
-        c += d * d;
+    extern __shared__ double s_gain[]; // [E] gains
+    const int32_t v = blockIdx.x;
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t VS = (int64_t)V * S;
+    double* tv = tempT + (int64_t)v * E;
+    double* iv = innovT + (int64_t)v * E;
+    double* gain = GLDS ? s_gain : tv;
+    double d[kEnkfRegs];
+    for (int32_t s = wid; s < S; s += kEnkfWaves) {
+        const double* src = w + (int64_t)v * S + s;
+        double* dst = wd + (int64_t)v * S + s;
+        const bool last = s == S - 1;
+        double noise[kEnkfRegs];
+        double a = 0.0;
+        if (HELD) {
+#pragma unroll
+            for (int k = 0; k < kEnkfRegs; ++k) {
+                const int32_t e = lane + 64 * k;
+                d[k] = e < E ? src[e * VS] : 0.0;
+                noise[k] = last && e < E ? xi[(int64_t)e * V + v] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < kEnkfRegs; ++k) a += d[k];
+        } else {
+#pragma unroll 8
+            for (int32_t e = lane; e < E; e += 64) a += src[e * VS];
+        }
+        const double mean = wave_sum_f64(a) / E;
+        double q = 0.0;
+        const double yv = y[v], sq = sqrt(sigma);
+        if (HELD) {
+#pragma unroll
+            for (int k = 0; k < kEnkfRegs; ++k) {
+                const int32_t e = lane + 64 * k;
+                if (e >= E) continue;
+                if (last) iv[e] = yv + sq * noise[k] - d[k];
+                d[k] -= mean;
+                dst[e * VS] = d[k];
+                q += d[k] * d[k];
+            }
+        } else {
+#pragma unroll 4
+            for (int32_t e = lane; e < E; e += 64) {
+                const double x = src[e * VS], dx = x - mean;
+                dst[e * VS] = dx;
+                q += dx * dx;
+                if (last) iv[e] = yv + sq * xi[(int64_t)e * V + v] - x;
+            }
+        }
+        if (last) {
+            const double c = wave_sum_f64(q) / (E - 1) + sigma;
+            if (HELD) {
+#pragma unroll
+                for (int k = 0; k < kEnkfRegs; ++k) {
+                    const int32_t e = lane + 64 * k;
+                    if (e >= E) continue;
+                    const double g = d[k] / c / (E - 1);
+                    gain[e] = g;
+                    if (GLDS) tv[e] = g;
+                }
+            } else {
+                for (int32_t e = lane; e < E; e += 64) {
+                    const double g = dst[e * VS] / c / (E - 1);
+                    gain[e] = g;
+                    if (GLDS) tv[e] = g;
+                }
+            }
+        }
     }
-    c = c / (E - 1) + sigma;
-    const double sq = sqrt(sigma);
-    for (int32_t e = 0; e < E; ++e) {
-        const int64_t ev = (int64_t)e * V + v;
-        temp[ev] = wd[ev * S + (S - 1)] / c / (E - 1);
-        innov[ev] = y[v] + sq * xi[ev] - w[ev * S + (S - 1)];
+    __syncthreads();
+    for (int32_t s = wid; s < S; s += kEnkfWaves) {
+        double a = 0.0;
+        if (HELD) {
+#pragma unroll
+            for (int k = 0; k < kEnkfRegs; ++k)
+                if (lane + 64 * k < E) a += gain[lane + 64 * k] * d[k];
+        } else {
+            const double* src = wd + (int64_t)v * S + s; // this lane's own stores
+#pragma unroll 8
+            for (int32_t e = lane; e < E; e += 64) a += gain[e] * src[e * VS];
+        }
+        a = wave_sum_f64(a);
+        if (lane == 0) gsum[(int64_t)v * S + s] = a;
     }
 }
 
-__global__ void enkf_local_kernel(int32_t E, int32_t V, int32_t S, const double* __restrict__ wd,
-                                  const double* __restrict__ temp, double* __restrict__ gsum)
+// w += rho innov gsum + (1 - rho) A wd, A_ef = sum_v innov_ev temp_fv / V.
+// A workgroup of four wavefronts takes 16 members (blockIdx.y) and 64 CT
+// columns of wd (blockIdx.x).  It computes its 16 rows of A, kEnkfChunk
+// members f at a time, into LDS and multiplies them with wd: every workgroup
+// of a row repeats that small product (E x V x 16), which costs less than a
+// launch between the two.  v_mfma_f64_16x16x4: lane l holds A[l % 16][l / 16]
+// and B[l / 16][l % 16]; register r of the result is D[4 r + l / 16][l % 16].
+// The chains of loads bound it, so they are issued in batches ahead of the
+// products: all of a chunk's wd values (CT = 1) before its A is computed, and
+// the gains eight steps at a time.
+// CT = 1 while the workgroups then still fit the device about twice (the
+// columns' loads spread over more of them), else 4 (A repeated less often).
+constexpr int kEnkfChunk = 256;
+constexpr int kEnkfBatch = 8;            // steps of four voxels whose loads are in flight together
+constexpr int kEnkfRow = kEnkfChunk + 4; // LDS row: 16 rows x 4 columns of a fragment fall on distinct banks
+
+template <int CT>
+__global__ __launch_bounds__(256) void enkf_update_kernel(int32_t E, int32_t V, int32_t S, double rho,
+                                                          const double* __restrict__ wd,
+                                                          const double* __restrict__ tempT,
+                                                          const double* __restrict__ innovT,
+                                                          const double* __restrict__ gsum, double* __restrict__ w)
 {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // (v, s)
-    if (x >= (int64_t)V * S) return;
-    const int32_t v = (int32_t)(x / S);
-    double acc = 0.0;
-    for (int32_t e = 0; e < E; ++e) acc += temp[(int64_t)e * V + v] * wd[(int64_t)e * V * S + x];
-    gsum[x] = acc;
+    __shared__ double sA[16 * kEnkfRow];
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int64_t VS = (int64_t)V * S;
+    const int32_t e0 = blockIdx.y * 16;
+    const int64_t x0 = ((int64_t)blockIdx.x * 4 + wid) * 16 * CT;
+    f64x4 acc[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) acc[j] = f64x4{0.0, 0.0, 0.0, 0.0};
+    const int32_t er = min(e0 + lr, E - 1); // rows and columns past the edge repeat the last one and are not stored
+    for (int32_t f0 = 0; f0 < E; f0 += kEnkfChunk) {
+        const int32_t nf = min(kEnkfChunk, E - f0);
+        double bv[CT == 1 ? kEnkfChunk / 4 : 1];
+        if (CT == 1) {
+            const int64_t x = min(x0 + lr, VS - 1);
+#pragma unroll
+            for (int k = 0; k < kEnkfChunk / 4; ++k)
+                bv[k] = 4 * k + lk < nf ? wd[(int64_t)(f0 + 4 * k + lk) * VS + x] : 0.0;
+        }
+        // columns f0 .. f0 + nf of A; wavefront wid takes the 16-column tiles wid, wid + 4, ...
+        f64x4 a4[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a4[j] = f64x4{0.0, 0.0, 0.0, 0.0};
+        for (int32_t v0 = 0; v0 < V; v0 += 4 * kEnkfBatch) {
+            double in[kEnkfBatch], tv[kEnkfBatch][4];
+#pragma unroll
+            for (int u = 0; u < kEnkfBatch; ++u) {
+                const int32_t v = v0 + 4 * u + lk;
+                const int64_t row = (int64_t)min(v, V - 1) * E;
+                const bool ok = v < V;
+                in[u] = ok ? innovT[row + er] : 0.0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int32_t f = f0 + (wid + 4 * j) * 16 + lr;
+                    tv[u][j] = ok && f < E ? tempT[row + f] : 0.0; // columns past the last member are zero
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kEnkfBatch; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    a4[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(in[u], tv[u][j], a4[j], 0, 0, 0);
+        }
+        if (f0 > 0) __syncthreads(); // the chunk before has been used
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int fl = (wid + 4 * j) * 16 + lr;
+                sA[(4 * r + lk) * kEnkfRow + fl] = f0 + fl < E ? a4[j][r] / V : 0.0;
+            }
+        __syncthreads();
+        if (CT == 1) {
+#pragma unroll
+            for (int k = 0; k < kEnkfChunk / 4; ++k) {
+                if (4 * k >= nf) break; // uniform
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(sA[lr * kEnkfRow + 4 * k + lk], bv[k], acc[0], 0, 0, 0);
+            }
+        } else {
+#pragma unroll 8
+            for (int32_t f = 0; f < nf; f += 4) {
+                const double av = sA[lr * kEnkfRow + f + lk];
+                const bool ok = f + lk < nf;
+                const double* src = wd + (int64_t)(f0 + (ok ? f + lk : 0)) * VS;
+                double b4[CT];
+#pragma unroll
+                for (int j = 0; j < CT; ++j) b4[j] = ok ? src[min(x0 + 16 * j + lr, VS - 1)] : 0.0;
+#pragma unroll
+                for (int j = 0; j < CT; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b4[j], acc[j], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+        const int64_t x = x0 + 16 * j + lr;
+        if (x >= VS) continue;
+        const int64_t v = x / S;
+        const double gs = gsum[x];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int32_t e = e0 + 4 * r + lk;
+            if (e < E) w[e * VS + x] += rho * innovT[v * E + e] * gs + (1.0 - rho) * acc[j][r];
+        }
+    }
 }
 
-__global__ void enkf_global_kernel(int32_t E, int32_t V, const double* __restrict__ innov,
-                                   const double* __restrict__ temp, double* __restrict__ A)
-{
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // (e, e')
-    if (x >= (int64_t)E * E) return;
-    const int32_t e = (int32_t)(x / E), f = (int32_t)(x % E);
-    double acc = 0.0;
-    for (int32_t v = 0; v < V; ++v) acc += innov[(int64_t)e * V + v] * temp[(int64_t)f * V + v];
-    A[x] = acc / V;
-}
-
-__global__ void enkf_update_kernel(int32_t E, int32_t V, int32_t S, double rho, const double* __restrict__ wd,
-                                   const double* __restrict__ innov, const double* __restrict__ gsum,
-                                   const double* __restrict__ A, double* __restrict__ w)
-{
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // (e, v, s)
-    if (x >= (int64_t)E * V * S) return;
-    const int64_t vs = x % ((int64_t)V * S);
-    const int32_t e = (int32_t)(x / ((int64_t)V * S));
-    const int32_t v = (int32_t)(vs / S);
-    double acc = 0.0;
-    for (int32_t f = 0; f < E; ++f) acc += A[(int64_t)e * E + f] * wd[(int64_t)f * V * S + vs];
-    w[x] += rho * innov[(int64_t)e * V + v] * gsum[vs] + (1.0 - rho) * acc;
-}
-
-// The six analysis kernels on a caller-chosen scratch of enkf_scratch_doubles
-// doubles: mean [V*S], wd [E*V*S], temp [E*V], innov [E*V], gsum [V*S],
-// A [E*E].  Every scratch element is written before it is read.
+// The analysis on a caller-chosen scratch of enkf_scratch_doubles doubles:
+// wd [E*V*S], the gains and innovations of each voxel [V*E] and gsum [V*S],
+// with room left over.  Every scratch element is written before it is read.
 static size_t enkf_scratch_doubles(int32_t E, int32_t V, int32_t S)
 {
     const size_t EVS = (size_t)E * V * S, VS = (size_t)V * S, EV = (size_t)E * V, EE = (size_t)E * E;
@@ -170,20 +329,28 @@ static size_t enkf_scratch_doubles(int32_t E, int32_t V, int32_t S)
 static int enkf_launch(int32_t E, int32_t V, int32_t S, double* w, double sigma, const double* y, double rho,
                        const double* xi, hipStream_t st, double* scratch)
 {
-    const size_t EVS = (size_t)E * V * S, VS = (size_t)V * S, EV = (size_t)E * V, EE = (size_t)E * E;
-    double* mean = scratch;
-    double* wd = mean + VS;
-    double* temp = wd + EVS;
-    double* innov = temp + EV;
-    double* gsum = innov + EV;
-    double* A = gsum + VS;
-    auto g = [](size_t n) { return dim3((unsigned)std::max<size_t>(1, (n + 255) / 256)); };
-    hipLaunchKernelGGL(enkf_mean_kernel, g(VS), dim3(256), 0, st, E, V, S, w, mean);
-    hipLaunchKernelGGL(enkf_diff_kernel, g(EVS), dim3(256), 0, st, E, V, S, w, mean, wd);
-    hipLaunchKernelGGL(enkf_gain_kernel, g((size_t)V), dim3(256), 0, st, E, V, S, w, wd, sigma, y, xi, temp, innov);
-    hipLaunchKernelGGL(enkf_local_kernel, g(VS), dim3(256), 0, st, E, V, S, wd, temp, gsum);
-    hipLaunchKernelGGL(enkf_global_kernel, g(EE), dim3(256), 0, st, E, V, innov, temp, A);
-    hipLaunchKernelGGL(enkf_update_kernel, g(EVS), dim3(256), 0, st, E, V, S, rho, wd, innov, gsum, A, w);
+    const size_t EVS = (size_t)E * V * S, VS = (size_t)V * S, EV = (size_t)E * V;
+    double* wd = scratch;
+    double* tempT = wd + EVS;
+    double* innovT = tempT + EV;
+    double* gsum = innovT + EV;
+    const dim3 vt(64 * kEnkfWaves);
+    if (E <= 64 * kEnkfRegs && S <= kEnkfWaves)
+        hipLaunchKernelGGL((enkf_voxel_kernel<true, true>), dim3((unsigned)V), vt, sizeof(double) * (size_t)E, st, E, V,
+                           S, w, sigma, y, xi, wd, tempT, innovT, gsum);
+    else if (E <= kEnkfLdsMembers)
+        hipLaunchKernelGGL((enkf_voxel_kernel<false, true>), dim3((unsigned)V), vt, sizeof(double) * (size_t)E, st, E,
+                           V, S, w, sigma, y, xi, wd, tempT, innovT, gsum);
+    else
+        hipLaunchKernelGGL((enkf_voxel_kernel<false, false>), dim3((unsigned)V), vt, 0, st, E, V, S, w, sigma, y, xi,
+                           wd, tempT, innovT, gsum);
+    const size_t rows = ((size_t)E + 15) / 16;
+    if (rows * ((VS + 63) / 64) <= 512)
+        hipLaunchKernelGGL(enkf_update_kernel<1>, dim3((unsigned)((VS + 63) / 64), (unsigned)rows), dim3(256), 0, st, E,
+                           V, S, rho, wd, tempT, innovT, gsum, w);
+    else
+        hipLaunchKernelGGL(enkf_update_kernel<4>, dim3((unsigned)((VS + 255) / 256), (unsigned)rows), dim3(256), 0, st,
+                           E, V, S, rho, wd, tempT, innovT, gsum, w);
     DTB_TRY_HIP(hipGetLastError());
     return DTB_OK;
 }
