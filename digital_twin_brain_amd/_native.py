@@ -105,6 +105,12 @@ SIGNATURES = {
     "dtb_mlp_transpose_bf16": [_i32, _i32, _vp, _vp, _vp],
     "dtb_mlp_f32_to_bf16": [_i64, _vp, _vp, _vp],
     "dtb_mlp_affine": [_i32, _i32, _i32, _vp, _i64, _vp, _vp, _vp, _vp, _i64, _vp],
+    "dtb_mlp_chain_fits": [_i32, _vp, _i32],
+    "dtb_mlp_predict": [_i32, _vp, _i32, _i32, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _i32, _vp, _i64, _vp],
+    "dtb_mlp_train_gradients": [_i32, _vp, _i32, _vp, _i64, _i32, _vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _i64,
+                                _f32, _vp, _vp, _vp],
+    "dtb_mlp_adam_multi": [_i32, _vp, _f32, _f32, _f32, _f32, _i32, _vp],
+    "dtb_mlp_refresh_bf16": [_i32, _vp, _vp],
     "dtb_gru_forward": [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp],
     "dtb_gru_backward": [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
 }
@@ -144,6 +150,8 @@ def exported_symbols():
             "dtb_enkf_analysis_f64", "dtb_enkf_analysis_f64_noalloc",
             "dtb_mlp_gemm_bf16_nt", "dtb_mlp_relu_backward", "dtb_mlp_bias_grad", "dtb_mlp_mse_grad",
             "dtb_mlp_adam", "dtb_mlp_transpose_bf16", "dtb_mlp_f32_to_bf16", "dtb_mlp_affine",
+            "dtb_mlp_chain_fits", "dtb_mlp_predict", "dtb_mlp_train_gradients", "dtb_mlp_adam_multi",
+            "dtb_mlp_refresh_bf16",
             "dtb_gru_forward", "dtb_gru_backward"]
 
 

@@ -11,6 +11,7 @@
 // MFMA operand layout (32x32x16 bf16): lane l holds 8 consecutive K values
 // k = 8*(l/32) .. +7 of row (l % 32) for A and of column (l % 32) for B; the
 // 16 accumulator registers hold C[8*(r/4) + 4*(l/32) + r%4][l % 32].
+#include <algorithm>
 #include <cmath>
 
 #include "dtb_internal.hpp"
@@ -27,6 +28,16 @@ __device__ inline uint16_t f2bf(float f)
     if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40); // NaN stays NaN
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
+}
+
+// two at a time with v_cvt_pk_bf16_f32: the same rounding (and quieting) as f2bf
+__device__ inline uint32_t f2bf_pk(float lo, float hi)
+{
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 h = {(__bf16)lo, (__bf16)hi};
+    uint32_t u;
+    __builtin_memcpy(&u, &h, 4);
+    return u;
 }
 
 __device__ inline float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -367,18 +378,26 @@ __global__ void mse_grad_kernel(int64_t n, const float* __restrict__ out, const 
 }
 
 // Adam (Kingma & Ba, 2015) on FP32 master weights, refreshing the bf16 copy
+__device__ __forceinline__ float adam_update(float w, float gi, float& m, float& v, float lr, float b1, float b2,
+                                             float eps, float c1, float c2)
+{
+    const float mi = b1 * m + (1.0f - b1) * gi;
+    const float vi = b2 * v + (1.0f - b2) * gi * gi;
+    m = mi;
+    v = vi;
+    return w - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+}
+
 __global__ void adam_kernel(int64_t n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
                             float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2,
                             uint16_t* __restrict__ wb)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+    float mi = m[i], vi = v[i];
+    const float wi = adam_update(w[i], g[i], mi, vi, lr, b1, b2, eps, c1, c2);
     m[i] = mi;
     v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     w[i] = wi;
     if (wb) wb[i] = f2bf(wi);
 }
@@ -417,6 +436,660 @@ __global__ void affine_kernel(int32_t rows, int32_t cin, int32_t cout, const flo
     if (c < cin) v = in[(int64_t)r * ldi + c] * (scale ? scale[c] : 1.0f) + (shift ? shift[c] : 0.0f);
     if (out) out[(int64_t)r * ldo + c] = v;
     if (outb) outb[(int64_t)r * ldo + c] = f2bf(v);
+}
+
+// ------------------------------------------------ whole-network MLP kernels
+// A surrogate's layers are small (512 x 512 weights, at most 2,048 rows a
+// batch), so a product per launch leaves the device idle between launches:
+// a training step was 43 launches, a 23,040-row prediction 72.  Rows never
+// mix inside the forward pass or in the chain of activation gradients, so one
+// workgroup takes 32 rows through every layer, with the activations in LDS:
+//   mlp_chain_kernel<false, RT>  normalise, all layers, denormalise (RT x 32 rows)
+//   mlp_chain_kernel<true, 1>  normalise, all layers, loss, and the gradients of
+//                            every layer's output down to the first; writes the
+//                            transposed bf16 operands of the weight gradients
+//                            and each 32-row tile's column sums of the gradients
+//   mlp_dw_kernel            the weight gradients of all layers (contraction
+//                            over the batch) and the bias gradients
+//   adam_multi_kernel        Adam on every parameter, with the bf16 copy and
+//                            its transpose
+// Bound of the chain: each workgroup reads every weight once from its XCD's L2.
+// A CU takes about 110 B/ns that way (one workgroup or 256 streaming at once),
+// 4.7 us for the 512 KB of a 512 x 512 layer, against 1.7 us of matrix work for
+// 32 rows; with the rounding to bf16 and the stores a layer takes 5.5 us.
+// Measured (18 -> 512 x 3 -> 6): a training step of 2,048 rows 210 -> 67 us
+// (chain 45, weight gradients 14, Adam 6.7), 23,040 predicted rows 465 -> 47 us.
+//
+// Every bf16 operand that these kernels read from memory is kept in fragment
+// order: for each 32 rows and 16 columns of a matrix [N][K] the 1 KB that one
+// v_mfma_f32_32x32x16_bf16 takes, lane by lane (frag_at).  A wavefront's load
+// is then 8 whole cache lines; from row-major weights it touched 32 lines for
+// 32 bytes each, and the first form of the chain took 91 us instead of 53 for a
+// 2,048-row batch and 130 instead of 74 for a 23,040-row prediction
+// (18 -> 512 x 3 -> 6).
+//
+// Each product is summed as dtb_mlp_gemm_bf16_nt sums it -- one chain over K
+// where the batch's product has at least 256 64x64 tiles, else four
+// consecutive ranges of K added in order -- so results equal the
+// layer-by-layer launches bit for bit.
+constexpr int kMlpMaxLayers = 8;
+constexpr int kMlpRows = 32;    // rows of a chain workgroup
+constexpr int kMlpWaves = 8;    // two 32-column tiles each of a 512-wide layer
+constexpr int kMlpThreads = 64 * kMlpWaves;
+
+// one chain over K (else four ranges), by the tile count of the whole product
+__host__ __device__ inline bool gemm_one_chain(int32_t M, int32_t N)
+{
+    return (int64_t)((N + 63) / 64) * ((M + 63) / 64) >= 256;
+}
+
+// where element (n, k) of a matrix [N][K] in fragment order is
+__host__ __device__ inline int64_t frag_at(int64_t K, int64_t n, int64_t k)
+{
+    return (n / 32 * (K / 16) + k / 16) * 512 + (k % 16 / 8 * 32 + n % 32) * 8 + k % 8;
+}
+
+// All bf16 arrays in fragment order.
+struct MlpLayerDev {
+    int32_t in, out;       // padded widths (multiples of 32)
+    const uint16_t* w;     // weights [out][in]
+    const uint16_t* wt;    // weights [in][out] (training)
+    const float* bias;     // [out]
+    uint16_t* hT;          // input of the layer [in][B] (training)
+    uint16_t* gT;          // gradient of the layer's output [out][B] (training)
+    float* dbp;            // [B / 32][out] column sums of that gradient per row tile (training)
+};
+
+struct MlpChainArgs {
+    int32_t rows, layers, cin, cout, max_batch, bufw;
+    const float* X;
+    int64_t ldx;
+    const float *xs, *xh;  // input scale and shift
+    const float *ys, *yh;  // prediction: output scale and shift; training: target scale and shift
+    float* out;            // prediction [rows][cout]; training: raw network output [B][last width]
+    int64_t ldo;
+    const float* Y;        // targets [rows][cout] (training)
+    int64_t ldy;
+    const float* mask;     // [rows][cout] or NULL (training)
+    int64_t ldm;
+    float scale;
+    float* lsum;
+    MlpLayerDev l[kMlpMaxLayers];
+};
+
+// tot[i][j] = A[32 i ..][K] W[tile + j][K]^T over steps s0 .. s1 of 16 of this
+// wavefront; A in LDS, W (fragment order, `steps` steps a tile) streamed from
+// L2: blocks of four steps (4 KB a tile), two blocks ahead of their use (one
+// where a block feeds two row tiles), in register buffers taken in turn.  Loads
+// past the end repeat the last block, so that no load sits behind a branch.
+// per > 0: the running sum is folded into tot after every `per` steps, which
+// splits K into consecutive ranges (FOLD 1: per is a multiple of the block, 2:
+// any).
+// SWAP: the operands change places, so a lane holds 16 columns of one row of
+// the result (mfma_row gives the column) instead of 16 rows of one column.
+template <int RT, int TN, int FOLD, bool SWAP>
+__device__ __forceinline__ void chain_gemm(const uint16_t* sA, int lda, const uint16_t* __restrict__ W, int steps,
+                                           int tile, int s0, int s1, int per, f32x16 (&tot)[RT][TN])
+{
+    const int lane = threadIdx.x & 63;
+    const uint16_t* pa = sA + (lane & 31) * lda + (lane >> 5) * 8;
+    const uint16_t* pb[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) pb[j] = W + (int64_t)(tile + j) * steps * 512 + lane * 8;
+    f32x16 acc[RT][TN];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) {
+                acc[i][j][x] = 0.0f;
+                if (FOLD) tot[i][j][x] = -0.0f; // the additive identity: the first fold leaves its sum as it is
+            }
+    int left = per; // steps until the next fold
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int x = 0; x < 16; ++x) {
+                    tot[i][j][x] += acc[i][j][x];
+                    acc[i][j][x] = 0.0f;
+                }
+        left = per;
+    };
+    auto step = [&](int s, const bf16x8 (&b)[TN]) {
+        if (FOLD == 2 && left == 0) fold();
+        --left;
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            const bf16x8 av = *reinterpret_cast<const bf16x8*>(pa + 32 * i * lda + 16 * s);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = SWAP ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], av, acc[i][j], 0, 0, 0)
+                                 : __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    const int nb = (s1 - s0) >> 2; // whole blocks
+    if (nb > 0) {
+        constexpr int D = RT == 1 ? 3 : 2; // register buffers
+        bf16x8 buf[D][4][TN];
+        auto load = [&](bf16x8 (&d)[4][TN], int blk) {
+            const int s = s0 + 4 * min(blk, nb - 1);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) d[u][j] = *reinterpret_cast<const bf16x8*>(pb[j] + (s + u) * 512);
+        };
+#pragma unroll
+        for (int q = 0; q + 1 < D; ++q) load(buf[q], q);
+        for (int blk = 0; blk < nb; blk += D) {
+#pragma unroll
+            for (int q = 0; q < D; ++q) {
+                if (blk + q >= nb) break; // uniform
+                load(buf[(q + D - 1) % D], blk + q + D - 1);
+                if (FOLD == 1 && left <= 0) fold();
+#pragma unroll
+                for (int u = 0; u < 4; ++u) step(s0 + 4 * (blk + q) + u, buf[q][u]);
+            }
+        }
+    }
+    for (int s = s0 + 4 * nb; s < s1; ++s) {
+        bf16x8 b[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const bf16x8*>(pb[j] + s * 512);
+        if (FOLD == 1 && left <= 0) fold();
+        step(s, b);
+    }
+    if (FOLD) fold();
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            if (!FOLD) tot[i][j] = acc[i][j];
+}
+
+// A split K takes the row tiles one after the other (its second accumulator
+// would not leave registers for two), reading the weights again.
+template <int RT, int TN, bool SWAP, typename F>
+__device__ __forceinline__ void chain_tiles(const uint16_t* sA, int lda, const uint16_t* __restrict__ W, int steps,
+                                            int tile, int per, F epi)
+{
+    if (per == 0) {
+        f32x16 acc[RT][TN];
+        chain_gemm<RT, TN, 0, SWAP>(sA, lda, W, steps, tile, 0, steps, 0, acc);
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) epi(i, tile + j, acc[i][j]);
+        return;
+    }
+    for (int i = 0; i < RT; ++i) {
+        f32x16 acc[1][TN];
+        if (per % 4 == 0) chain_gemm<1, TN, 1, SWAP>(sA + 32 * i * lda, lda, W, steps, tile, 0, steps, per, acc);
+        else chain_gemm<1, TN, 2, SWAP>(sA + 32 * i * lda, lda, W, steps, tile, 0, steps, per, acc);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) epi(i, tile + j, acc[0][j]);
+    }
+}
+
+// The product A[32 RT][K] W[N][K]^T of a workgroup: epi(row tile, tile, acc)
+// for every 32-column tile, called by the wavefront that holds it: the
+// neighbouring tiles 2 wid and 2 wid + 1 (which share their reads of A), then
+// 16 further.  A single tile with split K spreads the four ranges over four
+// wavefronts for each row tile (`red`: RT x 3 x 16 x 64 floats of LDS).
+template <int RT, bool SWAP, typename F>
+__device__ __forceinline__ void chain_layer(const uint16_t* sA, int lda, const uint16_t* __restrict__ W, int N, int K,
+                                            bool one_chain, float* red, F epi)
+{
+    static_assert(RT <= kMlpWaves / 4, "one wavefront per row tile and range");
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int steps = K / 16;
+    const int per = one_chain ? 0 : (steps + 3) / 4;
+    if (N == 32 && !one_chain) {
+        f32x16 acc[1][1];
+#pragma unroll
+        for (int x = 0; x < 16; ++x) acc[0][0][x] = 0.0f;
+        const int rt = wid >> 2, q = wid & 3; // row tile, range
+        if (rt < RT) {
+            const int sb = min(q * per, steps), se = min((q + 1) * per, steps);
+            if (sb < se) chain_gemm<1, 1, 0, SWAP>(sA + 32 * rt * lda, lda, W, steps, 0, sb, se, 0, acc);
+            if (q > 0) {
+#pragma unroll
+                for (int x = 0; x < 16; ++x) red[((rt * 3 + q - 1) * 16 + x) * 64 + lane] = acc[0][0][x];
+            }
+        }
+        __syncthreads();
+        if (rt < RT && q == 0) {
+#pragma unroll
+            for (int w = 0; w < 3; ++w)
+#pragma unroll
+                for (int x = 0; x < 16; ++x) acc[0][0][x] += red[((rt * 3 + w) * 16 + x) * 64 + lane];
+        }
+        __syncthreads(); // red may be where epi writes
+        if (rt < RT && q == 0) epi(rt, 0, acc[0][0]);
+        return;
+    }
+    const int tiles = N / 32;
+    for (int tile = 2 * wid; tile < tiles; tile += 2 * kMlpWaves) {
+        if (tile + 1 < tiles) chain_tiles<RT, 2, SWAP>(sA, lda, W, steps, tile, per, epi);
+        else chain_tiles<RT, 1, SWAP>(sA, lda, W, steps, tile, per, epi);
+    }
+}
+
+// the 16 rows of a 32x32 tile that a lane's accumulator holds
+__device__ inline int mfma_row(int x, int lane) { return 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3); }
+
+// a tile's values rounded to bf16 in row pairs (h), and into LDS [32][ld] at column c
+__device__ inline void put_tile(const float (&v)[16], uint32_t (&h)[8], uint16_t* dst, int ld, int c, int lane)
+{
+#pragma unroll
+    for (int x = 0; x < 8; ++x) h[x] = f2bf_pk(v[2 * x], v[2 * x + 1]);
+    uint16_t* p = dst + 4 * (lane >> 5) * ld + c;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) p[mfma_row(x, 0) * ld] = (uint16_t)(h[x >> 1] >> (16 * (x & 1)));
+}
+
+// store them (rows row0 .. row0 + 31 of column c) into [..][B] in fragment
+// order, four rows (8 bytes) at a time: 2 KB of a tile contiguous
+__device__ inline void store_transposed(uint16_t* __restrict__ T, int64_t B, int c, int row0, int lane,
+                                        const uint32_t (&h)[8])
+{
+    uint16_t* p = T + frag_at(B, c, row0) + 4 * (lane >> 5);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<uint2*>(p + (q >> 1) * 512 + (q & 1) * 256) = make_uint2(h[2 * q], h[2 * q + 1]);
+}
+
+template <bool TRAIN, int RT>
+__global__ __launch_bounds__(kMlpThreads) void mlp_chain_kernel(MlpChainArgs a)
+{
+    constexpr int kRows = 32 * RT;
+    extern __shared__ __align__(16) uint16_t smem[];
+    const int t = threadIdx.x, lane = t & 63;
+    // the last rows first: they may be a short batch whose products are split,
+    // which takes longer
+    const int row0 = (TRAIN ? blockIdx.x : gridDim.x - 1 - blockIdx.x) * kRows;
+    // batch of max_batch rows this tile belongs to: its padded size decides how products are summed
+    const int c0 = row0 / a.max_batch * a.max_batch;
+    const int B = (min(a.max_batch, a.rows - c0) + 31) / 32 * 32;
+    uint16_t* cur = smem;                       // activations or gradients [32 RT][bufw]
+    uint16_t* nxt = smem + kRows * a.bufw;
+    uint16_t* smask = smem + 2 * kRows * a.bufw; // [hidden tiles][64]: which of a lane's 16 outputs were > 0
+    const int ld = a.bufw;
+    const int I = a.l[0].in;
+    for (int x = t; x < kRows * I; x += kMlpThreads) {
+        const int r = x / I, c = x % I;
+        float v = 0.0f;
+        if (c < a.cin && row0 + r < a.rows)
+            v = a.X[(int64_t)(row0 + r) * a.ldx + c] * (a.xs ? a.xs[c] : 1.0f) + (a.xh ? a.xh[c] : 0.0f);
+        cur[r * ld + c] = f2bf(v);
+    }
+    __syncthreads();
+    if (TRAIN) {
+        for (int x = t; x < I * 8; x += kMlpThreads) { // eight groups of four rows per column
+            const int c = x >> 3, q = (x & 7) * 4;
+            *reinterpret_cast<ushort4*>(a.l[0].hT + frag_at(B, c, row0 + q)) =
+                make_ushort4(cur[q * ld + c], cur[(q + 1) * ld + c], cur[(q + 2) * ld + c], cur[(q + 3) * ld + c]);
+        }
+    }
+    int mbase = 0; // hidden tiles of the layers before
+    for (int l = 0; l + 1 < a.layers; ++l) {
+        const MlpLayerDev& L = a.l[l];
+        uint16_t* hT = TRAIN ? a.l[l + 1].hT : nullptr;
+        chain_layer<RT, !TRAIN>(
+            cur, ld, L.w, L.out, L.in, gemm_one_chain(B, L.out), reinterpret_cast<float*>(nxt),
+            [&](int rt, int tile, const f32x16& acc) {
+                if (!TRAIN) { // a lane holds four runs of four columns of one row: 8-byte stores
+                    const int c = tile * 32 + 4 * (lane >> 5);
+                    uint16_t* p = nxt + (32 * rt + (lane & 31)) * ld + c;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 bv = *reinterpret_cast<const float4*>(L.bias + c + 8 * q);
+                        float v[4] = {acc[4 * q] + bv.x, acc[4 * q + 1] + bv.y, acc[4 * q + 2] + bv.z,
+                                      acc[4 * q + 3] + bv.w};
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) v[x] = v[x] > 0.0f ? v[x] : 0.0f;
+                        *reinterpret_cast<uint2*>(p + 8 * q) = make_uint2(f2bf_pk(v[0], v[1]), f2bf_pk(v[2], v[3]));
+                    }
+                    return;
+                }
+                const int c = tile * 32 + (lane & 31);
+                const float bv = L.bias[c];
+                float v[16];
+                uint32_t m = 0;
+#pragma unroll
+                for (int x = 0; x < 16; ++x) {
+                    v[x] = acc[x] + bv;
+                    v[x] = v[x] > 0.0f ? v[x] : 0.0f;
+                    if (v[x] > 0.0f) m |= 1u << x;
+                }
+                uint32_t h[8];
+                put_tile(v, h, nxt, ld, c, lane);
+                smask[(mbase + tile) * 64 + lane] = (uint16_t)m;
+                store_transposed(hT, B, c, row0, lane, h);
+            });
+        __syncthreads();
+        mbase += L.out / 32;
+        uint16_t* sw = cur;
+        cur = nxt;
+        nxt = sw;
+    }
+    const MlpLayerDev& LL = a.l[a.layers - 1];
+    if (!TRAIN) {
+        chain_layer<RT, true>(cur, ld, LL.w, LL.out, LL.in, gemm_one_chain(B, LL.out), reinterpret_cast<float*>(nxt),
+                              [&](int rt, int tile, const f32x16& acc) {
+                                  const int row = row0 + 32 * rt + (lane & 31);
+                                  if (row >= a.rows) return;
+#pragma unroll
+                                  for (int x = 0; x < 16; ++x) {
+                                      const int c = tile * 32 + mfma_row(x, lane);
+                                      if (c >= a.cout) continue;
+                                      const float sc = a.ys ? a.ys[c] : 1.0f, sh = a.yh ? a.yh[c] : 0.0f;
+                                      a.out[(int64_t)row * a.ldo + c] = (acc[x] + LL.bias[c]) * sc + sh;
+                                  }
+                              });
+        return;
+    }
+    static_assert(!TRAIN || RT == 1, "the training kernel takes 32 rows");
+    // output and its gradient
+    const int no = LL.out;
+    auto residual = [&](int row, int c, float o) { // mask * (out - target)
+        float tgt = 0.0f, mk = 0.0f;
+        if (c < a.cout && row < a.rows) {
+            tgt = a.Y[(int64_t)row * a.ldy + c] * (a.ys ? a.ys[c] : 1.0f) + (a.yh ? a.yh[c] : 0.0f);
+            mk = a.mask ? a.mask[(int64_t)row * a.ldm + c] : 1.0f;
+        }
+        return (o - tgt) * mk;
+    };
+    chain_layer<RT, false>(cur, ld, LL.w, no, LL.in, gemm_one_chain(B, no), reinterpret_cast<float*>(nxt),
+                           [&](int, int tile, const f32x16& acc) {
+                               const int c = tile * 32 + (lane & 31);
+                               const float bv = LL.bias[c];
+                               float g[16];
+                               float colsum = 0.0f;
+#pragma unroll
+                               for (int x = 0; x < 16; ++x) {
+                                   const int row = row0 + mfma_row(x, lane);
+                                   const float o = acc[x] + bv;
+                                   a.out[(int64_t)row * a.ldo + c] = o;
+                                   g[x] = a.scale * residual(row, c, o);
+                                   colsum += g[x];
+                               }
+                               uint32_t h[8];
+                               put_tile(g, h, nxt, ld, c, lane);
+                               store_transposed(LL.gT, B, c, row0, lane, h);
+                               colsum += __shfl_xor(colsum, 32);
+                               if (lane < 32) LL.dbp[(int64_t)blockIdx.x * no + c] = colsum;
+                           });
+    __syncthreads();
+    // loss: squared errors in runs of 256 consecutive elements of [B][width]
+    for (int k = t >> 6; k < no / 8; k += kMlpWaves) {
+        float e = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int x = k * 256 + u * 64 + lane, row = row0 + x / no, c = x % no;
+            const float d = residual(row, c, a.out[(int64_t)row * a.ldo + c]);
+            e += d * d;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+        if (lane == 0) a.lsum[(int64_t)blockIdx.x * (no / 8) + k] = e;
+    }
+    {
+        uint16_t* sw = cur;
+        cur = nxt;
+        nxt = sw;
+    }
+    // the gradient of each hidden output, masked by its sign
+    for (int l = a.layers - 1; l > 0; --l) {
+        const MlpLayerDev& L = a.l[l];
+        const MlpLayerDev& P = a.l[l - 1];
+        mbase -= L.in / 32;
+        chain_layer<RT, false>(cur, ld, L.wt, L.in, L.out, gemm_one_chain(B, L.in), reinterpret_cast<float*>(nxt),
+                    [&](int rt, int tile, const f32x16& acc) {
+                        const int c = tile * 32 + (lane & 31);
+                        const uint32_t m = smask[(mbase + tile) * 64 + lane];
+                        float g[16];
+                        float colsum = 0.0f;
+#pragma unroll
+                        for (int x = 0; x < 16; ++x) {
+                            g[x] = m >> x & 1u ? acc[x] + 0.0f : 0.0f;
+                            colsum += g[x];
+                        }
+                        uint32_t h[8];
+                        put_tile(g, h, nxt, ld, c, lane);
+                        store_transposed(P.gT, B, c, row0, lane, h);
+                        colsum += __shfl_xor(colsum, 32);
+                        if (lane < 32) P.dbp[(int64_t)blockIdx.x * L.in + c] = colsum;
+                    });
+        __syncthreads();
+        uint16_t* sw = cur;
+        cur = nxt;
+        nxt = sw;
+    }
+}
+
+// Weight and bias gradients of every layer.  Workgroups [first[l], first[l+1])
+// take layer l: a 64x64 tile of dW = G^T H each (both operands [width][B] in
+// fragment order, K = B), K split in four ranges over the wavefronts and added in
+// order (or walked as one chain by each wavefront for its own quarter of the
+// tile, where dtb_mlp_gemm_bf16_nt would); the workgroups of the first tile
+// column also add the row tiles' column sums into db.
+struct MlpDwArgs {
+    int32_t layers, B;
+    int32_t first[kMlpMaxLayers + 1];
+    int32_t in[kMlpMaxLayers], out[kMlpMaxLayers];
+    const uint16_t* hT[kMlpMaxLayers];
+    const uint16_t* gT[kMlpMaxLayers];
+    const float* dbp[kMlpMaxLayers];
+    float* dW[kMlpMaxLayers];
+    float* db[kMlpMaxLayers];
+};
+
+__global__ __launch_bounds__(256) void mlp_dw_kernel(MlpDwArgs a)
+{
+    __shared__ float red[2][64][64]; // two wavefronts' partial tiles at a time: [register][lane]
+    __shared__ float dred[4][64];
+    int l = 0;
+    while (l + 1 < a.layers && (int)blockIdx.x >= a.first[l + 1]) ++l;
+    const int M = a.out[l], N = a.in[l], B = a.B;
+    const int tn = (N + 63) / 64;
+    const int tile = blockIdx.x - a.first[l];
+    const int m0 = tile / tn * 64, n0 = tile % tn * 64;
+    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = lane & 31;
+    const bool one = gemm_one_chain(M, N);
+    const int per = (B / 16 + 3) / 4 * 16;
+    const int kb = one ? 0 : min(wid * per, B), ke = one ? B : min((wid + 1) * per, B);
+    const uint16_t *pa[2], *pb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) { // a sub-tile past the edge repeats the last one and is not stored
+        pa[i] = a.gT[l] + (int64_t)min(m0 + 32 * i, M - 32) * B + lane * 8;
+        pb[i] = a.hT[l] + (int64_t)min(n0 + 32 * i, N - 32) * B + lane * 8;
+    }
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
+    if (one) {
+        // wavefront (wid / 2, wid % 2) walks all of K for one 32x32 sub-tile
+        const uint16_t* qa = pa[wid >> 1];
+        const uint16_t* qb = pb[wid & 1];
+#pragma unroll 4
+        for (int k = 0; k < B; k += 16)
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                *reinterpret_cast<const bf16x8*>(qa + (int64_t)k * 32),
+                *reinterpret_cast<const bf16x8*>(qb + (int64_t)k * 32), acc[0][0], 0, 0, 0);
+        const int ms = m0 + 32 * (wid >> 1), ns = n0 + 32 * (wid & 1);
+        if (ms < M && ns < N) {
+#pragma unroll
+            for (int x = 0; x < 16; ++x)
+                a.dW[l][(int64_t)(ms + mfma_row(x, lane)) * N + ns + r] = acc[0][0][x] + 0.0f;
+        }
+    } else {
+        bf16x8 ca[4][2], cb[4][2], xa[4][2], xb[4][2];
+        auto load = [&](bf16x8 (&da)[4][2], bf16x8 (&db)[4][2], int k) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k + 16 * u < ke) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        da[u][i] = *reinterpret_cast<const bf16x8*>(pa[i] + (int64_t)(k + 16 * u) * 32);
+                        db[u][i] = *reinterpret_cast<const bf16x8*>(pb[i] + (int64_t)(k + 16 * u) * 32);
+                    }
+                }
+        };
+        load(ca, cb, kb);
+        for (int k = kb; k < ke; k += 64) {
+            if (k + 64 < ke) load(xa, xb, k + 64);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (k + 16 * u >= ke) break; // uniform
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ca[u][i], cb[u][j], acc[i][j], 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    ca[u][i] = xa[u][i];
+                    cb[u][i] = xb[u][i];
+                }
+        }
+        // wavefronts 1 and 2, then 3, hand their tiles to wavefront 0, which adds them in order
+        if (wid == 1 || wid == 2) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int x = 0; x < 16; ++x) red[wid - 1][q * 16 + x][lane] = acc[q >> 1][q & 1][x];
+        }
+        __syncthreads();
+        if (wid == 0) {
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) acc[q >> 1][q & 1][x] += red[w][q * 16 + x][lane];
+        }
+        __syncthreads();
+        if (wid == 3) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int x = 0; x < 16; ++x) red[0][q * 16 + x][lane] = acc[q >> 1][q & 1][x];
+        }
+        __syncthreads();
+        if (wid == 0) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int ms = m0 + 32 * (q >> 1), ns = n0 + 32 * (q & 1);
+                if (ms >= M || ns >= N) continue;
+#pragma unroll
+                for (int x = 0; x < 16; ++x)
+                    a.dW[l][(int64_t)(ms + mfma_row(x, lane)) * N + ns + r] =
+                        acc[q >> 1][q & 1][x] + red[0][q * 16 + x][lane] + 0.0f;
+            }
+        }
+    }
+    if (tile % tn == 0) {
+        const int c = m0 + lane;
+        float s = 0.0f;
+        if (c < M) {
+#pragma unroll 8
+            for (int k = wid; k < B / 32; k += 4) s += a.dbp[l][(int64_t)k * M + c];
+        }
+        dred[wid][lane] = s;
+        __syncthreads();
+        if (wid == 0 && c < M) a.db[l][c] = (dred[0][lane] + dred[1][lane]) + (dred[2][lane] + dred[3][lane]);
+    }
+}
+
+// Adam (UPDATE) on a list of parameter tensors [rows][cols] in one launch:
+// 32x32 tiles, tile q of tensor i for first[i] <= q < first[i + 1].  The bf16
+// copies are written with the update, through LDS: row-major (wb), transposed
+// (wt), and in fragment order (wf, and wtf of the transpose; rows and cols
+// multiples of 32), a tile of which is 2 KB contiguous.
+constexpr int kAdamMax = 2 * kMlpMaxLayers;
+struct AdamMultiArgs {
+    int32_t n;
+    int32_t first[kAdamMax + 1];
+    int32_t rows[kAdamMax], cols[kAdamMax];
+    float* w[kAdamMax];
+    const float* g[kAdamMax];
+    float* m[kAdamMax];
+    float* v[kAdamMax];
+    uint16_t* wb[kAdamMax];
+    uint16_t* wt[kAdamMax];
+    uint16_t* wf[kAdamMax];
+    uint16_t* wtf[kAdamMax];
+    float lr, b1, b2, eps, c1, c2;
+};
+
+template <bool UPDATE>
+__global__ __launch_bounds__(256) void adam_multi_kernel(AdamMultiArgs a)
+{
+    __shared__ uint16_t tb[32][34];
+    int i = 0;
+    while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+    const int R = a.rows[i], C = a.cols[i], tc = (C + 31) / 32;
+    const int tile = blockIdx.x - a.first[i];
+    const int r0 = tile / tc * 32, c0 = tile % tc * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    float w[4], g[4], m[4], v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = r0 + ty + 8 * u, c = c0 + tx;
+        if (r >= R || c >= C) continue;
+        const int64_t x = (int64_t)r * C + c;
+        w[u] = a.w[i][x];
+        if (UPDATE) {
+            g[u] = a.g[i][x];
+            m[u] = a.m[i][x];
+            v[u] = a.v[i][x];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = r0 + ty + 8 * u, c = c0 + tx;
+        if (r >= R || c >= C) continue;
+        const int64_t x = (int64_t)r * C + c;
+        if (UPDATE) {
+            w[u] = adam_update(w[u], g[u], m[u], v[u], a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
+            a.w[i][x] = w[u];
+            a.m[i][x] = m[u];
+            a.v[i][x] = v[u];
+        }
+        const uint16_t h = f2bf(w[u]);
+        if (a.wb[i]) a.wb[i][x] = h;
+        tb[ty + 8 * u][tx] = h;
+    }
+    if (!a.wt[i] && !a.wf[i] && !a.wtf[i]) return; // workgroup-uniform
+    __syncthreads();
+    if (a.wt[i]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = c0 + ty + 8 * u, r = r0 + tx; // [cols][rows]
+            if (r < R && c < C) a.wt[i][(int64_t)c * R + r] = tb[tx][ty + 8 * u];
+        }
+    }
+    // fragment order: thread -> four consecutive k of one row, 8 bytes
+    const int x = threadIdx.x * 4;
+    const int k = x / 512 * 16 + x % 512 / 256 * 8 + x % 8, n = x % 256 / 8;
+    if (a.wf[i])
+        *reinterpret_cast<ushort4*>(a.wf[i] + frag_at(C, r0, c0) + x) =
+            make_ushort4(tb[n][k], tb[n][k + 1], tb[n][k + 2], tb[n][k + 3]);
+    if (a.wtf[i])
+        *reinterpret_cast<ushort4*>(a.wtf[i] + frag_at(R, c0, r0) + x) =
+            make_ushort4(tb[k][n], tb[k + 1][n], tb[k + 2][n], tb[k + 3][n]);
 }
 
 __device__ inline float sigm(float x) { return 1.0f / (1.0f + __expf(-x)); }
@@ -600,6 +1273,178 @@ int dtb_mlp_affine(int32_t rows, int32_t cin, int32_t cout, const float* in, int
                        in, ldi, scale, shift, out, (uint16_t*)outb, ldo);
     DTB_TRY_HIP(hipGetLastError());
     return DTB_OK;
+}
+
+// LDS of the chain kernel: two activation buffers of 32 rows (wide enough for
+// the widest layer and for the exchange of a split product; the row stride
+// keeps the 32 rows of a fragment on distinct banks), then in training the sign
+// masks of the hidden outputs.
+static int chain_layout(int32_t n_layers, const dtb_mlp_layer* L, bool train, int32_t* bufw, size_t* lds)
+{
+    DTB_REQUIRE(n_layers >= 1 && L != nullptr, "at least one layer is required");
+    int64_t wide = 192, hidden = 0;
+    for (int32_t l = 0; l < n_layers; ++l) {
+        DTB_REQUIRE(L[l].n_in > 0 && L[l].n_out > 0 && L[l].n_in % 32 == 0 && L[l].n_out % 32 == 0,
+                    "layer %d: widths must be positive multiples of 32", l);
+        DTB_REQUIRE(L[l].n_in < (1 << 24) && L[l].n_out < (1 << 24), "layer %d: widths must be below 2^24", l);
+        DTB_REQUIRE(l == 0 || L[l].n_in == L[l - 1].n_out, "layer %d does not take the width of the layer before", l);
+        wide = std::max(wide, std::max(L[l].n_in, L[l].n_out));
+        if (l + 1 < n_layers) hidden += L[l].n_out / 32;
+    }
+    wide = (wide + 63) / 64 * 64 + 8;
+    const int64_t need = 2 * kMlpRows * wide * 2 + (train ? hidden * 128 : 0);
+    if (n_layers > kMlpMaxLayers || need > 160 * 1024) {
+        set_error("the chain kernel holds at most %d layers and 160 KB of activations", kMlpMaxLayers);
+        return DTB_UNSUPPORTED;
+    }
+    *bufw = (int32_t)wide;
+    *lds = (size_t)need;
+    return DTB_OK;
+}
+
+static int chain_fill(MlpChainArgs& a, int32_t n_layers, const dtb_mlp_layer* L, bool train)
+{
+    for (int32_t l = 0; l < n_layers; ++l) {
+        DTB_REQUIRE(L[l].w && L[l].bias &&
+                        ((reinterpret_cast<uintptr_t>(L[l].w) | reinterpret_cast<uintptr_t>(L[l].bias)) & 15) == 0,
+                    "layer %d: bf16 weights and bias (16-byte aligned) are required", l);
+        DTB_REQUIRE(!train || (L[l].wt && L[l].dw && L[l].db && L[l].ht && L[l].gt && L[l].dbp &&
+                               ((reinterpret_cast<uintptr_t>(L[l].wt) | reinterpret_cast<uintptr_t>(L[l].ht) |
+                                 reinterpret_cast<uintptr_t>(L[l].gt)) & 15) == 0),
+                    "layer %d: training needs the transposed weights, gradients and scratch (16-byte aligned)", l);
+        a.l[l] = MlpLayerDev{(int32_t)L[l].n_in, (int32_t)L[l].n_out, (const uint16_t*)L[l].w, (const uint16_t*)L[l].wt,
+                             L[l].bias, (uint16_t*)L[l].ht, (uint16_t*)L[l].gt, L[l].dbp};
+    }
+    a.layers = n_layers;
+    return DTB_OK;
+}
+
+int dtb_mlp_chain_fits(int32_t n_layers, const dtb_mlp_layer* layers, int32_t train)
+{
+    int32_t bufw;
+    size_t lds;
+    return chain_layout(n_layers, layers, train != 0, &bufw, &lds);
+}
+
+int dtb_mlp_predict(int32_t n_layers, const dtb_mlp_layer* layers, int32_t rows, int32_t batch, const float* X,
+                    int64_t ldx, int32_t cin, const float* x_scale, const float* x_shift, const float* y_scale,
+                    const float* y_shift, int32_t cout, float* out, int64_t ldo, void* stream)
+{
+    MlpChainArgs a{};
+    size_t lds = 0;
+    DTB_TRY(chain_layout(n_layers, layers, false, &a.bufw, &lds));
+    DTB_TRY(chain_fill(a, n_layers, layers, false));
+    DTB_REQUIRE(rows >= 0 && rows < 0x7fffffe0 && batch > 0 && batch % 32 == 0, "batch must be a positive multiple of 32");
+    DTB_REQUIRE(cin >= 0 && cin <= layers[0].n_in && cout >= 0 && cout <= layers[n_layers - 1].n_out,
+                "cin and cout must be within the widths");
+    if (rows == 0 || cout == 0) return DTB_OK;
+    DTB_REQUIRE((X || cin == 0) && out && ldx >= cin && ldo >= cout, "X, out and their strides are required");
+    a.rows = rows; a.max_batch = batch; a.cin = cin; a.cout = cout;
+    a.X = X; a.ldx = ldx; a.xs = x_scale; a.xh = x_shift; a.ys = y_scale; a.yh = y_shift; a.out = out; a.ldo = ldo;
+    // 64 rows a workgroup, which halve the weights read per row, once 32-row
+    // ones would not all be resident (the second buffer must still fit, and a
+    // batch boundary must not fall inside a workgroup's rows)
+    const bool wide = rows > 32 * 256 && batch % 64 == 0 && 2 * lds <= 160 * 1024;
+    if (wide) {
+        DTB_TRY_HIP(hipFuncSetAttribute((const void*)mlp_chain_kernel<false, 2>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        hipLaunchKernelGGL((mlp_chain_kernel<false, 2>), dim3((unsigned)((rows + 63) / 64)), dim3(kMlpThreads), 2 * lds,
+                           (hipStream_t)stream, a);
+    } else {
+        DTB_TRY_HIP(hipFuncSetAttribute((const void*)mlp_chain_kernel<false, 1>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        hipLaunchKernelGGL((mlp_chain_kernel<false, 1>), dim3((unsigned)((rows + 31) / 32)), dim3(kMlpThreads), lds,
+                           (hipStream_t)stream, a);
+    }
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_train_gradients(int32_t n_layers, const dtb_mlp_layer* layers, int32_t rows, const float* X, int64_t ldx,
+                            int32_t cin, const float* x_scale, const float* x_shift, const float* Y, int64_t ldy,
+                            int32_t cout, const float* y_scale, const float* y_shift, const float* mask, int64_t ldm,
+                            float scale, float* out, float* lsum, void* stream)
+{
+    MlpChainArgs a{};
+    size_t lds = 0;
+    DTB_TRY(chain_layout(n_layers, layers, true, &a.bufw, &lds));
+    DTB_TRY(chain_fill(a, n_layers, layers, true));
+    DTB_REQUIRE(rows > 0 && rows < (1 << 26), "rows must be in 1 .. 2^26");
+    DTB_REQUIRE(cin >= 0 && cin <= layers[0].n_in && cout >= 0 && cout <= layers[n_layers - 1].n_out,
+                "cin and cout must be within the widths");
+    DTB_REQUIRE((X || cin == 0) && (Y || cout == 0) && out && lsum && ldx >= cin && ldy >= cout &&
+                    (!mask || ldm >= cout),
+                "X, Y, out, lsum and their strides are required");
+    const int32_t B = (rows + 31) / 32 * 32;
+    a.rows = rows; a.max_batch = B; a.cin = cin; a.cout = cout;
+    a.X = X; a.ldx = ldx; a.xs = x_scale; a.xh = x_shift; a.ys = y_scale; a.yh = y_shift;
+    a.out = out; a.ldo = layers[n_layers - 1].n_out;
+    a.Y = Y; a.ldy = ldy; a.mask = mask; a.ldm = ldm; a.scale = scale; a.lsum = lsum;
+    DTB_TRY_HIP(hipFuncSetAttribute((const void*)mlp_chain_kernel<true, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    160 * 1024));
+    hipLaunchKernelGGL((mlp_chain_kernel<true, 1>), dim3((unsigned)(B / 32)), dim3(kMlpThreads), lds, (hipStream_t)stream, a);
+    DTB_TRY_HIP(hipGetLastError());
+    MlpDwArgs d{};
+    d.layers = n_layers;
+    d.B = B;
+    for (int32_t l = 0; l < n_layers; ++l) {
+        d.in[l] = a.l[l].in; d.out[l] = a.l[l].out;
+        d.hT[l] = a.l[l].hT; d.gT[l] = a.l[l].gT; d.dbp[l] = a.l[l].dbp;
+        d.dW[l] = layers[l].dw; d.db[l] = layers[l].db;
+        d.first[l + 1] = d.first[l] + (a.l[l].out + 63) / 64 * ((a.l[l].in + 63) / 64);
+    }
+    hipLaunchKernelGGL(mlp_dw_kernel, dim3((unsigned)d.first[n_layers]), dim3(256), 0, (hipStream_t)stream, d);
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+static int adam_multi(int32_t n, const dtb_adam_param* p, bool update, float lr, float b1, float b2, float eps,
+                      int32_t t, void* stream)
+{
+    DTB_REQUIRE(n >= 0 && (n == 0 || p) && t >= 1, "bad arguments");
+    for (int32_t i = 0; i < n; ++i) {
+        DTB_REQUIRE(p[i].rows > 0 && p[i].cols > 0 && p[i].rows < (1 << 24) && p[i].cols < (1 << 24) && p[i].w &&
+                        (!update || (p[i].g && p[i].m && p[i].v)),
+                    "parameter %d: bad arguments", i);
+        DTB_REQUIRE((!p[i].wf && !p[i].wtf) ||
+                        (p[i].rows % 32 == 0 && p[i].cols % 32 == 0 &&
+                         ((reinterpret_cast<uintptr_t>(p[i].wf) | reinterpret_cast<uintptr_t>(p[i].wtf)) & 15) == 0),
+                    "parameter %d: fragment order needs multiples of 32 and 16-byte alignment", i);
+    }
+    const float c1 = 1.0f - powf(b1, (float)t), c2 = 1.0f - powf(b2, (float)t);
+    for (int32_t i0 = 0; i0 < n; i0 += kAdamMax) {
+        AdamMultiArgs a{};
+        a.n = std::min(kAdamMax, n - i0);
+        int64_t tiles = 0;
+        for (int32_t i = 0; i < a.n; ++i) {
+            const dtb_adam_param& q = p[i0 + i];
+            a.rows[i] = (int32_t)q.rows; a.cols[i] = (int32_t)q.cols;
+            a.w[i] = q.w; a.g[i] = q.g; a.m[i] = q.m; a.v[i] = q.v;
+            a.wb[i] = (uint16_t*)q.wb; a.wt[i] = (uint16_t*)q.wt;
+            a.wf[i] = (uint16_t*)q.wf; a.wtf[i] = (uint16_t*)q.wtf;
+            tiles += (q.rows + 31) / 32 * ((q.cols + 31) / 32);
+            DTB_REQUIRE(tiles < (1ll << 31), "too many parameters for one launch");
+            a.first[i + 1] = (int32_t)tiles;
+        }
+        a.lr = lr; a.b1 = b1; a.b2 = b2; a.eps = eps; a.c1 = c1; a.c2 = c2;
+        if (update)
+            hipLaunchKernelGGL(adam_multi_kernel<true>, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, a);
+        else
+            hipLaunchKernelGGL(adam_multi_kernel<false>, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, a);
+    }
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_adam_multi(int32_t n, const dtb_adam_param* params, float lr, float b1, float b2, float eps, int32_t t,
+                       void* stream)
+{
+    return adam_multi(n, params, true, lr, b1, b2, eps, t, stream);
+}
+
+int dtb_mlp_refresh_bf16(int32_t n, const dtb_adam_param* params, void* stream)
+{
+    return adam_multi(n, params, false, 0.0f, 0.0f, 0.0f, 0.0f, 1, stream);
 }
 
 int dtb_gru_forward(int32_t B, int32_t H, const float* gi, const float* gh, const float* h, float* hn, void* hnb,

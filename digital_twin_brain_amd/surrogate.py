@@ -25,6 +25,11 @@ def _pad(n, m=32):
     return (int(n) + m - 1) // m * m
 
 
+def _params(rows):
+    """dtb_adam_param table of (rows, cols, w, g, m, v, and the bf16 copies wb, wt, wf, wtf) tensors."""
+    return np.array([(r, c, *(0 if x is None else x.data_ptr() for x in ts)) for r, c, *ts in rows], dtype=np.int64)
+
+
 class MLPSurrogate:
     def __init__(self, n_in, n_out, hidden=(512, 512, 512), max_batch=256, device=0, seed=0, lr=1e-3,
                  betas=(0.9, 0.999), eps=1e-8):
@@ -38,7 +43,9 @@ class MLPSurrogate:
         self.t = 0
         g = torch.Generator().manual_seed(seed)
         f32, bf = dict(dtype=torch.float32, device=self.dev), dict(dtype=torch.bfloat16, device=self.dev)
-        self.W, self.b, self.Wb, self.WbT = [], [], [], []
+        # bf16 weights and their transposes in fragment order (dtb_adam_param)
+        self.W, self.b, self.Wf, self.WTf = [], [], [], []
+        self.Wb = self.WbT = None  # row-major copies of the launch-per-product path
         self.mW, self.vW, self.mb, self.vb, self.dW, self.db = [], [], [], [], [], []
         for l, (i, o) in enumerate(zip(self.sizes[:-1], self.sizes[1:])):
             w = torch.randn((o, i), generator=g) * np.sqrt(2.0 / i)  # He initialisation
@@ -46,22 +53,25 @@ class MLPSurrogate:
                 w[:, self.n_in:] = 0.0
             self.W.append(w.to(self.dev))
             self.b.append(torch.zeros(o, **f32))
-            self.Wb.append(torch.empty((o, i), **bf))
-            self.WbT.append(torch.empty((i, o), **bf))
+            self.Wf.append(torch.empty((o, i), **bf))
+            self.WTf.append(torch.empty((i, o), **bf))
             for lst in (self.mW, self.vW, self.dW):
                 lst.append(torch.zeros((o, i), **f32))
             for lst in (self.mb, self.vb, self.db):
                 lst.append(torch.zeros(o, **f32))
         B = self.max_batch
-        self.H = [torch.empty((B, s), **f32) for s in self.sizes]       # layer inputs (H[0] = X) and output
-        self.Hb = [torch.empty((B, s), **bf) for s in self.sizes[:-1]]
-        self.HbT = [torch.empty((s, B), **bf) for s in self.sizes[:-1]]
-        self.G = [torch.empty((B, s), **f32) for s in self.sizes[1:]]    # gradient of each layer's Z
-        self.Gb = [torch.empty((B, s), **bf) for s in self.sizes[1:]]
-        self.GbT = [torch.empty((s, B), **bf) for s in self.sizes[1:]]
-        self.dH = torch.empty((B, max(self.sizes)), **f32)
-        self.T = torch.empty((B, self.sizes[-1]), **f32)
-        self.M = torch.empty((B, self.sizes[-1]), **f32)
+        self.HbT = [torch.empty((s, B), **bf) for s in self.sizes[:-1]]  # bf16 layer inputs, transposed
+        self.GbT = [torch.empty((s, B), **bf) for s in self.sizes[1:]]   # bf16 gradient of each layer's Z, transposed
+        self.dbp = [torch.empty((B // 32, s), **f32) for s in self.sizes[1:]]
+        # the whole-network kernels, unless the network is too wide or deep for
+        # them: then a launch per product, whose activations live in memory
+        # (H: layer inputs, H[0] = X, and the output)
+        table = self._table()
+        self.chain = self.lib.dtb_mlp_chain_fits(len(self.W), table.ctypes.data, 0) == nat.DTB_OK
+        self.chain_train = self.lib.dtb_mlp_chain_fits(len(self.W), table.ctypes.data, 1) == nat.DTB_OK
+        self.H = [None] * len(self.W) + [torch.empty((B, self.sizes[-1]), **f32)]
+        if not (self.chain and self.chain_train):
+            self._alloc_layers()
         self.lsum = torch.empty(((B * self.sizes[-1] + 255) // 256,), **f32)
         self.x_scale = torch.ones(self.n_in, **f32)
         self.x_shift = torch.zeros(self.n_in, **f32)
@@ -75,12 +85,36 @@ class MLPSurrogate:
     def _stream(self):
         return torch.cuda.current_stream(self.dev).cuda_stream
 
+    def _alloc_layers(self):
+        """Buffers of the launch-per-product path."""
+        B = self.max_batch
+        f32, bf = dict(dtype=torch.float32, device=self.dev), dict(dtype=torch.bfloat16, device=self.dev)
+        self.Wb = [torch.empty(w.shape, **bf) for w in self.W]
+        self.WbT = [torch.empty((w.shape[1], w.shape[0]), **bf) for w in self.W]
+        self.H[:-1] = [torch.empty((B, s), **f32) for s in self.sizes[:-1]]
+        self.Hb = [torch.empty((B, s), **bf) for s in self.sizes[:-1]]
+        self.G = [torch.empty((B, s), **f32) for s in self.sizes[1:]]    # gradient of each layer's Z
+        self.Gb = [torch.empty((B, s), **bf) for s in self.sizes[1:]]
+        self.dH = torch.empty((B, max(self.sizes)), **f32)
+        self.T = torch.empty((B, self.sizes[-1]), **f32)
+        self.M = torch.empty((B, self.sizes[-1]), **f32)
+
+    def _table(self):
+        """dtb_mlp_layer [layers] (ten 8-byte fields each) of the current buffers."""
+        return np.array([(w.shape[1], w.shape[0], wf.data_ptr(), wt.data_ptr(), b.data_ptr(), dw.data_ptr(),
+                          db.data_ptr(), ht.data_ptr(), gt.data_ptr(), dbp.data_ptr())
+                         for w, wf, wt, b, dw, db, ht, gt, dbp in zip(self.W, self.Wf, self.WTf, self.b, self.dW,
+                                                                      self.db, self.HbT, self.GbT, self.dbp)],
+                        dtype=np.int64)
+
+    def _weights(self):
+        none = [None] * len(self.W)
+        return [(w.shape[0], w.shape[1], w, *r) for w, *r in
+                zip(self.W, self.dW, self.mW, self.vW, self.Wb or none, self.WbT or none, self.Wf, self.WTf)]
+
     def _refresh_bf16(self):
-        s = self._stream()
-        for l, w in enumerate(self.W):
-            o, i = w.shape
-            nat.check(self.lib.dtb_mlp_f32_to_bf16(o * i, w.data_ptr(), self.Wb[l].data_ptr(), s))
-            nat.check(self.lib.dtb_mlp_transpose_bf16(o, i, self.Wb[l].data_ptr(), self.WbT[l].data_ptr(), s))
+        table = _params(self._weights())
+        nat.check(self.lib.dtb_mlp_refresh_bf16(len(table), table.ctypes.data, self._stream()))
 
     def set_normalization(self, X, Y):
         """Per-feature standardisation from training data (host or device arrays)."""
@@ -117,6 +151,15 @@ class MLPSurrogate:
         X = torch.as_tensor(X)
         n = X.shape[0]
         out = torch.empty((n, self.n_out), dtype=torch.float32, device=self.dev)
+        if self.chain:
+            X = X.to(self.dev, torch.float32).contiguous()
+            table = self._table()
+            nat.check(self.lib.dtb_mlp_predict(len(self.W), table.ctypes.data, n, self.max_batch, X.data_ptr(),
+                                               X.stride(0), self.n_in, self.x_scale.data_ptr(),
+                                               self.x_shift.data_ptr(), self._y_std.data_ptr(),
+                                               self._y_mean.data_ptr(), self.n_out, out.data_ptr(), self.n_out,
+                                               self._stream()))
+            return out
         for r0 in range(0, n, self.max_batch):
             r = min(self.max_batch, n - r0)
             B = _pad(r)
@@ -139,8 +182,19 @@ class MLPSurrogate:
         assert r <= self.max_batch
         B = _pad(r)
         no = self.sizes[-1]
-        self._load_x(X, r)
         Yd = torch.as_tensor(Y).to(self.dev, torch.float32).contiguous()
+        if self.chain_train:
+            X = X.to(self.dev, torch.float32).contiguous()
+            Md = None if mask is None else \
+                torch.as_tensor(mask).to(self.dev, torch.float32).expand(r, self.n_out).contiguous()
+            table = self._table()
+            nat.check(self.lib.dtb_mlp_train_gradients(
+                len(self.W), table.ctypes.data, r, X.data_ptr(), X.stride(0), self.n_in, self.x_scale.data_ptr(),
+                self.x_shift.data_ptr(), Yd.data_ptr(), Yd.stride(0), self.n_out, self.y_scale.data_ptr(),
+                self.y_shift.data_ptr(), nat.ptr(Md), self.n_out, 1.0 / max(r, 1), self.H[-1].data_ptr(),
+                self.lsum.data_ptr(), s))
+            return self.lsum[: (B * no + 255) // 256]
+        self._load_x(X, r)
         nat.check(self.lib.dtb_mlp_affine(r, self.n_out, no, Yd.data_ptr(), Yd.stride(0), self.y_scale.data_ptr(),
                                           self.y_shift.data_ptr(), self.T.data_ptr(), None, no, s))
         self.M[:B].zero_()
@@ -175,17 +229,11 @@ class MLPSurrogate:
 
     def step(self):
         """One Adam step on every parameter from the last `gradients` call."""
-        s = self._stream()
         self.t += 1
-        for l in range(len(self.W)):
-            o, i = self.W[l].shape
-            nat.check(self.lib.dtb_mlp_adam(o * i, self.W[l].data_ptr(), self.dW[l].data_ptr(), self.mW[l].data_ptr(),
-                                            self.vW[l].data_ptr(), self.lr, self.b1, self.b2, self.eps, self.t,
-                                            self.Wb[l].data_ptr(), s))
-            nat.check(self.lib.dtb_mlp_adam(o, self.b[l].data_ptr(), self.db[l].data_ptr(), self.mb[l].data_ptr(),
-                                            self.vb[l].data_ptr(), self.lr, self.b1, self.b2, self.eps, self.t, None,
-                                            s))
-            nat.check(self.lib.dtb_mlp_transpose_bf16(o, i, self.Wb[l].data_ptr(), self.WbT[l].data_ptr(), s))
+        table = _params(self._weights() + [(1, b.shape[0], b, g, m, v, None, None, None, None) for b, g, m, v in
+                                           zip(self.b, self.db, self.mb, self.vb)])
+        nat.check(self.lib.dtb_mlp_adam_multi(len(table), table.ctypes.data, self.lr, self.b1, self.b2, self.eps,
+                                              self.t, self._stream()))
 
     def fit(self, X, Y, epochs=50, batch=None, seed=0, verbose=False):
         """Mini-batch Adam over (X, Y) kept on the device; returns the mean
@@ -390,15 +438,11 @@ class GRUSurrogate:
         return self.lsum[: (TB * O + 255) // 256]
 
     def step(self):
-        s = self._stream()
         self.t += 1
-        for k, w in self.p.items():
-            nat.check(self.lib.dtb_mlp_adam(w.numel(), w.data_ptr(), self.grad[k].data_ptr(), self.m[k].data_ptr(),
-                                            self.v[k].data_ptr(), self.lr, self.b1, self.b2, self.eps, self.t,
-                                            nat.ptr(self.pb.get(k)), s))
-        for k in self.pbT:
-            r, c = self.p[k].shape
-            nat.check(self.lib.dtb_mlp_transpose_bf16(r, c, self.pb[k].data_ptr(), self.pbT[k].data_ptr(), s))
+        table = _params([(w.shape[0] if w.dim() == 2 else 1, w.shape[-1], w, self.grad[k], self.m[k], self.v[k],
+                          self.pb.get(k), self.pbT.get(k), None, None) for k, w in self.p.items()])
+        nat.check(self.lib.dtb_mlp_adam_multi(len(table), table.ctypes.data, self.lr, self.b1, self.b2, self.eps,
+                                              self.t, self._stream()))
 
     def fit(self, X, Y, epochs=50, batch=None, seed=0):
         """X [T, n, n_in], Y [T, n, n_out] sequences; mini-batches over n."""

@@ -391,6 +391,66 @@ int dtb_mlp_transpose_bf16(int32_t M, int32_t N, const void* in, void* out, void
  * stride ldo; scale/shift may be NULL (1 and 0). */
 int dtb_mlp_affine(int32_t rows, int32_t cin, int32_t cout, const float* in, int64_t ldi, const float* scale,
                    const float* shift, float* out, void* outb, int64_t ldo, void* stream);
+/* Whole-network calls of the MLP surrogate: the layers of one network in one
+ * kernel for a prediction, two for a training batch, with the results of the
+ * calls above (bit for bit; bias gradients up to FP32 summation order).
+ * Layer l takes n_in values and gives n_out (padded widths, multiples of 32;
+ * hidden layers ReLU, the last identity); w and wt are the bf16 weights
+ * [n_out][n_in] and their transpose in fragment order (wf and wtf of
+ * dtb_adam_param).  Training fills dw [n_out][n_in] and db [n_out] and uses the
+ * scratch ht (bf16 [n_in][B]), gt (bf16 [n_out][B]) and dbp (FP32
+ * [B/32][n_out]) for B rows padded to a multiple of 32; prediction leaves
+ * everything but w and bias unread.  bf16 arrays 16-byte aligned. */
+typedef struct {
+    int64_t n_in, n_out;
+    const void* w;
+    const void* wt;
+    const float* bias;
+    float* dw;
+    float* db;
+    void* ht;
+    void* gt;
+    float* dbp;
+} dtb_mlp_layer;
+
+/* DTB_OK if the network fits the whole-network kernels (at most 8 layers,
+ * activations of 32 rows within 160 KB of LDS), else DTB_UNSUPPORTED. */
+int dtb_mlp_chain_fits(int32_t n_layers, const dtb_mlp_layer* layers, int32_t train);
+/* out[rows][cout] = (network(X * x_scale + x_shift)) * y_scale + y_shift;
+ * `batch` is the rows that the layer-by-layer calls would take at a time (a
+ * product's summation order depends on its row count). */
+int dtb_mlp_predict(int32_t n_layers, const dtb_mlp_layer* layers, int32_t rows, int32_t batch, const float* X,
+                    int64_t ldx, int32_t cin, const float* x_scale, const float* x_shift, const float* y_scale,
+                    const float* y_shift, int32_t cout, float* out, int64_t ldo, void* stream);
+/* Forward and backward of one batch: the masked squared error of the
+ * standardised outputs against Y * y_scale + y_shift; gradient of the output
+ * = scale * mask * (out - target).  out [B][n_out of the last layer] is the
+ * raw output, lsum one partial sum per 256 consecutive elements of it. */
+int dtb_mlp_train_gradients(int32_t n_layers, const dtb_mlp_layer* layers, int32_t rows, const float* X, int64_t ldx,
+                            int32_t cin, const float* x_scale, const float* x_shift, const float* Y, int64_t ldy,
+                            int32_t cout, const float* y_scale, const float* y_shift, const float* mask, int64_t ldm,
+                            float scale, float* out, float* lsum, void* stream);
+/* dtb_mlp_adam on n parameter tensors [rows][cols] in one launch, refreshing
+ * the bf16 copies that are not NULL: wb [rows][cols], wt its transpose, and
+ * both in fragment order (wf, wtf; rows and cols multiples of 32, 16-byte
+ * aligned).  Fragment order of [N][K]: element (n, k) at
+ * (n/32 * (K/16) + k/16) * 512 + (k%16/8 * 32 + n%32) * 8 + k%8, the operand
+ * of one 32x32x16 matrix instruction contiguous. */
+typedef struct {
+    int64_t rows, cols;
+    float* w;
+    const float* g;
+    float* m;
+    float* v;
+    void* wb;
+    void* wt;
+    void* wf;
+    void* wtf;
+} dtb_adam_param;
+int dtb_mlp_adam_multi(int32_t n, const dtb_adam_param* params, float lr, float b1, float b2, float eps, int32_t t,
+                       void* stream);
+/* the bf16 copies alone (g, m and v unread) */
+int dtb_mlp_refresh_bf16(int32_t n, const dtb_adam_param* params, void* stream);
 /* GRU cell, gate order (r, z, n) as torch.nn.GRU.  gi = x W_ih^T + b_ih and
  * gh = h W_hh^T + b_hh are [B][3H] FP32 (from dtb_mlp_gemm_bf16_nt);
  * forward: hn = (1-z) n + z h with r = sigmoid(gi_r+gh_r),

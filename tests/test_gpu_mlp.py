@@ -290,3 +290,68 @@ def test_bias_grad_over_row_and_column_remainders(M, N):
     bound = (M / 64 + 6) * 2.0 ** -24 * dZ.double().abs().sum(0)
     assert ((db[:N].double() - dZ.double().sum(0)).abs() <= bound).all()
     assert float(db[N]) == 7.0
+
+
+# one layer; one 32-wide tile; widths of one, two and more tiles per wavefront; a batch whose
+# products are one chain over K (2048 x 512) beside ones split in four; wide inputs and outputs
+# (two output tiles a wavefront and a half-empty second round); rows at the edges of the 32-row tiles
+@pytest.mark.parametrize("n_in,n_out,hidden,rows,batch", [
+    (18, 6, (), 5, 32), (18, 6, (32,), 31, 32), (40, 70, (64, 96), 33, 64), (18, 6, (512, 512, 512), 2048, 2048),
+    (18, 6, (512, 256), 2047, 2048), (720, 540, (512, 512, 512), 64, 64), (100, 300, (544, 32), 130, 256),
+    (8, 600, (128,), 96, 96), (33, 5, (64, 64, 64, 64, 64, 64, 64), 40, 64)])
+def test_whole_network_kernels_equal_the_layer_by_layer_launches(n_in, n_out, hidden, rows, batch):
+    """Prediction and weight gradients bit for bit; the bias gradients and loss
+    sums, FP32 sums in another order, to (terms) roundings."""
+    from digital_twin_brain_amd.surrogate import MLPSurrogate
+
+    g = torch.Generator().manual_seed(rows + n_in)
+    X = torch.randn((rows, n_in), generator=g)
+    Y = torch.randn((rows, n_out), generator=g)
+    mask = (torch.rand((rows, n_out), generator=g) > 0.3).float()
+    Xp = torch.randn((batch + 70, n_in), generator=g)  # a whole batch and a part
+    sur = [MLPSurrogate(n_in, n_out, hidden=hidden, max_batch=batch, seed=4) for _ in range(2)]
+    for s in sur:
+        assert s.chain and s.chain_train
+        for b in s.b:
+            b.copy_(torch.linspace(-0.1, 0.2, b.shape[0]))
+        s.set_normalization(X, Y + 0.3)
+    sur[1].chain = sur[1].chain_train = False
+    sur[1]._alloc_layers()
+    sur[1]._refresh_bf16()
+    for m in (None, mask):
+        for step in range(2):
+            a, b = (s.gradients(X, Y, m).clone() for s in sur)
+            B = (rows + 31) // 32 * 32
+            assert a.shape == b.shape
+            torch.testing.assert_close(a, b, rtol=256 * 2.0 ** -23, atol=0)
+            assert torch.equal(sur[0].H[-1][:B], sur[1].H[-1][:B])
+            for l in range(len(hidden) + 1):
+                assert torch.equal(sur[0].dW[l], sur[1].dW[l]), l
+                G = sur[1].G[l][:B].double()
+                bound = B * 2.0 ** -23 * G.abs().sum(0)
+                assert ((sur[0].db[l].double() - G.sum(0)).abs() <= bound).all(), l
+            for s in sur:
+                for l in range(len(hidden) + 1):
+                    s.db[l].copy_(sur[1].db[l])  # the same bias step on both sides
+                s.step()
+            for l in range(len(hidden) + 1):
+                assert torch.equal(sur[0].W[l], sur[1].W[l]) and torch.equal(sur[0].b[l], sur[1].b[l])
+                assert torch.equal(_bits(sur[1].Wb[l]), _bits(sur[1].W[l].to(torch.bfloat16)))
+                assert torch.equal(_bits(sur[1].WbT[l]), _bits(sur[1].Wb[l].T))
+    assert torch.equal(sur[0].predict(Xp), sur[1].predict(Xp))
+
+
+def test_networks_beyond_the_whole_network_kernels_run_layer_by_layer():
+    from digital_twin_brain_amd.surrogate import MLPSurrogate
+
+    for hidden in ((2560,), (32,) * 8):  # wider than 160 KB of activations; nine layers
+        sur = MLPSurrogate(10, 4, hidden=hidden, max_batch=32, seed=1)
+        assert not sur.chain and not sur.chain_train
+        sur.gradients(torch.randn(20, 10), torch.randn(20, 4))
+        sur.step()
+        assert sur.predict(torch.randn(40, 10)).isfinite().all()
+    mixed = MLPSurrogate(10, 4, hidden=(1184, 1184), max_batch=32, seed=1)  # the sign masks do not fit beside 1,184 columns
+    assert mixed.chain and not mixed.chain_train
+    mixed.gradients(torch.randn(20, 10), torch.randn(20, 4))
+    mixed.step()
+    assert mixed.predict(torch.randn(40, 10)).isfinite().all()
