@@ -111,6 +111,13 @@ SIGNATURES = {
                                 _f32, _vp, _vp, _vp],
     "dtb_mlp_adam_multi": [_i32, _vp, _f32, _f32, _f32, _f32, _i32, _vp],
     "dtb_mlp_refresh_bf16": [_i32, _vp, _vp],
+    "dtb_gru_sequence_fits": [_i32, _i32],
+    "dtb_gru_sequence_forward": [_i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _vp],
+    "dtb_gru_sequence_backward": [_i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+    "dtb_mlp_column_sums": [_i32, _vp, _i64, _vp],
+    "dtb_mlp_sequence_loss": [_i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp],
+    "dtb_mlp_pack_transposed": [_i32, _vp, _vp],
+    "dtb_mlp_weight_gradients": [_i32, _vp, _i32, _vp],
     "dtb_gru_forward": [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp],
     "dtb_gru_backward": [_i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
 }
@@ -152,6 +159,8 @@ def exported_symbols():
             "dtb_mlp_adam", "dtb_mlp_transpose_bf16", "dtb_mlp_f32_to_bf16", "dtb_mlp_affine",
             "dtb_mlp_chain_fits", "dtb_mlp_predict", "dtb_mlp_train_gradients", "dtb_mlp_adam_multi",
             "dtb_mlp_refresh_bf16",
+            "dtb_gru_sequence_fits", "dtb_gru_sequence_forward", "dtb_gru_sequence_backward",
+            "dtb_mlp_sequence_loss", "dtb_mlp_pack_transposed", "dtb_mlp_weight_gradients", "dtb_mlp_column_sums",
             "dtb_gru_forward", "dtb_gru_backward"]
 
 

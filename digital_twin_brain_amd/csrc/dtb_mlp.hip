@@ -315,41 +315,71 @@ __global__ void relu_backward_kernel(int64_t n, const float* __restrict__ dY, co
     if (dZb) dZb[i] = f2bf(v);
 }
 
-// db[j] = sum_i dZ[i][j].  Bound by the latency of the loads down a column,
-// so the rows are split: a workgroup takes kBiasCols columns (64 contiguous
-// bytes a row) and 64 row lanes, each of which has kBiasUnroll loads in flight
-// and sums every 64th row; the row lanes are then added pairwise in LDS.  The
-// order is fixed by M alone.  2048 x 512: 465 us with one thread walking a
-// column, 5 us split.
-constexpr int kBiasCols = 16, kBiasRows = 64, kBiasUnroll = 16;
+// db[j] = sum_i dZ[i][j], added in row order (a bias one rounding away from
+// another one's changes which way a GRU's states round, and so every gradient
+// after the next update).  One thread walking a column waits for its loads, 465
+// us for 2,048 rows; here a workgroup stages kBiasRows rows x 64 columns in
+// LDS at a time, all 1024 threads' loads of the next rows in flight while the
+// first wavefront adds the staged ones (a lane per column).  The adds, a
+// dependent chain, are then what is left: 21 us for 2,048 x 1,056.
+constexpr int kBiasCols = 64, kBiasRows = 256, kBiasThreads = 1024;
+constexpr int kBiasLoads = kBiasRows * kBiasCols / kBiasThreads;
 
-__global__ __launch_bounds__(kBiasCols* kBiasRows) void bias_grad_kernel(int32_t M, int32_t N,
-                                                                         const float* __restrict__ dZ,
-                                                                         float* __restrict__ db)
+__device__ __forceinline__ void column_sums(int64_t M, int32_t N, const float* __restrict__ src, int64_t ld, int j0,
+                                            float* lds, float* __restrict__ dst, float* __restrict__ dst2)
 {
-    __shared__ float red[kBiasRows][kBiasCols];
-    const int c = threadIdx.x % kBiasCols, r = threadIdx.x / kBiasCols;
-    const int32_t j = blockIdx.x * kBiasCols + c;
-    float s = 0.0f;
-    if (j < N) {
-        for (int64_t i0 = r; i0 < M; i0 += (int64_t)kBiasRows * kBiasUnroll) {
-            float v[kBiasUnroll];
+    const int c = threadIdx.x % kBiasCols, r0 = threadIdx.x / kBiasCols;
+    const int j = j0 + c;
+    float v[kBiasLoads];
+    auto load = [&](int64_t i0) {
 #pragma unroll
-            for (int u = 0; u < kBiasUnroll; ++u) {
-                const int64_t i = i0 + (int64_t)u * kBiasRows;
-                v[u] = i < M ? dZ[i * N + j] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < kBiasUnroll; ++u) s += v[u];
+        for (int u = 0; u < kBiasLoads; ++u) {
+            const int64_t i = i0 + r0 + u * (kBiasThreads / kBiasCols);
+            v[u] = i < M && j < N ? src[i * ld + j] : 0.0f;
         }
-    }
-    red[r][c] = s;
-    __syncthreads();
-    for (int h = kBiasRows / 2; h > 0; h >>= 1) {
-        if (r < h) red[r][c] += red[r + h][c];
+    };
+    float s = 0.0f;
+    load(0);
+    for (int64_t i0 = 0; i0 < M; i0 += kBiasRows) {
+#pragma unroll
+        for (int u = 0; u < kBiasLoads; ++u) lds[(r0 + u * (kBiasThreads / kBiasCols)) * kBiasCols + c] = v[u];
+        __syncthreads();
+        if (i0 + kBiasRows < M) load(i0 + kBiasRows);
+        if (threadIdx.x < kBiasCols) {
+            const int n = (int)(M - i0 < kBiasRows ? M - i0 : kBiasRows);
+            // the next 16 rows are read while the 16 before are added
+            float x[2][16];
+            auto read = [&](float (&d)[16], int i) {
+#pragma unroll
+                for (int u = 0; u < 16; ++u) d[u] = lds[(i + u) * kBiasCols + c];
+            };
+            read(x[0], 0);
+#pragma unroll
+            for (int q = 0; q < kBiasRows / 16; ++q) {
+                if (q + 1 < kBiasRows / 16) read(x[(q + 1) & 1], 16 * (q + 1));
+                if (16 * q + 16 <= n) { // uniform
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) s += x[q & 1][u];
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 16; ++u)
+                        if (16 * q + u < n) s += x[q & 1][u];
+                }
+            }
+        }
         __syncthreads();
     }
-    if (r == 0 && j < N) db[j] = red[0][c];
+    if (threadIdx.x < kBiasCols && j < N) {
+        dst[j] = s;
+        if (dst2) dst2[j] = s;
+    }
+}
+
+__global__ __launch_bounds__(kBiasThreads) void bias_grad_kernel(int32_t M, int32_t N, const float* __restrict__ dZ,
+                                                                 float* __restrict__ db)
+{
+    __shared__ float lds[kBiasRows * kBiasCols];
+    column_sums(M, N, dZ, N, blockIdx.x * kBiasCols, lds, db, nullptr);
 }
 
 // grad = scale * (out - target) masked; loss partial sums in lsum[blockIdx]
@@ -878,15 +908,38 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_chain_kernel(MlpChainArgs a)
 // tile, where dtb_mlp_gemm_bf16_nt would); the workgroups of the first tile
 // column also add the row tiles' column sums into db.
 struct MlpDwArgs {
-    int32_t layers, B;
+    int32_t layers, B;     // B: rows (K of the products)
     int32_t first[kMlpMaxLayers + 1];
     int32_t in[kMlpMaxLayers], out[kMlpMaxLayers];
+    int64_t ldh[kMlpMaxLayers], ldg[kMlpMaxLayers]; // columns of the arrays that hT and gT are part of
+    int32_t parts[kMlpMaxLayers]; // partial column sums (rows of dbp)
     const uint16_t* hT[kMlpMaxLayers];
     const uint16_t* gT[kMlpMaxLayers];
     const float* dbp[kMlpMaxLayers];
     float* dW[kMlpMaxLayers];
     float* db[kMlpMaxLayers];
 };
+
+// Column sums of FP32 arrays [rows][ld] in row order, workgroups
+// [first[i], first[i + 1]) for array i, 64 columns each.
+struct ColsumArgs {
+    int32_t n;
+    int64_t rows;
+    int32_t first[kMlpMaxLayers + 1];
+    int32_t cols[kMlpMaxLayers];
+    int64_t ld[kMlpMaxLayers];
+    const float* src[kMlpMaxLayers];
+    float* dst[kMlpMaxLayers];
+    float* dst2[kMlpMaxLayers]; // a second copy, or NULL
+};
+
+__global__ __launch_bounds__(kBiasThreads) void colsum_kernel(ColsumArgs a)
+{
+    __shared__ float lds[kBiasRows * kBiasCols];
+    int i = 0;
+    while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+    column_sums(a.rows, a.cols[i], a.src[i], a.ld[i], (blockIdx.x - a.first[i]) * kBiasCols, lds, a.dst[i], a.dst2[i]);
+}
 
 __global__ __launch_bounds__(256) void mlp_dw_kernel(MlpDwArgs a)
 {
@@ -906,8 +959,8 @@ __global__ __launch_bounds__(256) void mlp_dw_kernel(MlpDwArgs a)
     const uint16_t *pa[2], *pb[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) { // a sub-tile past the edge repeats the last one and is not stored
-        pa[i] = a.gT[l] + (int64_t)min(m0 + 32 * i, M - 32) * B + lane * 8;
-        pb[i] = a.hT[l] + (int64_t)min(n0 + 32 * i, N - 32) * B + lane * 8;
+        pa[i] = a.gT[l] + min(m0 + 32 * i, M - 32) * a.ldg[l] + lane * 8;
+        pb[i] = a.hT[l] + min(n0 + 32 * i, N - 32) * a.ldh[l] + lane * 8;
     }
     f32x16 acc[2][2];
 #pragma unroll
@@ -1000,12 +1053,12 @@ __global__ __launch_bounds__(256) void mlp_dw_kernel(MlpDwArgs a)
             }
         }
     }
-    if (tile % tn == 0) {
+    if (tile % tn == 0 && a.db[l]) {
         const int c = m0 + lane;
         float s = 0.0f;
         if (c < M) {
 #pragma unroll 8
-            for (int k = wid; k < B / 32; k += 4) s += a.dbp[l][(int64_t)k * M + c];
+            for (int k = wid; k < a.parts[l]; k += 4) s += a.dbp[l][(int64_t)k * M + c];
         }
         dred[wid][lane] = s;
         __syncthreads();
@@ -1108,7 +1161,7 @@ __global__ void gru_forward_kernel(int32_t B, int32_t H, const float* __restrict
     const float r = sigm(a[j] + c[j]);
     const float z = sigm(a[H + j] + c[H + j]);
     const float n = tanhf(a[2 * H + j] + r * c[2 * H + j]);
-    const float v = (1.0f - z) * n + z * h[i];
+    const float v = fmaf(1.0f - z, n, z * h[i]); // the sequence kernel's rounding too
     hn[i] = v;
     if (hnb) hnb[i] = f2bf(v);
 }
@@ -1156,6 +1209,365 @@ __global__ void gru_backward_kernel(int32_t B, int32_t H, const float* __restric
         dghb[o + 2 * H + j] = f2bf(dn * r);
     }
 }
+
+// ------------------------------------------------------ whole-sequence GRU
+// A GRU step is a 64 x 768 x 256 product and 16,384 gates, so a launch per
+// product and gate kernel left the device idle between them: 32 steps forward
+// and backward were 128 launches, about 10 us each.  Batch rows never mix in
+// the recurrence, so a workgroup takes kGruRows rows through all steps of the
+// sequence, and keeps the recurrent weights on its CU: wavefront w holds the
+// 16-row tiles w, w + 16, ... of W_hh (forward, 3H x H) or of its transpose
+// (backward, H x 3H) as operands of v_mfma_f32_16x16x32_bf16, in registers and
+// the rest in LDS (GruWeights).  Four rows a workgroup fill a quarter of an instruction's 16
+// columns; more workgroups share the gates' arithmetic, which costs more than
+// the products.  A step: products -> LDS -> barrier -> gates (a thread owns its
+// rows' hidden units and keeps their h or gradient) -> LDS -> barrier; the
+// step's inputs are loaded one step ahead.
+// The products are summed as dtb_mlp_gemm_bf16_nt splits them (four
+// consecutive ranges of K, added in order; a 16x16x32 instruction adds 32
+// terms as two 32x32x16 ones do), so results equal the launch-per-step path.
+// 32 steps x 64 rows x H = 256: 73 us forward and 112 us backward, against
+// about 320 us each; the training step 2007 -> 251 us.
+constexpr int kGruRows = 4;
+constexpr int kGruFwdWaves = 8, kGruFwdHeld = 34;  // wavefronts and operands that each holds in registers
+constexpr int kGruBwdWaves = 16, kGruBwdHeld = 16;
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// The recurrent weights of one of NW wavefronts: TW tiles of KS instructions'
+// operands, the first HELD in registers and the others in LDS, 112 to 128 KB
+// of it at H = 256.  Forward, eight wavefronts that hold 34 of their 48
+// operands leave least to LDS (32 steps of 64 rows: 73 us, 109 with sixteen);
+// backward the loaded gates need the registers too, and sixteen wavefronts that
+// hold 16 of 24 do not spill (111 us, 189 with eight).
+template <int TW, int KS, int NW, int HELD>
+struct GruWeights {
+    static constexpr int N = TW * KS;
+    static constexpr int kReg = N < HELD ? N : HELD;
+    static constexpr int kLds = (N - kReg) * NW * 64 * 16; // bytes of a workgroup
+    bf16x8 r[kReg];
+    const bf16x8* l;
+
+    // rows of W: tile wid + NW i, [16 tiles][K]; past the last tile the last one again
+    __device__ __forceinline__ void load(const uint16_t* __restrict__ W, int tiles, int wid, int lane, uint16_t* lds)
+    {
+        bf16x8* p = reinterpret_cast<bf16x8*>(lds) + (size_t)wid * (N - kReg) * 64 + lane;
+        l = p;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int tile = min(wid + NW * i, tiles - 1);
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const bf16x8 v = *reinterpret_cast<const bf16x8*>(W + (int64_t)(tile * 16 + (lane & 15)) * (32 * KS) +
+                                                                  32 * s + (lane >> 4) * 8);
+                if (i * KS + s < kReg) r[i * KS + s] = v;
+                else p[(i * KS + s - kReg) * 64] = v; // read back by this lane alone
+            }
+        }
+    }
+    __device__ __forceinline__ bf16x8 get(int f) const { return f < kReg ? r[f < kReg ? f : 0] : l[(f - kReg) * 64]; }
+};
+
+// KS = K / 32.  tot = sum over K in four consecutive ranges of `per` steps of
+// 16: tile i of the weights by h, the other operand in LDS.
+template <int KS, typename Weights>
+__device__ __forceinline__ f32x4v gru_product(const Weights& W, int i, const uint16_t* h, bool upper)
+{
+    constexpr int per = (2 * KS + 3) / 4;
+    f32x4v acc = {0.0f, 0.0f, 0.0f, 0.0f}, tot = {-0.0f, -0.0f, -0.0f, -0.0f};
+    const bf16x8 zero = {};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(h + 32 * s);
+        const bf16x8 a = W.get(i * KS + s);
+        if (s > 0 && (2 * s) % per == 0) {
+            tot += acc;
+            acc = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        if ((2 * s + 1) % per == 0) { // a range ends inside this instruction's 32 columns: its halves apart
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(upper ? zero : a, b, acc, 0, 0, 0);
+            tot += acc;
+            acc = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(upper ? a : zero, b, acc, 0, 0, 0);
+        } else {
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+        }
+    }
+    return tot + acc;
+}
+
+// G = H / 32.  gi [T][B][3H]; h0 [rows][H] or NULL (zeros; rows past h0_rows
+// start at zero); writes gh [T][B][3H], hs [T + 1][B][H] and its bf16 copy.
+template <int G>
+__global__ __launch_bounds__(64 * kGruFwdWaves) void gru_seq_forward_kernel(int32_t T, int32_t B, const float* __restrict__ gi,
+                                                                     const uint16_t* __restrict__ W,
+                                                                     const float* __restrict__ bhh,
+                                                                     const float* __restrict__ h0, int32_t h0_rows,
+                                                                     float* __restrict__ gh, float* __restrict__ hs,
+                                                                     uint16_t* __restrict__ hb)
+{
+    constexpr int kGruWaves = kGruFwdWaves, kGruThreads = 64 * kGruWaves;
+    constexpr int H = 32 * G, NT = 3 * H / 16, TW = (NT + kGruWaves - 1) / kGruWaves;
+    constexpr int EP = (kGruRows * H + kGruThreads - 1) / kGruThreads;
+    constexpr int LH = H + 8, LG = 3 * H + 4;
+    __shared__ __align__(16) uint16_t sh[kGruRows * LH];
+    __shared__ __align__(16) float sg[kGruRows * LG];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int row0 = blockIdx.x * kGruRows;
+    extern __shared__ __align__(16) uint16_t sw[];
+    GruWeights<TW, G, kGruWaves, kGruFwdHeld> w;
+    w.load(W, NT, wid, lane, sw);
+    // this thread's elements (row, unit j): x = t + threads u
+    float h[EP], b3[EP][3], g[EP][3];
+    uint32_t at[EP], at3[EP]; // element of a step's [B][H] and [B][3H]
+    auto own = [&](int u) { return (kGruRows * H) % kGruThreads == 0 || t + kGruThreads * u < kGruRows * H; };
+#pragma unroll
+    for (int u = 0; u < EP; ++u) {
+        const int x = t + kGruThreads * u, r = x / H, j = x % H;
+        const int rr = own(u) ? r : 0, jj = own(u) ? j : 0;
+        at[u] = (uint32_t)(row0 + rr) * H + jj;
+        at3[u] = (uint32_t)(row0 + rr) * 3 * H + jj;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            b3[u][q] = bhh[q * H + jj];
+            g[u][q] = gi[at3[u] + q * H];
+        }
+        h[u] = h0 && row0 + rr < h0_rows ? h0[at[u]] : 0.0f;
+        if (own(u)) {
+            const uint16_t hv = (uint16_t)f2bf_pk(h[u], 0.0f);
+            hs[at[u]] = h[u];
+            hb[at[u]] = hv;
+            sh[r * LH + j] = hv;
+        }
+    }
+    __syncthreads();
+    for (int32_t k = 0; k < T; ++k) {
+        const int64_t step = (int64_t)k * B;
+        float gn[EP][3]; // the next step's input projections
+        const float* gk = gi + (k + 1 < T ? step + B : step) * 3 * H;
+        float* ghk = gh + step * 3 * H;
+        float* hsk = hs + (step + B) * H;
+        uint16_t* hbk = hb + (step + B) * H;
+#pragma unroll
+        for (int u = 0; u < EP; ++u)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) gn[u][q] = gk[at3[u] + q * H];
+        const uint16_t* ph = sh + (lane & (kGruRows - 1)) * LH + (lane >> 4) * 8;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int tile = wid + kGruWaves * i;
+            if (tile >= NT) break; // uniform
+            const f32x4v p = gru_product<G>(w, i, ph, lane >= 32);
+            if ((lane & 15) < kGruRows)
+                *reinterpret_cast<f32x4v*>(sg + (lane & 15) * LG + tile * 16 + 4 * (lane >> 4)) = p;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < EP; ++u) {
+            if (!own(u)) continue;
+            const int x = t + kGruThreads * u, r = x / H, j = x % H;
+            const float c0 = sg[r * LG + j] + b3[u][0], c1 = sg[r * LG + H + j] + b3[u][1],
+                        c2 = sg[r * LG + 2 * H + j] + b3[u][2];
+            ghk[at3[u]] = c0;
+            ghk[at3[u] + H] = c1;
+            ghk[at3[u] + 2 * H] = c2;
+            const float rr = sigm(g[u][0] + c0);
+            const float z = sigm(g[u][1] + c1);
+            const float n = tanhf(g[u][2] + rr * c2);
+            h[u] = fmaf(1.0f - z, n, z * h[u]);
+            const uint16_t hv = (uint16_t)f2bf_pk(h[u], 0.0f);
+            hsk[at[u]] = h[u];
+            hbk[at[u]] = hv;
+            sh[r * LH + j] = hv;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) g[u][q] = gn[u][q];
+        }
+        __syncthreads();
+    }
+}
+
+// Backward through the sequence.  dho [T][B][H] gradients from the readout;
+// writes dgi and dgh in bf16 [T][B][3H], and in FP32 dg [T][B][4H] = dr, dz, dn
+// (of gi) and dn r (of gh), whose sums are the bias gradients.
+template <int G>
+__global__ __launch_bounds__(64 * kGruBwdWaves) void gru_seq_backward_kernel(int32_t T, int32_t B,
+                                                                      const float* __restrict__ gi,
+                                                                      const float* __restrict__ gh,
+                                                                      const float* __restrict__ hs,
+                                                                      const float* __restrict__ dho,
+                                                                      const uint16_t* __restrict__ WT,
+                                                                      uint16_t* __restrict__ dgib,
+                                                                      uint16_t* __restrict__ dghb,
+                                                                      float* __restrict__ dg)
+{
+    constexpr int kGruWaves = kGruBwdWaves, kGruThreads = 64 * kGruWaves;
+    constexpr int H = 32 * G, NT = H / 16, TW = (NT + kGruWaves - 1) / kGruWaves, KS = 3 * G;
+    constexpr int EP = (kGruRows * H + kGruThreads - 1) / kGruThreads;
+    constexpr int LG = 3 * H + 8, LD = H + 4;
+    __shared__ __align__(16) uint16_t sg[kGruRows * LG]; // dgh of the step, bf16
+    __shared__ __align__(16) float sd[kGruRows * LD];    // its product with W_hh
+    const int t = threadIdx.x, lane = t & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int row0 = blockIdx.x * kGruRows;
+    extern __shared__ __align__(16) uint16_t sw[];
+    GruWeights<TW, KS, kGruWaves, kGruBwdHeld> w;
+    w.load(WT, NT, wid, lane, sw);
+    struct In {
+        float gi[3], gh[3], h, dho;
+    };
+    uint32_t at[EP], at3[EP]; // element of a step's [B][H] and [B][3H]
+    auto own = [&](int u) { return (kGruRows * H) % kGruThreads == 0 || t + kGruThreads * u < kGruRows * H; };
+    float dhz[EP];
+    In cur[EP];
+    auto load = [&](In& v, int u, int64_t k) {
+        const float* gik = gi + k * B * 3 * H;
+        const float* ghk = gh + k * B * 3 * H;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            v.gi[q] = gik[at3[u] + q * H];
+            v.gh[q] = ghk[at3[u] + q * H];
+        }
+        v.h = (hs + k * B * H)[at[u]];
+        v.dho = (dho + k * B * H)[at[u]];
+    };
+#pragma unroll
+    for (int u = 0; u < EP; ++u) {
+        const int x = t + kGruThreads * u;
+        const int r = own(u) ? x / H : 0, j = own(u) ? x % H : 0;
+        at[u] = (uint32_t)(row0 + r) * H + j;
+        at3[u] = (uint32_t)(row0 + r) * 3 * H + j;
+        dhz[u] = 0.0f;
+        load(cur[u], u, T - 1);
+    }
+    for (int32_t k = T - 1; k >= 0; --k) {
+        In next[EP];
+#pragma unroll
+        for (int u = 0; u < EP; ++u) load(next[u], u, k > 0 ? k - 1 : 0);
+#pragma unroll
+        for (int u = 0; u < EP; ++u) {
+            if (!own(u)) continue;
+            const int x = t + kGruThreads * u, r = x / H, j = x % H;
+            const In& v = cur[u];
+            const float rr = sigm(v.gi[0] + v.gh[0]);
+            const float z = sigm(v.gi[1] + v.gh[1]);
+            const float n = tanhf(v.gi[2] + rr * v.gh[2]);
+            float d = v.dho;
+            if (k < T - 1) {
+                d += dhz[u];
+                d += sd[r * LD + j] + 0.0f;
+            }
+            const float dn = d * (1.0f - z) * (1.0f - n * n);
+            const float dz = d * (v.h - n) * z * (1.0f - z);
+            const float dr = dn * v.gh[2] * rr * (1.0f - rr);
+            const float dnr = dn * rr;
+            dhz[u] = d * z;
+            const uint32_t a = f2bf_pk(dr, dz), c = f2bf_pk(dn, dnr);
+            uint16_t* gib = dgib + (int64_t)k * B * 3 * H;
+            uint16_t* ghb = dghb + (int64_t)k * B * 3 * H;
+            gib[at3[u]] = (uint16_t)a;
+            gib[at3[u] + H] = (uint16_t)(a >> 16);
+            gib[at3[u] + 2 * H] = (uint16_t)c;
+            ghb[at3[u]] = (uint16_t)a;
+            ghb[at3[u] + H] = (uint16_t)(a >> 16);
+            ghb[at3[u] + 2 * H] = (uint16_t)(c >> 16);
+            uint16_t* p = sg + r * LG + j;
+            p[0] = (uint16_t)a;
+            p[H] = (uint16_t)(a >> 16);
+            p[2 * H] = (uint16_t)(c >> 16);
+            float* g4 = dg + (int64_t)k * B * 4 * H + at3[u] + (at3[u] - j) / 3; // row * 4H + j
+            g4[0] = dr;
+            g4[H] = dz;
+            g4[2 * H] = dn;
+            g4[3 * H] = dnr;
+        }
+        __syncthreads();
+        if (k == 0) break; // uniform: nothing before the first step
+        const uint16_t* ph = sg + (lane & (kGruRows - 1)) * LG + (lane >> 4) * 8;
+#pragma unroll
+        for (int i = 0; i < TW; ++i) {
+            const int tile = wid + kGruWaves * i;
+            if (tile >= NT) break; // uniform
+            const f32x4v p = gru_product<KS>(w, i, ph, lane >= 32);
+            if ((lane & 15) < kGruRows)
+                *reinterpret_cast<f32x4v*>(sd + (lane & 15) * LD + tile * 16 + 4 * (lane >> 4)) = p;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < EP; ++u) cur[u] = next[u];
+    }
+}
+
+// Row-major bf16 [K][N] (row stride ld) into the fragment order of [N][K]:
+// tile q of matrix i for first[i] <= q < first[i + 1], 32 rows x 32 columns.
+struct PackArgs {
+    int32_t n;
+    int32_t first[kMlpMaxLayers * 2 + 1];
+    int32_t K[kMlpMaxLayers * 2], N[kMlpMaxLayers * 2];
+    const uint16_t* in[kMlpMaxLayers * 2];
+    int64_t ld[kMlpMaxLayers * 2];
+    uint16_t* out[kMlpMaxLayers * 2];
+};
+
+__global__ __launch_bounds__(256) void pack_transposed_kernel(PackArgs a)
+{
+    __shared__ uint16_t tb[32][34]; // [k][n]
+    int i = 0;
+    while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+    const int tn = a.N[i] / 32, tile = blockIdx.x - a.first[i];
+    const int k0 = tile / tn * 32, n0 = tile % tn * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) tb[ty + 8 * u][tx] = a.in[i][(int64_t)(k0 + ty + 8 * u) * a.ld[i] + n0 + tx];
+    __syncthreads();
+    const int x = threadIdx.x * 4;
+    const int k = x / 512 * 16 + x % 512 / 256 * 8 + x % 8, n = x % 256 / 8;
+    *reinterpret_cast<ushort4*>(a.out[i] + frag_at(a.K[i], n0, k0) + x) =
+        make_ushort4(tb[k][n], tb[k + 1][n], tb[k + 2][n], tb[k + 3][n]);
+}
+
+// Gradient and loss of a sequence's outputs [T][B][O]: targets and mask
+// [T][rows][n_out] (masked out past rows and n_out), the arithmetic of
+// affine_kernel and mse_grad_kernel.
+__global__ __launch_bounds__(256) void seq_loss_kernel(int64_t n, int32_t B, int32_t O, int32_t rows, int32_t n_out,
+                                                       const float* __restrict__ out, const float* __restrict__ Y,
+                                                       const float* __restrict__ ys, const float* __restrict__ yh,
+                                                       const float* __restrict__ mask, float scale,
+                                                       float* __restrict__ grad, uint16_t* __restrict__ gradb,
+                                                       float* __restrict__ lsum)
+{
+    __shared__ float red[256];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    float e = 0.0f;
+    if (i < n) {
+        const int32_t c = (int32_t)(i % O);
+        const int64_t tb = i / O;
+        const int32_t b = (int32_t)(tb % B);
+        float tgt = 0.0f, mk = 0.0f;
+        if (c < n_out) tgt = yh[c]; // a padded row's target is the shift of a zero
+        if (c < n_out && b < rows) {
+            const int64_t x = (tb / B * rows + b) * n_out + c;
+            tgt = Y[x] * ys[c] + yh[c];
+            mk = mask ? mask[x] : 1.0f;
+        }
+        const float d = (out[i] - tgt) * mk;
+        e = d * d;
+        const float g = scale * d;
+        grad[i] = g;
+        gradb[i] = f2bf(g);
+    }
+    red[threadIdx.x] = e;
+    __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) lsum[blockIdx.x] = red[0];
+}
+
+template <int G>
+using GruFwdWeights = GruWeights<(6 * G + kGruFwdWaves - 1) / kGruFwdWaves, G, kGruFwdWaves, kGruFwdHeld>;
+template <int G>
+using GruBwdWeights = GruWeights<(2 * G + kGruBwdWaves - 1) / kGruBwdWaves, 3 * G, kGruBwdWaves, kGruBwdHeld>;
 
 static inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
@@ -1217,7 +1629,7 @@ int dtb_mlp_relu_backward(int64_t n, const float* dY, const float* Z, float* dZ,
 int dtb_mlp_bias_grad(int32_t M, int32_t N, const float* dZ, float* db, void* stream)
 {
     DTB_REQUIRE(M > 0 && N > 0 && dZ && db, "bad arguments");
-    hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((N + kBiasCols - 1) / kBiasCols)), dim3(kBiasCols * kBiasRows),
+    hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned)((N + kBiasCols - 1) / kBiasCols)), dim3(kBiasThreads),
                        0, (hipStream_t)stream, M, N, dZ, db);
     DTB_TRY_HIP(hipGetLastError());
     return DTB_OK;
@@ -1389,6 +1801,7 @@ int dtb_mlp_train_gradients(int32_t n_layers, const dtb_mlp_layer* layers, int32
     d.B = B;
     for (int32_t l = 0; l < n_layers; ++l) {
         d.in[l] = a.l[l].in; d.out[l] = a.l[l].out;
+        d.ldh[l] = d.ldg[l] = B; d.parts[l] = B / 32;
         d.hT[l] = a.l[l].hT; d.gT[l] = a.l[l].gT; d.dbp[l] = a.l[l].dbp;
         d.dW[l] = layers[l].dw; d.db[l] = layers[l].db;
         d.first[l + 1] = d.first[l] + (a.l[l].out + 63) / 64 * ((a.l[l].in + 63) / 64);
@@ -1464,6 +1877,154 @@ int dtb_gru_backward(int32_t B, int32_t H, const float* gi, const float* gh, con
     DTB_REQUIRE(B > 0 && H > 0 && gi && gh && h && dh_a && dgi && dgh && dh_z, "bad arguments");
     hipLaunchKernelGGL(gru_backward_kernel, g1((int64_t)B * H), dim3(256), 0, (hipStream_t)stream, B, H, gi, gh, h,
                        dh_a, dh_b, dh_c, dgi, (uint16_t*)dgib, dgh, (uint16_t*)dghb, dh_z);
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+
+int dtb_gru_sequence_fits(int32_t B, int32_t H)
+{
+    // the products must be ones that dtb_mlp_gemm_bf16_nt splits over K
+    if (B > 0 && B % 32 == 0 && H > 0 && H % 32 == 0 && H <= 256 && !gemm_one_chain(B, 3 * H) && !gemm_one_chain(B, H))
+        return DTB_OK;
+    set_error("the sequence kernels take B and H multiples of 32, H <= 256 and products of fewer than 256 tiles");
+    return DTB_UNSUPPORTED;
+}
+
+static int gru_lds(const void* kernel, int bytes)
+{
+    if (bytes > 0) DTB_TRY_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    return DTB_OK;
+}
+
+int dtb_gru_sequence_forward(int32_t T, int32_t B, int32_t H, const float* gi, const void* w_hh, const float* b_hh,
+                             const float* h0, int32_t h0_rows, float* gh, float* hs, void* hb, void* stream)
+{
+    DTB_TRY(dtb_gru_sequence_fits(B, H));
+    DTB_REQUIRE(T > 0 && gi && w_hh && b_hh && gh && hs && hb && (!h0 || (h0_rows >= 0 && h0_rows <= B)), "bad arguments");
+    DTB_REQUIRE((reinterpret_cast<uintptr_t>(w_hh) & 15) == 0, "W_hh must be 16-byte aligned");
+    const dim3 g((unsigned)(B / kGruRows)), b(64 * kGruFwdWaves);
+    const uint16_t* w = (const uint16_t*)w_hh;
+    switch (H / 32) {
+#define DTB_GRU_CASE(G)                                                                                              \
+    case G:                                                                                                          \
+        DTB_TRY(gru_lds((const void*)gru_seq_forward_kernel<G>, GruFwdWeights<G>::kLds));                \
+        hipLaunchKernelGGL(gru_seq_forward_kernel<G>, g, b, (GruFwdWeights<G>::kLds),                   \
+                           (hipStream_t)stream, T, B, gi, w, b_hh, h0, h0_rows, gh, hs, (uint16_t*)hb);               \
+        break;
+        DTB_GRU_CASE(1) DTB_GRU_CASE(2) DTB_GRU_CASE(3) DTB_GRU_CASE(4) DTB_GRU_CASE(5) DTB_GRU_CASE(6) DTB_GRU_CASE(7)
+        DTB_GRU_CASE(8)
+#undef DTB_GRU_CASE
+    }
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_gru_sequence_backward(int32_t T, int32_t B, int32_t H, const float* gi, const float* gh, const float* hs,
+                              const float* dho, const void* w_hh_t, void* dgib, void* dghb, float* dg, void* stream)
+{
+    DTB_TRY(dtb_gru_sequence_fits(B, H));
+    DTB_REQUIRE(T > 0 && gi && gh && hs && dho && w_hh_t && dgib && dghb && dg, "bad arguments");
+    DTB_REQUIRE((reinterpret_cast<uintptr_t>(w_hh_t) & 15) == 0, "the transpose of W_hh must be 16-byte aligned");
+    const dim3 g((unsigned)(B / kGruRows)), b(64 * kGruBwdWaves);
+    const uint16_t* w = (const uint16_t*)w_hh_t;
+    switch (H / 32) {
+#define DTB_GRU_CASE(G)                                                                                              \
+    case G:                                                                                                          \
+        DTB_TRY(gru_lds((const void*)gru_seq_backward_kernel<G>, GruBwdWeights<G>::kLds));           \
+        hipLaunchKernelGGL(gru_seq_backward_kernel<G>, g, b, (GruBwdWeights<G>::kLds),               \
+                           (hipStream_t)stream, T, B, gi, gh, hs, dho, w, (uint16_t*)dgib, (uint16_t*)dghb, dg);      \
+        break;
+        DTB_GRU_CASE(1) DTB_GRU_CASE(2) DTB_GRU_CASE(3) DTB_GRU_CASE(4) DTB_GRU_CASE(5) DTB_GRU_CASE(6) DTB_GRU_CASE(7)
+        DTB_GRU_CASE(8)
+#undef DTB_GRU_CASE
+    }
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_sequence_loss(int32_t T, int32_t B, int32_t O, int32_t rows, int32_t n_out, const float* out,
+                          const float* Y, const float* y_scale, const float* y_shift, const float* mask, float scale,
+                          float* grad, void* gradb, float* lsum, void* stream)
+{
+    DTB_REQUIRE(T > 0 && B > 0 && O > 0 && rows >= 0 && rows <= B && n_out >= 0 && n_out <= O && out &&
+                    (Y || rows == 0 || n_out == 0) && y_scale && y_shift && grad && gradb && lsum,
+                "bad arguments");
+    const int64_t n = (int64_t)T * B * O;
+    hipLaunchKernelGGL(seq_loss_kernel, g1(n), dim3(256), 0, (hipStream_t)stream, n, B, O, rows, n_out, out, Y, y_scale,
+                       y_shift, mask, scale, grad, (uint16_t*)gradb, lsum);
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_pack_transposed(int32_t n, const dtb_pack_item* p, void* stream)
+{
+    DTB_REQUIRE(n >= 0 && n <= 2 * kMlpMaxLayers && (n == 0 || p), "at most %d matrices", 2 * kMlpMaxLayers);
+    PackArgs a{};
+    a.n = n;
+    int64_t tiles = 0;
+    for (int32_t i = 0; i < n; ++i) {
+        DTB_REQUIRE(p[i].rows > 0 && p[i].cols > 0 && p[i].rows % 32 == 0 && p[i].cols % 32 == 0 &&
+                        p[i].rows < (1ll << 30) && p[i].cols < (1 << 24) && p[i].ld >= p[i].cols && p[i].in &&
+                        p[i].out && (reinterpret_cast<uintptr_t>(p[i].out) & 15) == 0,
+                    "matrix %d: bad arguments", i);
+        a.K[i] = (int32_t)p[i].rows; a.N[i] = (int32_t)p[i].cols; a.ld[i] = p[i].ld;
+        a.in[i] = (const uint16_t*)p[i].in; a.out[i] = (uint16_t*)p[i].out;
+        tiles += p[i].rows / 32 * (p[i].cols / 32);
+        DTB_REQUIRE(tiles < (1ll << 31), "too many tiles for one launch");
+        a.first[i + 1] = (int32_t)tiles;
+    }
+    if (tiles == 0) return DTB_OK;
+    hipLaunchKernelGGL(pack_transposed_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, a);
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_column_sums(int32_t n, const dtb_colsum_item* p, int64_t rows, void* stream)
+{
+    DTB_REQUIRE(n >= 1 && n <= kMlpMaxLayers && p && rows >= 0, "1 to %d arrays", kMlpMaxLayers);
+    ColsumArgs a{};
+    a.n = n;
+    a.rows = rows;
+    int64_t wgs = 0;
+    for (int32_t i = 0; i < n; ++i) {
+        DTB_REQUIRE(p[i].cols > 0 && p[i].cols < (1 << 30) && p[i].ld >= p[i].cols && (p[i].src || rows == 0) && p[i].dst,
+                    "array %d: bad arguments", i);
+        a.cols[i] = (int32_t)p[i].cols; a.ld[i] = p[i].ld; a.src[i] = p[i].src;
+        a.dst[i] = p[i].dst; a.dst2[i] = p[i].dst2;
+        wgs += (p[i].cols + kBiasCols - 1) / kBiasCols;
+        DTB_REQUIRE(wgs < (1ll << 31), "too many columns for one launch");
+        a.first[i + 1] = (int32_t)wgs;
+    }
+    hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)wgs), dim3(kBiasThreads), 0, (hipStream_t)stream, a);
+    DTB_TRY_HIP(hipGetLastError());
+    return DTB_OK;
+}
+
+int dtb_mlp_weight_gradients(int32_t n, const dtb_dw_item* p, int32_t rows, void* stream)
+{
+    DTB_REQUIRE(n >= 1 && n <= kMlpMaxLayers && p && rows > 0 && rows % 32 == 0, "1 to %d products over a multiple of 32 rows",
+                kMlpMaxLayers);
+    MlpDwArgs d{};
+    d.layers = n;
+    d.B = rows;
+    int64_t tiles = 0;
+    for (int32_t l = 0; l < n; ++l) {
+        DTB_REQUIRE(p[l].n_in > 0 && p[l].n_out > 0 && p[l].n_in % 32 == 0 && p[l].n_out % 32 == 0 &&
+                        p[l].n_in < (1 << 24) && p[l].n_out < (1 << 24) && p[l].h && p[l].g && p[l].dw &&
+                        p[l].ldh >= rows && p[l].ldg >= rows && p[l].ldh % 32 == 0 && p[l].ldg % 32 == 0 &&
+                        ((reinterpret_cast<uintptr_t>(p[l].h) | reinterpret_cast<uintptr_t>(p[l].g)) & 15) == 0 &&
+                        (!p[l].db || (p[l].dbp && p[l].parts >= 0)),
+                    "product %d: bad arguments", l);
+        d.in[l] = (int32_t)p[l].n_in; d.out[l] = (int32_t)p[l].n_out;
+        d.ldh[l] = p[l].ldh; d.ldg[l] = p[l].ldg; d.parts[l] = (int32_t)p[l].parts;
+        d.hT[l] = (const uint16_t*)p[l].h; d.gT[l] = (const uint16_t*)p[l].g; d.dbp[l] = p[l].dbp;
+        d.dW[l] = p[l].dw; d.db[l] = p[l].db;
+        tiles += (p[l].n_out + 63) / 64 * ((p[l].n_in + 63) / 64);
+        DTB_REQUIRE(tiles < (1ll << 31), "too many tiles for one launch");
+        d.first[l + 1] = (int32_t)tiles;
+    }
+    hipLaunchKernelGGL(mlp_dw_kernel, dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream, d);
     DTB_TRY_HIP(hipGetLastError());
     return DTB_OK;
 }

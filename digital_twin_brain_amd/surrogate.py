@@ -268,11 +268,12 @@ class GRUSurrogate:
     library's kernels.
 
     Forward over a sequence X [T, B, n_in]: one GEMM for every step's input
-    projection, then per step a recurrent GEMM and the fused gate kernel,
-    then one GEMM for every step's readout.  Backward: one GEMM each for the
-    readout gradients, per step (reverse order) the fused gate backward and
-    the recurrent-gradient GEMM, then one GEMM each for dW_ih and dW_hh over
-    all T*B rows."""
+    projection, one kernel for all steps of the recurrence, one GEMM for every
+    step's readout.  Backward: the loss and its gradient, one GEMM to the
+    hidden states, one kernel for all steps in reverse, then all weight
+    gradients over the T*B rows together.  Hidden sizes past 256 (or batches
+    whose products the sequence kernels do not take) run a recurrent GEMM and
+    a gate kernel per step instead."""
 
     def __init__(self, n_in, n_out, hidden=256, max_batch=64, max_steps=32, device=0, seed=0, lr=1e-3,
                  betas=(0.9, 0.999), eps=1e-8):
@@ -301,7 +302,6 @@ class GRUSurrogate:
         self.pb = {k: torch.empty(self.p[k].shape, **bf) for k in ("W_ih", "W_hh", "W_o")}
         self.pbT = {k: torch.empty(tuple(reversed(self.p[k].shape)), **bf) for k in ("W_hh", "W_o")}
         B, T = self.max_batch, self.max_steps
-        self.X = torch.empty((T * B, I), **f32)
         self.Xb = torch.empty((T * B, I), **bf)
         self.XbT = torch.empty((I, T * B), **bf)
         self.Gi = torch.empty((T * B, 3 * H), **f32)
@@ -310,19 +310,20 @@ class GRUSurrogate:
         self.Hb = torch.empty(((T + 1) * B, H), **bf)
         self.HbT = torch.empty((H, (T + 1) * B), **bf)
         self.Y = torch.empty((T * B, O), **f32)
-        self.Tg = torch.empty((T * B, O), **f32)
-        self.M = torch.empty((T * B, O), **f32)
         self.Gy = torch.empty((T * B, O), **f32)
         self.Gyb = torch.empty((T * B, O), **bf)
         self.GybT = torch.empty((O, T * B), **bf)
         self.dHo = torch.empty((T * B, H), **f32)
-        self.dGi = torch.empty((T * B, 3 * H), **f32)
         self.dGib = torch.empty((T * B, 3 * H), **bf)
-        self.dGh = torch.empty((T * B, 3 * H), **f32)
         self.dGhb = torch.empty((T * B, 3 * H), **bf)
-        self.dGT = torch.empty((3 * H, T * B), **bf)
-        self.dhz = torch.empty((B, H), **f32)
-        self.dhg = torch.empty((B, H), **f32)
+        self.dGiT = torch.empty((3 * H, T * B), **bf)
+        self.dGhT = torch.empty((3 * H, T * B), **bf)
+        # every batch up to max_batch takes the sequence kernels, or none does
+        self.sequence = self.lib.dtb_gru_sequence_fits(B, H) == nat.DTB_OK
+        if self.sequence:
+            self.dG = torch.empty((T * B, 4 * H), **f32)
+        else:
+            self._alloc_steps()
         self.lsum = torch.empty(((T * B * O + 255) // 256,), **f32)
         self.x_scale = torch.ones(self.n_in, **f32)
         self.x_shift = torch.zeros(self.n_in, **f32)
@@ -335,13 +336,19 @@ class GRUSurrogate:
     def _stream(self):
         return torch.cuda.current_stream(self.dev).cuda_stream
 
+    def _alloc_steps(self):
+        """Buffers of the launch-per-step path."""
+        B, T, H = self.max_batch, self.max_steps, self.H
+        f32 = dict(dtype=torch.float32, device=self.dev)
+        self.dGi = torch.empty((T * B, 3 * H), **f32)
+        self.dGh = torch.empty((T * B, 3 * H), **f32)
+        self.dhz = torch.empty((B, H), **f32)
+        self.dhg = torch.empty((B, H), **f32)
+
     def _refresh_bf16(self):
-        s = self._stream()
-        for k in ("W_ih", "W_hh", "W_o"):
-            r, c = self.p[k].shape
-            nat.check(self.lib.dtb_mlp_f32_to_bf16(r * c, self.p[k].data_ptr(), self.pb[k].data_ptr(), s))
-            if k in self.pbT:
-                nat.check(self.lib.dtb_mlp_transpose_bf16(r, c, self.pb[k].data_ptr(), self.pbT[k].data_ptr(), s))
+        table = _params([(w.shape[0], w.shape[1], w, None, None, None, self.pb[k], self.pbT.get(k), None, None)
+                         for k, w in self.p.items() if k in self.pb])
+        nat.check(self.lib.dtb_mlp_refresh_bf16(len(table), table.ctypes.data, self._stream()))
 
     def set_normalization(self, X, Y):
         """Per-feature standardisation over every step and sequence."""
@@ -360,22 +367,32 @@ class GRUSurrogate:
         assert T <= self.max_steps and r <= self.max_batch
         B = _pad(r)
         H, I, O = self.H, self.I, self.O
-        Xp = torch.zeros((T, B, self.n_in), dtype=torch.float32, device=self.dev)
-        Xp[:, :r] = torch.as_tensor(X).to(self.dev, torch.float32)
+        X = torch.as_tensor(X).to(self.dev, torch.float32)
+        Xp = X.expand(T, r, self.n_in).contiguous()
+        if r < B:
+            Xp = torch.zeros((T, B, self.n_in), dtype=torch.float32, device=self.dev)
+            Xp[:, :r] = X
         nat.check(self.lib.dtb_mlp_affine(T * B, self.n_in, I, Xp.data_ptr(), self.n_in, self.x_scale.data_ptr(),
                                           self.x_shift.data_ptr(), None, self.Xb.data_ptr(), I, s))
         self._gemm(T * B, 3 * H, I, self.Xb, I, self.pb["W_ih"], I, self.p["b_ih"], self.Gi, 3 * H)
-        self.Hs[:B].zero_()
         if h0 is not None:
-            self.Hs[:r].copy_(torch.as_tensor(h0).to(self.dev, torch.float32))
-        nat.check(self.lib.dtb_mlp_f32_to_bf16(B * H, self.Hs.data_ptr(), self.Hb.data_ptr(), s))
-        for t in range(T):
-            hb = self.Hb[t * B:(t + 1) * B]
-            gh = self.Gh[t * B:(t + 1) * B]
-            self._gemm(B, 3 * H, H, hb, H, self.pb["W_hh"], H, self.p["b_hh"], gh, 3 * H)
-            nat.check(self.lib.dtb_gru_forward(B, H, self.Gi[t * B:].data_ptr(), gh.data_ptr(),
-                                               self.Hs[t * B:].data_ptr(), self.Hs[(t + 1) * B:].data_ptr(),
-                                               self.Hb[(t + 1) * B:].data_ptr(), s))
+            h0 = torch.as_tensor(h0).to(self.dev, torch.float32).expand(r, H).contiguous()
+        if self.sequence:
+            nat.check(self.lib.dtb_gru_sequence_forward(T, B, H, self.Gi.data_ptr(), self.pb["W_hh"].data_ptr(),
+                                                        self.p["b_hh"].data_ptr(), nat.ptr(h0), r, self.Gh.data_ptr(),
+                                                        self.Hs.data_ptr(), self.Hb.data_ptr(), s))
+        else:
+            self.Hs[:B].zero_()
+            if h0 is not None:
+                self.Hs[:r].copy_(h0)
+            nat.check(self.lib.dtb_mlp_f32_to_bf16(B * H, self.Hs.data_ptr(), self.Hb.data_ptr(), s))
+            for t in range(T):
+                hb = self.Hb[t * B:(t + 1) * B]
+                gh = self.Gh[t * B:(t + 1) * B]
+                self._gemm(B, 3 * H, H, hb, H, self.pb["W_hh"], H, self.p["b_hh"], gh, 3 * H)
+                nat.check(self.lib.dtb_gru_forward(B, H, self.Gi[t * B:].data_ptr(), gh.data_ptr(),
+                                                   self.Hs[t * B:].data_ptr(), self.Hs[(t + 1) * B:].data_ptr(),
+                                                   self.Hb[(t + 1) * B:].data_ptr(), s))
         self._gemm(T * B, O, H, self.Hb[B:], H, self.pb["W_o"], H, self.p["b_o"], self.Y, O)
         return T, r, B
 
@@ -394,46 +411,55 @@ class GRUSurrogate:
         T, r, B = self._forward(X, h0)
         H, I, O = self.H, self.I, self.O
         TB = T * B
-        Yp = torch.zeros((T, B, self.n_out), dtype=torch.float32, device=self.dev)
-        Yp[:, :r] = torch.as_tensor(Y).to(self.dev, torch.float32)
-        nat.check(self.lib.dtb_mlp_affine(TB, self.n_out, O, Yp.data_ptr(), self.n_out, self.y_scale.data_ptr(),
-                                          self.y_shift.data_ptr(), self.Tg.data_ptr(), None, O, s))
-        M = self.M[:TB].view(T, B, O)
-        M.zero_()
-        if mask is None:
-            M[:, :r, :self.n_out] = 1.0
-        else:
-            M[:, :r, :self.n_out] = torch.as_tensor(mask).to(self.dev, torch.float32)
-        nat.check(self.lib.dtb_mlp_mse_grad(TB * O, self.Y.data_ptr(), self.Tg.data_ptr(), self.M.data_ptr(),
-                                            1.0 / (T * r), self.Gy.data_ptr(), self.Gyb.data_ptr(),
-                                            self.lsum.data_ptr(), s))
-        # readout
-        tr = self.lib.dtb_mlp_transpose_bf16
-        nat.check(tr(TB, O, self.Gyb.data_ptr(), self.GybT.data_ptr(), s))
-        nat.check(tr(TB, H, self.Hb[B:].data_ptr(), self.HbT.data_ptr(), s))
-        self._gemm(O, H, TB, self.GybT, TB, self.HbT, TB, None, self.grad["W_o"], H)
-        nat.check(self.lib.dtb_mlp_bias_grad(TB, O, self.Gy.data_ptr(), self.grad["b_o"].data_ptr(), s))
+        Yd = torch.as_tensor(Y).to(self.dev, torch.float32).expand(T, r, self.n_out).contiguous()
+        Md = None if mask is None else \
+            torch.as_tensor(mask).to(self.dev, torch.float32).expand(T, r, self.n_out).contiguous()
+        nat.check(self.lib.dtb_mlp_sequence_loss(T, B, O, r, self.n_out, self.Y.data_ptr(), Yd.data_ptr(),
+                                                 self.y_scale.data_ptr(), self.y_shift.data_ptr(), nat.ptr(Md),
+                                                 1.0 / (T * r), self.Gy.data_ptr(), self.Gyb.data_ptr(),
+                                                 self.lsum.data_ptr(), s))
         self._gemm(TB, H, O, self.Gyb, O, self.pbT["W_o"], O, None, self.dHo, H)
         # recurrence, last step first
-        for t in range(T - 1, -1, -1):
-            last = t == T - 1
-            nat.check(self.lib.dtb_gru_backward(
-                B, H, self.Gi[t * B:].data_ptr(), self.Gh[t * B:].data_ptr(), self.Hs[t * B:].data_ptr(),
-                self.dHo[t * B:].data_ptr(), None if last else self.dhz.data_ptr(),
-                None if last else self.dhg.data_ptr(), self.dGi[t * B:].data_ptr(), self.dGib[t * B:].data_ptr(),
-                self.dGh[t * B:].data_ptr(), self.dGhb[t * B:].data_ptr(), self.dhz.data_ptr(), s))
-            if t > 0:
-                self._gemm(B, H, 3 * H, self.dGhb[t * B:(t + 1) * B], 3 * H, self.pbT["W_hh"], 3 * H, None, self.dhg,
-                           H)
-        # weight gradients over all T*B rows
-        nat.check(tr(TB, 3 * H, self.dGib.data_ptr(), self.dGT.data_ptr(), s))
-        nat.check(tr(TB, I, self.Xb.data_ptr(), self.XbT.data_ptr(), s))
-        self._gemm(3 * H, I, TB, self.dGT, TB, self.XbT, TB, None, self.grad["W_ih"], I)
-        nat.check(tr(TB, 3 * H, self.dGhb.data_ptr(), self.dGT.data_ptr(), s))
-        nat.check(tr(TB, H, self.Hb.data_ptr(), self.HbT.data_ptr(), s))
-        self._gemm(3 * H, H, TB, self.dGT, TB, self.HbT, TB, None, self.grad["W_hh"], H)
-        nat.check(self.lib.dtb_mlp_bias_grad(TB, 3 * H, self.dGi.data_ptr(), self.grad["b_ih"].data_ptr(), s))
-        nat.check(self.lib.dtb_mlp_bias_grad(TB, 3 * H, self.dGh.data_ptr(), self.grad["b_hh"].data_ptr(), s))
+        if self.sequence:
+            nat.check(self.lib.dtb_gru_sequence_backward(
+                T, B, H, self.Gi.data_ptr(), self.Gh.data_ptr(), self.Hs.data_ptr(), self.dHo.data_ptr(),
+                self.pbT["W_hh"].data_ptr(), self.dGib.data_ptr(), self.dGhb.data_ptr(), self.dG.data_ptr(),
+                s))
+            dg = self.dG.data_ptr()
+            sums = np.array([(2 * H, 4 * H, dg, self.grad["b_ih"].data_ptr(), self.grad["b_hh"].data_ptr()),
+                             (H, 4 * H, dg + 8 * H, self.grad["b_ih"].data_ptr() + 8 * H, 0),
+                             (H, 4 * H, dg + 12 * H, self.grad["b_hh"].data_ptr() + 8 * H, 0),
+                             (O, O, self.Gy.data_ptr(), self.grad["b_o"].data_ptr(), 0)], dtype=np.int64)
+            nat.check(self.lib.dtb_mlp_column_sums(len(sums), sums.ctypes.data, TB, s))
+        else:
+            for t in range(T - 1, -1, -1):
+                last = t == T - 1
+                nat.check(self.lib.dtb_gru_backward(
+                    B, H, self.Gi[t * B:].data_ptr(), self.Gh[t * B:].data_ptr(), self.Hs[t * B:].data_ptr(),
+                    self.dHo[t * B:].data_ptr(), None if last else self.dhz.data_ptr(),
+                    None if last else self.dhg.data_ptr(), self.dGi[t * B:].data_ptr(), self.dGib[t * B:].data_ptr(),
+                    self.dGh[t * B:].data_ptr(), self.dGhb[t * B:].data_ptr(), self.dhz.data_ptr(), s))
+                if t > 0:
+                    self._gemm(B, H, 3 * H, self.dGhb[t * B:(t + 1) * B], 3 * H, self.pbT["W_hh"], 3 * H, None,
+                               self.dhg, H)
+            nat.check(self.lib.dtb_mlp_bias_grad(TB, 3 * H, self.dGi.data_ptr(), self.grad["b_ih"].data_ptr(), s))
+            nat.check(self.lib.dtb_mlp_bias_grad(TB, 3 * H, self.dGh.data_ptr(), self.grad["b_hh"].data_ptr(), s))
+            nat.check(self.lib.dtb_mlp_bias_grad(TB, O, self.Gy.data_ptr(), self.grad["b_o"].data_ptr(), s))
+        # weight gradients over all T*B rows, from transposed operands in fragment order
+        KH = (T + 1) * B  # the states before (first T*B) and after (last T*B) every step
+        pack = np.array([(TB, O, O, self.Gyb.data_ptr(), self.GybT.data_ptr()),
+                         (KH, H, H, self.Hb.data_ptr(), self.HbT.data_ptr()),
+                         (TB, I, I, self.Xb.data_ptr(), self.XbT.data_ptr()),
+                         (TB, 3 * H, 3 * H, self.dGib.data_ptr(), self.dGiT.data_ptr()),
+                         (TB, 3 * H, 3 * H, self.dGhb.data_ptr(), self.dGhT.data_ptr())], dtype=np.int64)
+        nat.check(self.lib.dtb_mlp_pack_transposed(len(pack), pack.ctypes.data, s))
+        dw = np.array([(H, O, KH, TB, 0, self.HbT.data_ptr() + 2 * 32 * B, self.GybT.data_ptr(), 0,
+                        self.grad["W_o"].data_ptr(), 0),
+                       (I, 3 * H, TB, TB, 0, self.XbT.data_ptr(), self.dGiT.data_ptr(), 0,
+                        self.grad["W_ih"].data_ptr(), 0),
+                       (H, 3 * H, KH, TB, 0, self.HbT.data_ptr(), self.dGhT.data_ptr(), 0,
+                        self.grad["W_hh"].data_ptr(), 0)], dtype=np.int64)
+        nat.check(self.lib.dtb_mlp_weight_gradients(len(dw), dw.ctypes.data, TB, s))
         # the partial sums this batch wrote (the buffer is sized for the longest, largest batch)
         return self.lsum[: (TB * O + 255) // 256]
 

@@ -463,6 +463,53 @@ int dtb_gru_forward(int32_t B, int32_t H, const float* gi, const float* gh, cons
 int dtb_gru_backward(int32_t B, int32_t H, const float* gi, const float* gh, const float* h, const float* dh_a,
                      const float* dh_b, const float* dh_c, float* dgi, void* dgib, float* dgh, void* dghb, float* dh_z,
                      void* stream);
+/* Whole-sequence calls of the GRU surrogate: all T steps of the recurrence in
+ * one kernel, with the results of the calls above bit for bit.  fits: B and H
+ * multiples of 32, H <= 256 (else DTB_UNSUPPORTED).  Forward: gi [T][B][3H],
+ * w_hh bf16 [3H][H], h0 [h0_rows][H] or NULL (zeros); writes gh [T][B][3H],
+ * hs [T+1][B][H] and its bf16 copy hb.  Backward: dho [T][B][H] from the
+ * readout, w_hh_t bf16 [H][3H]; writes the gradients of gi and gh in bf16
+ * [T][B][3H], and dg [T][B][4H] in FP32: dr, dz and dn, the gradient of gi,
+ * then dn r, the last third of that of gh.  Weights 16-byte aligned. */
+int dtb_gru_sequence_fits(int32_t B, int32_t H);
+int dtb_gru_sequence_forward(int32_t T, int32_t B, int32_t H, const float* gi, const void* w_hh, const float* b_hh,
+                             const float* h0, int32_t h0_rows, float* gh, float* hs, void* hb, void* stream);
+int dtb_gru_sequence_backward(int32_t T, int32_t B, int32_t H, const float* gi, const float* gh, const float* hs,
+                              const float* dho, const void* w_hh_t, void* dgib, void* dghb, float* dg, void* stream);
+/* dtb_mlp_mse_grad of outputs [T][B][O] against Y [T][rows][n_out] * y_scale +
+ * y_shift under mask [T][rows][n_out] (NULL: ones); padding has no gradient. */
+int dtb_mlp_sequence_loss(int32_t T, int32_t B, int32_t O, int32_t rows, int32_t n_out, const float* out,
+                          const float* Y, const float* y_scale, const float* y_shift, const float* mask, float scale,
+                          float* grad, void* gradb, float* lsum, void* stream);
+/* bf16 [rows][cols] (row stride ld) into the fragment order of its transpose
+ * (dtb_adam_param); rows and cols multiples of 32, at most 16 matrices. */
+typedef struct {
+    int64_t rows, cols, ld;
+    const void* in;
+    void* out;
+} dtb_pack_item;
+int dtb_mlp_pack_transposed(int32_t n, const dtb_pack_item* items, void* stream);
+/* dst[j] (and dst2[j] unless NULL) = sum over rows of src [rows][ld], cols
+ * columns, added in row order (as dtb_mlp_bias_grad); at most 8 arrays. */
+typedef struct {
+    int64_t cols, ld;
+    const float* src;
+    float* dst;
+    float* dst2;
+} dtb_colsum_item;
+int dtb_mlp_column_sums(int32_t n, const dtb_colsum_item* items, int64_t rows, void* stream);
+/* dw [n_out][n_in] = g h^T over `rows` rows for at most 8 products, h [n_in][rows]
+ * and g [n_out][rows] in fragment order, as parts of arrays of ldh and ldg
+ * columns; db (NULL: none) [n_out] = the sums of dbp [parts][n_out]. */
+typedef struct {
+    int64_t n_in, n_out, ldh, ldg, parts;
+    const void* h;
+    const void* g;
+    const float* dbp;
+    float* dw;
+    float* db;
+} dtb_dw_item;
+int dtb_mlp_weight_gradients(int32_t n, const dtb_dw_item* items, int32_t rows, void* stream);
 /* round-to-nearest-even FP32 -> bf16 */
 int dtb_mlp_f32_to_bf16(int64_t n, const float* in, void* out, void* stream);
 
