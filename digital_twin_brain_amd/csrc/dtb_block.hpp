@@ -73,6 +73,7 @@ struct Block {
     float* rec_vsum = nullptr;    // [kmax][S]
     float* rec_isum = nullptr;    // [kmax][S]
     uint64_t* rec_events = nullptr; // [kmax]
+    uint64_t* ev_part = nullptr;    // partial event counters of a step (zero between steps)
     uint32_t* rec_nspk = nullptr;   // [kmax]
     uint8_t* rec_sspk = nullptr;    // [kmax][ns]
     float* rec_sv = nullptr;        // [kmax][ns]
