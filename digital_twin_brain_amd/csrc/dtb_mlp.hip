@@ -5,14 +5,15 @@
 // GEMM form "NT": C[M,N] = act(A[M,K] * B[N,K]^T + bias[N]); both operands are
 // K-contiguous row-major bf16, so a forward layer is (X, W^T) and the two
 // backward products use transposed copies made by dtb_mlp_transpose_bf16.
-// One workgroup (4 wavefronts) computes a 64x64 tile; each wavefront owns a
-// 32x32 sub-tile and issues v_mfma_f32_32x32x16_bf16 over K in steps of 16.
+// A workgroup of four wavefronts computes a tile of C with
+// v_mfma_f32_32x32x16_bf16 over K in steps of 16.
 //
 // MFMA operand layout (32x32x16 bf16): lane l holds 8 consecutive K values
 // k = 8*(l/32) .. +7 of row (l % 32) for A and of column (l % 32) for B; the
 // 16 accumulator registers hold C[8*(r/4) + 4*(l/32) + r%4][l % 32].
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "dtb_internal.hpp"
 
@@ -43,32 +44,108 @@ __device__ inline uint32_t f2bf_pk(float lo, float hi)
 __device__ inline float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // act: 0 identity, 1 ReLU
-// A workgroup of four wavefronts (2x2) computes a (64 TM) x (64 TN) tile of C;
-// each wavefront TM x TN sub-tiles of 32x32, one v_mfma_f32_32x32x16_bf16 per
-// sub-tile and 16-wide K step, so each fragment it loads feeds TN (or TM)
-// products.  The fragments of the next K step are loaded before the products
-// of the current one.  M and N are multiples of 32 only: a sub-tile past the
-// edge loads clamped rows (inside A and B) and is not stored.
-template <int TM, int TN>
-__global__ __launch_bounds__(256) void gemm_nt_kernel(int32_t M, int32_t N, int32_t K, const uint16_t* __restrict__ A,
-                                                      int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
-                                                      const float* __restrict__ bias, int32_t act,
-                                                      float* __restrict__ C, int64_t ldc,
-                                                      uint16_t* __restrict__ Cb, int64_t ldcb)
+
+// Products of one chain over K (gemm_one_chain): LDS-staged tiles filled by
+// direct global-to-LDS loads.  A workgroup of four wavefronts (2 x 2), one on
+// each SIMD of its CU, computes a (64 TM) x (64 TN) tile of C, each wavefront
+// TM x TN sub-tiles of 32x32.  The bound is the matrix pipe, and next to it
+// the LDS ports: with 128x128 per wavefront (TM = TN = 4) a 16-wide K step
+// reads 8 KB of fragments for 16 MFMAs, half the port rate (64x128 per
+// wavefront, as eight wavefronts had it, saturated the ports, and the copies
+// through registers came on top).
+// K advances 64 at a time.  A and B slices go through a ring of five LDS
+// slots (two and a half slices: all 160 KB with TM = TN = 4), and the loop is
+// pipelined so that neither a fragment read, nor the barrier, nor the latency
+// of a slice leaves the matrix pipe idle:
+//   K step s of a slice multiplies fragments read during step s - 1;
+//   at the last step of slice t the wavefronts meet (slice t + 1 has landed,
+//   nobody reads slice t any more) and read slice t + 1's first fragments;
+//   from there to the next meeting they request, spread over the MFMAs, B of
+//   slice t + 2 into A(t)'s slot, then A of slice t + 3 into B(t)'s.  (All at
+//   once the requests queue up: 64 of 16 cycles each at the load unit of the
+//   CU.)  B has most of a slice's time to arrive, A most of two.
+// A slot row is 64 bf16 = 8 chunks of 16 bytes; the load unit writes 64
+// lanes' chunks back to back, so the lanes permute what they fetch: chunk c
+// of row r sits at position c ^ (r / 2 % 8), and the 16 rows that a quarter of
+// a fragment read touches fall on distinct banks without padding.
+// M and N are multiples of 32, K of 16: rows past the edge are clamped (and
+// not stored), a last slice shorter than 64 fetches clamped chunks that no
+// step multiplies.  Workgroups are dealt to tiles XCD by XCD (workgroup w
+// runs on XCD w mod 8): each XCD takes a contiguous run of tiles, ordered in
+// bands of GM tile rows, column by column, so that the tiles it has in flight
+// form a near-square block and share their slices in its L2.
+// 8192^3: 1136 -> 859 us (1.28 PFLOP/s; matrix pipe busy 74% of the cycles, no
+// LDS bank conflicts); 960 x 960 x 6144: 112 -> 39 us; 992 x 4160 x 3008 (no
+// multiples of 128): 181 -> 44 us.
+__device__ __forceinline__ void lds_dma16(const uint16_t* src, uint32_t lds_byte)
 {
-    const int wid = threadIdx.x >> 6;
+    // the wavefront's 64 chunks of 16 bytes, to consecutive LDS addresses from lds_byte (M0);
+    // counted by vmcnt, for which the caller waits
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_byte), "v"(src)
+                 : "memory", "m0");
+}
+
+// N of this wavefront's loads may still be under way, its LDS reads are done; then all wavefronts meet
+template <int N>
+__device__ __forceinline__ void lds_dma_meet()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// RANGES: each wavefront's sums are those of four consecutive ranges of K added
+// in order, as gemm_nt_splitk_kernel adds them, instead of one chain.
+template <int T, int GM, bool RANGES>
+__global__ __launch_bounds__(256, T == 4 ? 1 : T == 2 ? 2 : 4) void gemm_nt_tile_kernel(
+    int32_t M, int32_t N, int32_t K, const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B,
+    int64_t ldb, const float* __restrict__ bias, int32_t act, float* __restrict__ C, int64_t ldc,
+    uint16_t* __restrict__ Cb, int64_t ldcb)
+{
+    constexpr int TM = T, TN = T;
+    constexpr int kSlot = 64 * T * 64; // elements: 64 T rows of A or B
+    extern __shared__ __align__(128) uint16_t lds[]; // [5][kSlot]
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int m0 = blockIdx.y * (64 * TM) + (wid >> 1) * (32 * TM);
-    const int n0 = blockIdx.x * (64 * TN) + (wid & 1) * (32 * TN);
-    if (m0 >= M || n0 >= N) return; // wavefront-uniform
-    const int r = lane & 31;
-    const int kh = (lane >> 5) * 8;
-    const uint16_t* pa[TM];
-    const uint16_t* pb[TN];
+    const int wm = wid >> 1, wn = wid & 1;
+    // this workgroup's tile
+    const int tm = (M + 64 * TM - 1) / (64 * TM), tn = (N + 64 * TN - 1) / (64 * TN);
+    const int tiles = tm * tn;
+    const int per = (tiles + 7) / 8;
+    const int tile = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per || tile >= tiles) return; // workgroup-uniform
+    const int band = tile / (GM * tn);
+    const int rows = min(GM, tm - band * GM);
+    const int in = tile - band * GM * tn;
+    const int m_blk = (band * GM + in % rows) * (64 * TM), n_blk = in / rows * (64 * TN);
+    // what this wavefront fetches of a slice: 2 TM groups of 8 rows of A, 2 TN of B
+    constexpr int kFetch = 2 * (TM + TN);
+    // columns of this lane's chunk in the slice, in even and odd groups of 8 rows
+    const int ch[2] = {((lane & 7) ^ (lane >> 4)) * 8, ((lane & 7) ^ (4 + (lane >> 4))) * 8};
+    const uint16_t* src[kFetch];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) pa[i] = A + (int64_t)(min(m0 + 32 * i, M - 32) + r) * lda + kh;
+    for (int u = 0; u < kFetch; ++u) {
+        if (u < 2 * TM) src[u] = A + (int64_t)min(m_blk + (wid * 2 * TM + u) * 8 + (lane >> 3), M - 1) * lda;
+        else src[u] = B + (int64_t)min(n_blk + (wid * 2 * TN + u - 2 * TM) * 8 + (lane >> 3), N - 1) * ldb;
+    }
+    auto fetch = [&](int u, int kt, int slot) { // group u of K slice kt to a slot of the ring
+        const int row0 = (wid * 2 * T + u % (2 * T)) * 8;
+        lds_dma16(src[u] + min(kt * 64 + ch[u & 1], K - 8), lds0 + (uint32_t)(slot * kSlot + row0 * 64) * 2u);
+    };
+    const int r = lane & 31, kh = lane >> 5;
+    int oa[4], ob[4]; // element offset of this lane's fragments in a slot, by K step
 #pragma unroll
-    for (int j = 0; j < TN; ++j) pb[j] = B + (int64_t)(min(n0 + 32 * j, N - 32) + r) * ldb + kh;
+    for (int s = 0; s < 4; ++s) {
+        const int slot = ((2 * s + kh) ^ ((r >> 1) & 7)) * 8;
+        oa[s] = (wm * 32 * TM + r) * 64 + slot;
+        ob[s] = (wn * 32 * TN + r) * 64 + slot;
+    }
+    bf16x8 fr[2][TM + TN];
+    int sa = 0, sb = 1; // the slots of the current slice: 2 t mod 5 and 2 t + 1 mod 5
+    auto next = [](int slot) { return slot < 3 ? slot + 2 : slot - 3; };
+    auto read = [&](int f, int x, int a, int b, int s) { // fragment x of K step s of the slice in slots a, b
+        fr[f][x] = *reinterpret_cast<const bf16x8*>(x < TM ? lds + a * kSlot + oa[s] + x * 32 * 64
+                                                           : lds + b * kSlot + ob[s] + (x - TM) * 32 * 64);
+    };
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -76,30 +153,113 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(int32_t M, int32_t N, int3
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
-    bf16x8 a[TM], b[TN];
+    const int nk = (K + 63) / 64;
+    constexpr int kHalf = kFetch / 2;        // this wavefront's loads of one operand's slice
+    constexpr int kFirst = (3 * kHalf + 3) / 4; // of them, those of B requested right after a meeting
 #pragma unroll
-    for (int i = 0; i < TM; ++i) a[i] = *reinterpret_cast<const bf16x8*>(pa[i]);
+    for (int u = 0; u < kFetch; ++u) fetch(u, 0, u / kHalf);
+    if (nk > 1) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) b[j] = *reinterpret_cast<const bf16x8*>(pb[j]);
-    for (int k0 = 16; k0 < K; k0 += 16) {
-        bf16x8 an[TM], bn[TN];
+        for (int u = 0; u < kHalf + kFirst; ++u) fetch(u, 1, 2 + u / kHalf);
+        lds_dma_meet<kHalf + kFirst>(); // slice 0 has landed
+    } else {
+        lds_dma_meet<0>();
+    }
 #pragma unroll
-        for (int i = 0; i < TM; ++i) an[i] = *reinterpret_cast<const bf16x8*>(pa[i] + k0);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) bn[j] = *reinterpret_cast<const bf16x8*>(pb[j] + k0);
+    for (int x = 0; x < TM + TN; ++x) read(0, x, 0, 1, 0);
+    // one K step's MFMAs from fr[f]; after the i-th, side(i) issues what overlaps it
+    auto multiply = [&](int f, auto&& side) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f][i], fr[f][TM + j], acc[i][j], 0, 0, 0);
+                side(i * TN + j);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    constexpr int kProd = TM * TN;
+    // RANGES: the sum of the finished ranges, and the K steps left in the current one
+    f32x16 tot[RANGES ? TM : 1][RANGES ? TN : 1];
+    const int range_steps = RANGES ? (K / 16 + 3) / 4 : 0;
+    int range = 0, to_fold = range_steps;
+    auto step_done = [&]() {
+        if constexpr (RANGES) {
+            if (--to_fold == 0) {
+                to_fold = range_steps;
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = an[i];
+                for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b[j] = bn[j];
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int x = 0; x < 16; ++x) {
+                            tot[i][j][x] = range == 0 ? acc[i][j][x] : tot[i][j][x] + acc[i][j][x];
+                            acc[i][j][x] = 0.0f;
+                        }
+                ++range;
+            }
+        }
+    };
+    // a slice that one other (more: several others) follows
+    auto slice = [&](int kt, auto more_) {
+        constexpr bool more = decltype(more_)::value;
+        constexpr int kRest = kFetch - kFirst; // requests in steps 0 to 2
+        const int na = next(sa), nb = next(sb);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            multiply(s & 1, [&](int i) {
+                // the next step's fragments, two after each MFMA while they last
+#pragma unroll
+                for (int x = 0; x < TM + TN; ++x)
+                    if (x / 2 == i || (i == kProd - 1 && x / 2 > i)) read((s + 1) & 1, x, sa, sb, s + 1);
+#pragma unroll
+                for (int y = 0; y < kRest; ++y)
+                    if (y * 3 * kProd / kRest == s * kProd + i) {
+                        if (y < kHalf - kFirst) fetch(kHalf + kFirst + y, kt + 1, nb);
+                        else if (more) fetch(y - (kHalf - kFirst), kt + 2, next(na));
+                    }
+            });
+            step_done();
+        }
+        // slice kt + 1 has landed (A of slice kt + 2 may be under way), and
+        // this wavefront's last fragments of slice kt are in registers
+        lds_dma_meet<more ? kHalf : 0>();
+        multiply(1, [&](int i) {
+#pragma unroll
+            for (int x = 0; x < TM + TN; ++x)
+                if (x / 2 == i || (i == kProd - 1 && x / 2 > i)) read(0, x, na, nb, 0);
+#pragma unroll
+            for (int u = 0; u < kFirst; ++u)
+                if (more && u * kProd / kFirst == i) fetch(kHalf + u, kt + 2, sa);
+        });
+        step_done();
+        sa = na;
+        sb = nb;
+    };
+    int kt = 0;
+    for (; kt + 2 < nk; ++kt) slice(kt, std::true_type{});
+    if (kt + 1 < nk) slice(kt++, std::false_type{});
+    // the last slice, of one to four steps
+    for (int s = 0; 64 * kt + 16 * s < K; ++s) {
+        const int slot = ((2 * s + kh) ^ ((r >> 1) & 7)) * 8 + r * 64;
+#pragma unroll
+        for (int x = 0; x < TM + TN; ++x)
+            fr[0][x] = *reinterpret_cast<const bf16x8*>(x < TM ? lds + sa * kSlot + slot + (wm * TM + x) * 32 * 64
+                                                               : lds + sb * kSlot + slot + (wn * TN + x - TM) * 32 * 64);
+        multiply(0, [](int) {});
+        step_done();
     }
+    if constexpr (RANGES) {
+        // a range that K's steps do not fill, or the empty ones after it (adding zeros as they would)
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int x = 0; x < 16; ++x)
+                    acc[i][j][x] = range == 0 ? acc[i][j][x] : range < 4 ? tot[i][j][x] + acc[i][j][x] : tot[i][j][x];
+    }
+    const int m0 = m_blk + wm * 32 * TM, n0 = n_blk + wn * 32 * TN;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
         if (n0 + 32 * j >= N) continue;
@@ -108,142 +268,19 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(int32_t M, int32_t N, int3
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             if (m0 + 32 * i >= M) continue;
+            // one running pointer an output (addresses kept for all stores would spill)
+            const int64_t row = m0 + 32 * i + 4 * kh;
+            float* c = C + row * ldc + col;
+            uint16_t* cb = Cb + row * ldcb + col;
 #pragma unroll
             for (int x = 0; x < 16; ++x) {
-                const int row = m0 + 32 * i + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
                 float v = acc[i][j][x] + bv;
                 if (act == 1) v = v > 0.0f ? v : 0.0f;
-                if (C) C[(int64_t)row * ldc + col] = v;
-                if (Cb) Cb[(int64_t)row * ldcb + col] = f2bf(v);
-            }
-        }
-    }
-}
-
-// Large products: LDS-staged tiles.  A workgroup of eight wavefronts (4 x 2)
-// computes a 256x256 tile of C; each wavefront a 64x128 sub-tile (2 x 4
-// MFMA tiles of 32x32, eight v_mfma_f32_32x32x16_bf16 per 16-wide K step
-// from six LDS fragments).  K advances 64 at a time: the next 256x64 slices
-// of A and B are loaded from global memory into registers (16-byte loads, 8
-// lanes per 128-byte row) while the current ones are multiplied out of LDS,
-// then stored to the other half of a double buffer; one barrier per slice.
-// LDS rows are 64 + 8 bf16 long, so the 32 rows a fragment read touches
-// fall on distinct banks.  Workgroups are dealt to tiles XCD by XCD
-// (workgroup w runs on XCD w mod 8): each XCD takes a contiguous run of
-// tiles, whose A and B slices then repeat in its own L2.
-// Requires M, N multiples of 256 and K of 64.
-constexpr int kLdsBM = 256, kLdsBN = 256, kLdsKT = 64, kLdsRow = kLdsKT + 8;
-
-__global__ __launch_bounds__(512, 1) void gemm_nt_lds_kernel(int32_t M, int32_t N, int32_t K,
-                                                             const uint16_t* __restrict__ A, int64_t lda,
-                                                             const uint16_t* __restrict__ B, int64_t ldb,
-                                                             const float* __restrict__ bias, int32_t act,
-                                                             float* __restrict__ C, int64_t ldc,
-                                                             uint16_t* __restrict__ Cb, int64_t ldcb)
-{
-    extern __shared__ __align__(16) uint16_t lds[]; // [2][A 256 x 72 | B 256 x 72]
-    constexpr int kStage = (kLdsBM + kLdsBN) * kLdsRow;
-    const int t = threadIdx.x;
-    const int wid = t >> 6;
-    const int lane = t & 63;
-    const int wm = wid >> 1, wn = wid & 1;
-    // tile of this workgroup: XCD-contiguous runs of tiles, row-major within
-    const int tn = N / kLdsBN;
-    const int tiles = (M / kLdsBM) * tn;
-    const int nx = 8;
-    const int w = blockIdx.x;
-    const int per = (tiles + nx - 1) / nx;
-    const int xcd = w % nx, slot = w / nx;
-    const int tile = xcd * per + slot;
-    if (tile >= tiles) return; // workgroup-uniform
-    const int m_blk = (tile / tn) * kLdsBM, n_blk = (tile % tn) * kLdsBN;
-    // global -> register copies: chunk c = t + 512 u (u < 4) of each operand,
-    // row c / 8, 8 bf16 at column 8 (c % 8) of the 64-wide slice
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const uint16_t* ga[4];
-    const uint16_t* gb[4];
-    int so[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int c = t + 512 * u;
-        const int row = c >> 3, kc = (c & 7) * 8;
-        ga[u] = A + (int64_t)(m_blk + row) * lda + kc;
-        gb[u] = B + (int64_t)(n_blk + row) * ldb + kc;
-        so[u] = row * kLdsRow + kc;
-    }
-    u32x4 ra[4], rb[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        ra[u] = *reinterpret_cast<const u32x4*>(ga[u]);
-        rb[u] = *reinterpret_cast<const u32x4*>(gb[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        *reinterpret_cast<u32x4*>(lds + so[u]) = ra[u];
-        *reinterpret_cast<u32x4*>(lds + kLdsBM * kLdsRow + so[u]) = rb[u];
-    }
-    __syncthreads();
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int x = 0; x < 16; ++x) acc[i][j][x] = 0.0f;
-    const int r = lane & 31;
-    const int kh = (lane >> 5) * 8;
-    const int nk = K / kLdsKT;
-    for (int kt = 0; kt < nk; ++kt) {
-        const bool more = kt + 1 < nk;
-        if (more) {
-            const int64_t k1 = (int64_t)(kt + 1) * kLdsKT;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                ra[u] = *reinterpret_cast<const u32x4*>(ga[u] + k1);
-                rb[u] = *reinterpret_cast<const u32x4*>(gb[u] + k1);
-            }
-        }
-        const uint16_t* sa = lds + (kt & 1) * kStage;
-        const uint16_t* sb = sa + kLdsBM * kLdsRow;
-#pragma unroll
-        for (int ks = 0; ks < kLdsKT / 16; ++ks) {
-            bf16x8 a[2], b[4];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                a[i] = *reinterpret_cast<const bf16x8*>(sa + (wm * 64 + 32 * i + r) * kLdsRow + ks * 16 + kh);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[j] = *reinterpret_cast<const bf16x8*>(sb + (wn * 128 + 32 * j + r) * kLdsRow + ks * 16 + kh);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            uint16_t* da = lds + ((kt + 1) & 1) * kStage;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                *reinterpret_cast<u32x4*>(da + so[u]) = ra[u];
-                *reinterpret_cast<u32x4*>(da + kLdsBM * kLdsRow + so[u]) = rb[u];
-            }
-        }
-        __syncthreads();
-    }
-    const int m0 = m_blk + wm * 64, n0 = n_blk + wn * 128;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = n0 + 32 * j + r;
-        const float bv = bias ? bias[col] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-#pragma unroll
-            for (int x = 0; x < 16; ++x) {
-                const int row = m0 + 32 * i + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3);
-                float v = acc[i][j][x] + bv;
-                if (act == 1) v = v > 0.0f ? v : 0.0f;
-                if (C) C[(int64_t)row * ldc + col] = v;
-                if (Cb) Cb[(int64_t)row * ldcb + col] = f2bf(v);
+                if (C) *c = v;
+                if (Cb) *cb = f2bf(v);
+                c += (x & 3) == 3 ? 5 * ldc : ldc; // rows 0..3, 8..11, 16..19, 24..27
+                cb += (x & 3) == 3 ? 5 * ldcb : ldcb;
+                asm volatile("" : "+v"(c), "+v"(cb));
             }
         }
     }
@@ -1569,6 +1606,43 @@ using GruFwdWeights = GruWeights<(6 * G + kGruFwdWaves - 1) / kGruFwdWaves, G, k
 template <int G>
 using GruBwdWeights = GruWeights<(2 * G + kGruBwdWaves - 1) / kGruBwdWaves, 3 * G, kGruBwdWaves, kGruBwdHeld>;
 
+// Which kernel takes a product: the tile of gemm_nt_tile_kernel in units of 64
+// (-1: 64x64 tiles, K in four ranges), or 0 for the split-K kernel.
+// Rules from both sides' times, us (K = 2048 unless given):
+//   128 or more 64x64 tiles: split-K's 32x32 tiles read each operand row twice
+//     as often, in 32-byte pieces (768^2 K = 768: 13.5 split, 7.1 tiles; 96 x
+//     6144 K = 3008: 38.3, 21.1); up to 64 its workgroups are the only ones
+//     that fill the CUs (512^2 K = 512: 4.7, 6.0);
+//   128x128 tiles once every CU gets one (2048^2: 64x64 29.4, 128x128 23.8;
+//     1536^2 K = 1536, 144 tiles: 15.5, 17.0);
+//   256x256 tiles, one a CU and 1.75 times the time of a round of 128x128
+//     tiles, two a CU, where that many fewer rounds do (8192^3: 808 against
+//     1033; 5024 x 1632 K = 2000: 51 against 59; 6144^3, 2.25 rounds: 426
+//     against 416).
+static int gemm_tile(int32_t M, int32_t N)
+{
+    auto tiles = [&](int32_t t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
+    if (!gemm_one_chain(M, N)) return tiles(64) >= 128 ? -1 : 0;
+    if (tiles(128) < 256) return 1;
+    const int64_t r4 = (tiles(256) + 255) / 256, r2 = (tiles(128) + 511) / 512;
+    return 7 * r4 <= 4 * r2 ? 4 : 2;
+}
+
+template <int T, bool RANGES>
+static int launch_gemm_tile(int32_t M, int32_t N, int32_t K, const void* A, int64_t lda, const void* B, int64_t ldb,
+                            const float* bias, int32_t act, float* C, int64_t ldc, void* Cb, int64_t ldcb, void* stream)
+{
+    constexpr int GM = T == 4 ? 4 : 8; // about the square root of the tiles an XCD's 32 CUs hold
+    constexpr int lds = 5 * 64 * T * 64 * (int)sizeof(uint16_t);
+    const int64_t tiles = (int64_t)((M + 64 * T - 1) / (64 * T)) * ((N + 64 * T - 1) / (64 * T));
+    DTB_TRY_HIP(hipFuncSetAttribute((const void*)gemm_nt_tile_kernel<T, GM, RANGES>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL((gemm_nt_tile_kernel<T, GM, RANGES>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds,
+                       (hipStream_t)stream, M, N, K, (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, act, C, ldc,
+                       (uint16_t*)Cb, ldcb);
+    return DTB_OK;
+}
+
 static inline dim3 g1(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
 } // namespace dtb
@@ -1587,31 +1661,16 @@ int dtb_mlp_gemm_bf16_nt(int32_t M, int32_t N, int32_t K, const void* A, int64_t
     DTB_REQUIRE(act == 0 || act == 1, "act must be 0 (identity) or 1 (ReLU)");
     DTB_REQUIRE((reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0,
                 "A and B must be 16-byte aligned");
-    // 128x128 workgroup tiles while they still give every compute unit a
-    // workgroup, else 64x64, else 32x32 tiles with K split over the wavefronts
-    // (the surrogate's own products are that small)
-    const int64_t big = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
-    const int64_t lds_tiles = (int64_t)(N / kLdsBN) * (M / kLdsBM);
-    if (M % kLdsBM == 0 && N % kLdsBN == 0 && K % kLdsKT == 0 && lds_tiles >= 64) {
-        // LDS-staged 256x256 tiles, one workgroup per tile (the tile map deals them XCD by XCD)
-        const size_t lds = sizeof(uint16_t) * 2 * (size_t)(kLdsBM + kLdsBN) * kLdsRow;
-        DTB_TRY_HIP(hipFuncSetAttribute((const void*)gemm_nt_lds_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)lds));
-        const unsigned nwg = (unsigned)((lds_tiles + 7) / 8 * 8);
-        hipLaunchKernelGGL(gemm_nt_lds_kernel, dim3(nwg), dim3(512), lds, (hipStream_t)stream, M, N, K,
-                           (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, act, C, ldc, (uint16_t*)Cb, ldcb);
-    } else if (big >= 256) {
-        dim3 grid((unsigned)((N + 127) / 128), (unsigned)((M + 127) / 128));
-        hipLaunchKernelGGL((gemm_nt_kernel<2, 2>), grid, dim3(256), 0, (hipStream_t)stream, M, N, K,
-                           (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, act, C, ldc, (uint16_t*)Cb, ldcb);
-    } else if ((int64_t)((N + 63) / 64) * ((M + 63) / 64) >= 256) {
-        dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-        hipLaunchKernelGGL((gemm_nt_kernel<1, 1>), grid, dim3(256), 0, (hipStream_t)stream, M, N, K,
-                           (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, act, C, ldc, (uint16_t*)Cb, ldcb);
-    } else {
+    switch (gemm_tile(M, N)) {
+    case 4: DTB_TRY((launch_gemm_tile<4, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
+    case 2: DTB_TRY((launch_gemm_tile<2, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
+    case 1: DTB_TRY((launch_gemm_tile<1, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
+    case -1: DTB_TRY((launch_gemm_tile<1, true>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
+    default: {
         dim3 grid((unsigned)(N / 32), (unsigned)(M / 32));
         hipLaunchKernelGGL(gemm_nt_splitk_kernel, grid, dim3(256), 0, (hipStream_t)stream, M, N, K,
                            (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, act, C, ldc, (uint16_t*)Cb, ldcb);
+    }
     }
     DTB_TRY_HIP(hipGetLastError());
     return DTB_OK;

@@ -497,17 +497,22 @@ class GRUSurrogate:
 
 def gemm_kernel_name(M, N, K):
     """The kernel dtb_mlp_gemm_bf16_nt dispatches an M x N x K product to:
-    LDS-staged 256x256 tiles when M and N are multiples of 256, K of 64 and
-    there are at least 64 such tiles; else 128x128 tiles while they give at
-    least 256 workgroups, else 64x64 tiles, else 32x32 tiles with K split
-    over the four wavefronts."""
-    if M % 256 == 0 and N % 256 == 0 and K % 64 == 0 and (M // 256) * (N // 256) >= 64:
-        return "gemm_nt_lds_kernel (256x256 LDS-staged tiles, bf16 MFMA, FP32 accumulate)"
-    if ((N + 127) // 128) * ((M + 127) // 128) >= 256:
-        return "gemm_nt_kernel<2,2> (128x128 tiles, bf16 MFMA, FP32 accumulate)"
-    if ((N + 63) // 64) * ((M + 63) // 64) >= 256:
-        return "gemm_nt_kernel<1,1> (64x64 tiles, bf16 MFMA, FP32 accumulate)"
-    return "gemm_nt_splitk_kernel (32x32 tiles, K split over 4 wavefronts, bf16 MFMA, FP32 accumulate)"
+    LDS-staged square tiles of 256, 128 or 64 (the fewest rounds of
+    workgroups, weighed by a round's time; 64 with K in four ranges where
+    there are fewer than 256 such tiles), or below 128 tiles of 64 the
+    32x32 tiles with K split over the four wavefronts."""
+    def tiles(t):
+        return -(-M // t) * -(-N // t)
+
+    if tiles(64) < 128:
+        return "gemm_nt_splitk_kernel (32x32 tiles, K split over 4 wavefronts, bf16 MFMA, FP32 accumulate)"
+    if tiles(64) < 256:
+        return "gemm_nt_tile_kernel<1> (64x64 LDS-staged tiles, K in 4 ranges, bf16 MFMA, FP32 accumulate)"
+    if tiles(128) < 256:
+        t = 1
+    else:
+        t = 4 if 7 * -(-tiles(256) // 256) <= 4 * -(-tiles(128) // 512) else 2
+    return f"gemm_nt_tile_kernel<{t}> ({64 * t}x{64 * t} LDS-staged tiles, bf16 MFMA, FP32 accumulate)"
 
 
 def gemm_throughput(M, N, K, reps=50, warmup=5, device=0):

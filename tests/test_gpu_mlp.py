@@ -65,6 +65,26 @@ def test_gemm_strided_operands_and_random_values(M, N, K):
     torch.testing.assert_close(C.cpu(), want, rtol=1e-5, atol=1e-5 * K ** 0.5)
 
 
+# edges of the LDS-staged tiles (256, 128, 64, and 64 with K in four ranges) with
+# ragged last rows and columns of tiles; K from less than one 64-wide slice over
+# one, two and three slices to a slice ring used more than once, whole and short
+# last slices.  Integers: every partial sum is exact.  The columns and rows
+# around C stay untouched.
+@pytest.mark.parametrize("K", [16, 48, 64, 112, 128, 144, 192, 208, 256, 400, 704])
+@pytest.mark.parametrize("M,N", [(3808, 3104), (2080, 2144), (1056, 992), (736, 800)])
+def test_gemm_tile_edges(M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randint(-4, 5, (M, K + 8), generator=g, device="cuda").to(torch.bfloat16)
+    B = torch.randint(-4, 5, (N, K + 16), generator=g, device="cuda").to(torch.bfloat16)
+    bias = torch.randint(-8, 9, (N,), generator=g, device="cuda").float()
+    C = torch.full((M + 1, N + 4), 0.5, device="cuda")
+    nat.check(nat.lib().dtb_mlp_gemm_bf16_nt(M, N, K, A.data_ptr(), K + 8, B.data_ptr(), K + 16, bias.data_ptr(), 0,
+                                             C.data_ptr(), N + 4, None, 0, ctypes_stream()))
+    want = torch.full_like(C, 0.5)
+    want[:M, :N] = A[:, :K].float() @ B[:, :K].float().T + bias
+    assert torch.equal(C, want)
+
+
 def test_gemm_rejects_bad_shapes():
     L = nat.lib()
     A = torch.zeros((32, 16), dtype=torch.bfloat16, device="cuda")
