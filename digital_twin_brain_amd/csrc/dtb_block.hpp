@@ -70,7 +70,8 @@ struct Block {
 
     // per-step records of the current batch
     uint32_t* rec_freq = nullptr; // [kmax][S]
-    float* rec_vsum = nullptr;    // [kmax][S]
+    double* rec_vsum = nullptr;   // [kmax][S]
+    float* rec_vmean = nullptr;   // [kmax][S]
     float* rec_isum = nullptr;    // [kmax][S]
     uint64_t* rec_events = nullptr; // [kmax]
     uint64_t* ev_part = nullptr;    // partial event counters of a step (zero between steps)
@@ -154,6 +155,7 @@ struct Block {
     // order), rebuilt when the weights change
     int32_t* pbptr = nullptr;   // [pG][n*D+1] start of workgroup g's synapses of each segment
     uint32_t* pcol = nullptr;   // [nnz] records: local index | kind << 31, round(scaled weight) (x2 pair, + pad)
+    void* pin = nullptr;        // pinned host buffer for small records (kPinBytes)
     uint32_t* pbar = nullptr;   // [0] barrier counter, [64] abort flag
     int32_t pG = 0, pm = 0;     // workgroups, 256-neuron blocks of LDS slice per workgroup
     int32_t pper = 0;           // neurons per workgroup (consecutive ranges)
