@@ -93,6 +93,19 @@ def csr_from_w(w_uij):
                 w1=None if np.array_equal(w0, w1) else w1)
 
 
+# Blocks of these sizes run their steps in the persistent launch.  Above, its 32
+# workgroups no longer keep a neuron per thread in registers; below, a step is
+# all launch cost either way.  us, persistent against direct delivery: 20 steps
+# in one call 229 and 238 (1,000 neurons), 205 and 234 (2,000), 195 and 343
+# (10,000), 314 and 497 (32,768); a one-step call 34.6 and 31.4, 33.7 and 31.7,
+# 33.3 and 36.9, 41.2 and 37.2.
+PERSIST_N = (2000, 32 * 1024)
+# Steps after a weight change that run on the per-step kernels: the persistent
+# launch keeps a copy of the synapses grouped on the host, which a program that
+# changes weights between steps should not pay for each time.
+PERSIST_HOLD = 1000
+
+
 class block:
     """GPU LIF block with the interface of models/block.py:5-177."""
 
@@ -112,6 +125,7 @@ class block:
         self._nb = NativeBlock.from_csr(props, csr["rowptr"], csr["post"], csr["kind"], csr["w0"], csr["w1"],
                                         dt=float(delta_t), noise_seed=self._seed, device=device)
         self.N = self._nb.n
+        self._choose_launch()
         if src is None:
             self.src_neuron = None
             self.iter = None
@@ -129,6 +143,30 @@ class block:
         self._set_property_attrs(node_property)
         self._freq = np.zeros(self._nb.S, np.uint32)
         self._vmean = np.zeros(self._nb.S, np.float32)
+
+    # The persistent launch (deliver mode 2) takes blocks without sources whose
+    # sums fit its fixed point; steps with injected uniforms, and those soon
+    # after a weight change, run on the kernels the block was created with.
+    def _choose_launch(self, hold=0):
+        self._base_mode = self._mode = self._nb.get_launch()["deliver_mode"]
+        self._persist = self.src is None and PERSIST_N[0] <= self.N <= PERSIST_N[1]
+        self._hold = hold
+
+    def _set_mode(self, steps, persist=True):
+        mode = self._base_mode
+        if persist and self._persist:
+            if self._hold > 0:
+                self._hold -= steps
+            else:
+                mode = 2
+        if mode != self._mode:
+            try:
+                self._nb.set_launch(deliver_mode=mode)
+                self._mode = mode
+            except nat.DTBError as e:
+                if e.code != nat.DTB_INVALID_PARAMETER:
+                    raise
+                self._persist = False  # no fixed point for these weights
 
     def _apply_sources(self, nb):
         k, t = np.nonzero(self._sched)
@@ -174,6 +212,9 @@ class block:
         w = np.broadcast_to(w, ch.shape).copy()
         if ((ch < 0) | (ch > 3)).any() or ((post < 0) | (post >= self.N) | (pre < 0) | (pre >= self.N)).any():
             raise IndexError("conn_idx out of range")
+        if self._mode != self._base_mode:
+            self._set_mode(0, persist=False)
+        self._hold = PERSIST_HOLD
         try:
             self._nb.set_weights(pre, post, ch, w)
         except nat.DTBError as e:
@@ -227,6 +268,7 @@ class block:
         new.load_state(snap)
         nb.close()
         self._nb = new
+        self._choose_launch(hold=PERSIST_HOLD)
 
     def _t(self, a):
         return torch.from_numpy(a).to(self._out_device)
@@ -243,6 +285,7 @@ class block:
             uniforms = np.ascontiguousarray(np.asarray(uniforms, dtype=np.float32).reshape(-1))
         if self.src_neuron is not None and self.iter >= self._sched.shape[1]:
             raise IndexError(f"src has {self._sched.shape[1]} columns: no forced spikes for step {self.iter + 1}")
+        self._set_mode(1, persist=uniforms is None)
         self._nb.run(1, noise_mode=mode, noise_rate=float(noise_rate), uniforms=uniforms, isolated=isolated,
                      graph=False, freqs=self._freq, vmeans=self._vmean)
         if self.src_neuron is not None:
@@ -265,6 +308,7 @@ class block:
         freq = np.zeros((steps, S), np.uint32)
         vmean = np.zeros((steps, S), np.float32)
         if steps:
+            self._set_mode(steps)
             self._nb.run(steps, noise_mode=nat.NOISE_SCALAR, noise_rate=float(noise_rate), isolated=isolated,
                          graph=True, freqs=freq, vmeans=vmean)
         if self.src_neuron is not None:

@@ -404,3 +404,47 @@ def test_dropin_run_steps_equals_repeated_run():
     assert np.array_equal(a.V_i.numpy(), b.V_i.numpy())
     assert np.array_equal(a.J_ui.numpy(), b.J_ui.numpy())
     assert float(a.t) == float(b.t)
+
+
+# the persistent launch that drop-in blocks of 2,000 to 32,768 neurons take, against the
+# per-step kernels (dyadic weights: every delivery order gives the same sums), with
+# neurons of one population per wavefront, several, and a partial last one
+@pytest.mark.parametrize("n,npop", [(1999, 1), (2000, 1), (2085, 7), (4100, 300)])
+def test_dropin_persistent_launch_equals_per_step_kernels(n, npop):
+    from digital_twin_brain_amd import block as block_class
+
+    rng = np.random.default_rng(n)
+    csr = orc.gen_fixed_indegree(n, n * 4 // 5, 40, 1, 0.0, 1.0, True, seed=n)
+    for k in ("w0", "w1"):
+        csr[k] = (np.floor(csr[k] * 256) / 256).astype(np.float32)
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    _, first = np.unique(pre * n + csr["post"], return_index=True)
+    keep = np.zeros(pre.shape[0], bool)
+    keep[first] = True
+    csr = _keep_synapses(n, csr, keep)
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    p = _lif_props(n, rng, g_scale=1.5, sub=np.sort(rng.integers(0, npop, n)) if npop != 7 else rng.integers(0, 7, n))
+    idx = torch.from_numpy(np.stack([csr["kind"].astype(np.int64) * 2, csr["post"], pre]))
+    idx = torch.cat([idx, idx + torch.tensor([[1], [0], [0]])], dim=1)
+    W = torch.sparse_coo_tensor(idx, torch.from_numpy(np.concatenate([csr["w0"], csr["w1"]])), (4, n, n))
+    a = block_class(torch.from_numpy(p), W, delta_t=0.1, seed=5)
+    b = block_class(torch.from_numpy(p), W, delta_t=0.1, seed=5)
+    b._persist = False
+    u = rng.random(n).astype(np.float32)
+    ch, post, src = (x[:50].numpy() for x in idx)
+
+    def both(f):
+        for x, y in zip(f(a), f(b)):
+            np.testing.assert_allclose(x.numpy(), y.numpy(), rtol=2.0 ** -23, atol=0)
+
+    for k in range(2):
+        both(lambda x: x.run_steps(40, noise_rate=2.0 ** -6))
+        both(lambda x: x.run(noise_rate=2.0 ** -6))
+        both(lambda x: x.run(noise_rate=2.0 ** -6, uniforms=u))
+        both(lambda x: x.run_steps(1100, noise_rate=2.0 ** -6))  # more than one batch
+        assert a._mode == (2 if n >= 2000 and k == 0 else 0) and b._mode == 0
+        a.update_conn_weight((ch, post, src), np.full(50, 0.5, np.float32))
+        b.update_conn_weight((ch, post, src), np.full(50, 0.5, np.float32))
+    both(lambda x: x.run_steps(3, noise_rate=2.0 ** -6))
+    assert np.array_equal(a.V_i.numpy(), b.V_i.numpy())
+    assert np.array_equal(a.J_ui.numpy(), b.J_ui.numpy())
