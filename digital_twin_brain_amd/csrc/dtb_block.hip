@@ -25,6 +25,7 @@
 // instead of a [D][n] ring.  J_n = Jp_n + acc once the step's delivery ran.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
@@ -86,6 +87,10 @@ constexpr int kSubLists = 32;
 constexpr int kCntStride = 32;
 constexpr int kMaxEntries = DTB_MAX_DELAY * kSubLists; // (delay, sub-list) entries of a delivery
 constexpr int kCursorStride = 32;    // one 128-byte line per bucket cursor / overflow flag / list count
+constexpr int64_t kFewEventsNnz = 1ll << 26;
+constexpr int64_t kMinEvents = 160;  // events that a stage workgroup takes at least (58,000 events a step on a
+                                     // 160,000-neuron block: 37.0 us a step with 1,024 workgroups of 57,
+                                     // 26.8 with 256, 27.8 with 512)
 constexpr int kEvParts = 32;         // partial event counters of a stage kernel, a line each
 constexpr int kEvStride = 16;        // 64-bit words between them
 
@@ -151,6 +156,8 @@ struct NeuronArgs {
     void* __restrict__ acc;
     int32_t* __restrict__ spk;     // [L][kSubLists][spk_cap]
     uint32_t* __restrict__ spk_cnt; // [L][kSubLists] (kCntStride apart)
+    uint32_t* __restrict__ cc;      // [L][kSubLists] the counts of earlier steps, contiguous
+    uint32_t* __restrict__ pcum;    // [(D - 1) kSubLists + 1] prefix sums of the earlier steps' counts
     int64_t spk_cap;
     int32_t L;         // spike-list slots (D + 1)
     int32_t clear_acc; // direct delivery accumulates into acc, so it is cleared after reading
@@ -318,7 +325,7 @@ __device__ __forceinline__ void neuron_update(const NeuronArgs& a, int64_t i, in
 }
 
 // Per sub-population statistics of a step (threshold spikes, V sum).  Bound by
-// the adds to one address, ~11 ns each in turn when a block has few
+// the adds to one address, ~11 ns each in turn, when a block has few
 // populations, so a population gets one add per workgroup: every wavefront
 // whose neurons share a population leaves its sums in LDS (others add theirs
 // lane by lane), and after a barrier the first wavefront of each population
@@ -375,96 +382,9 @@ __device__ __forceinline__ void group_stats(const NeuronArgs& a, int32_t k, int 
     if (a.rec_vsum) unsafeAtomicAdd(&a.rec_vsum[(int64_t)k * a.S + p], v);
 }
 
-template <bool PAIR, bool PSET>
-__global__ __launch_bounds__(256) void neuron_step_kernel(NeuronArgs a, int32_t k)
-{
-    __shared__ uint32_t s_wcnt[4];
-    __shared__ uint32_t s_base;
-    __shared__ StatsLds<4> s_stats;
-    __shared__ float s_tab[kMaxPsets * 16];
-    if (PSET) {
-        for (int x = threadIdx.x; x < a.npsets * 16; x += 256) s_tab[x] = a.ptab[x];
-        __syncthreads();
-    }
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t step = a.ctl->nbase + k + 1;
-    const double t = a.ttab[k];
-    const int32_t slot = (int32_t)(step % a.L);
-    // the list of step+1 reuses the slot of step+1-L, whose last delivery was step
-    if (blockIdx.x == 0 && threadIdx.x < kSubLists)
-        a.spk_cnt[((int64_t)((step + 1) % a.L) * kSubLists + threadIdx.x) * kCntStride] = 0;
-
-    bool act = false, spike = false;
-    float vout = 0.0f;
-    int32_t p = -1;
-    if (i < a.n) {
-        p = a.pop[i];
-        neuron_update<PAIR, PSET, true>(a, i, step, t, k, make_float4(0.f, 0.f, 0.f, 0.f), s_tab, act, spike, vout);
-    }
-
-    // spike compaction: ballot + per-wave prefix, one global atomic per workgroup
-    const uint32_t lane = __lane_id();
-    const uint32_t wid = threadIdx.x >> 6;
-    const uint64_t m = __ballot(spike);
-    const uint32_t pre = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) s_wcnt[wid] = (uint32_t)__popcll(m);
-    const bool stats = a.rec_freq || a.rec_vsum;
-    if (stats) wave_stats<4>(a, k, p, act, vout, wid, s_stats);
-    __syncthreads();
-    if (stats && threadIdx.x >= 64 && threadIdx.x < 68) group_stats<4>(a, k, (int)threadIdx.x - 64, s_stats);
-    const int64_t sl = (int64_t)slot * kSubLists + blockIdx.x % kSubLists;
-    if (threadIdx.x == 0) {
-        const uint32_t tot = s_wcnt[0] + s_wcnt[1] + s_wcnt[2] + s_wcnt[3];
-        s_base = tot ? atomicAdd(&a.spk_cnt[sl * kCntStride], tot) : 0u;
-    }
-    __syncthreads();
-    if (spike) {
-        uint32_t off = s_base;
-        for (uint32_t w = 0; w < wid; ++w) off += s_wcnt[w];
-        a.spk[sl * a.spk_cap + off + pre] = (int32_t)i;
-    }
-}
-
-struct DeliverArgs {
-    int64_t n;
-    int32_t D, L;
-    SynPack pk;
-    const int64_t* __restrict__ rowptr;
-    const uint16_t* __restrict__ dend; // [n][D] end of each delay segment, relative to the row start
-    const uint32_t* __restrict__ col;
-    const float* __restrict__ w;
-    const float2* __restrict__ w2;
-    void* __restrict__ acc;
-    const int32_t* __restrict__ spk;
-    const uint32_t* __restrict__ spk_cnt;
-    int64_t spk_cap;
-    const StepCtl* __restrict__ ctl;
-    uint64_t* __restrict__ rec_events;
-    uint32_t* __restrict__ rec_nspk;
-};
-
 // Inclusive scan over the 256 lanes of a workgroup (shuffles within each
 // wavefront, then the four wavefront totals through LDS).
 __device__ inline uint32_t block_inclusive_scan_256(uint32_t v, uint32_t* wtot)
-{
-    const uint32_t lane = __lane_id();
-    const uint32_t wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t y = __shfl_up(v, off);
-        if (lane >= (uint32_t)off) v += y;
-    }
-    if (lane == kWave - 1) wtot[wid] = v;
-    __syncthreads();
-    uint32_t add = 0;
-    for (uint32_t w = 0; w < wid; ++w) add += wtot[w];
-    __syncthreads();
-    return v + add;
-}
-
-// Inclusive scan over the W wavefronts of a workgroup (W * 64 lanes).
-template <int W>
-__device__ inline uint32_t block_inclusive_scan_n(uint32_t v, uint32_t* wtot)
 {
     const uint32_t lane = __lane_id();
     const uint32_t wid = threadIdx.x >> 6;
@@ -489,23 +409,159 @@ __device__ inline int32_t delay_slot(int32_t s0, int32_t d, int32_t L)
     return s < 0 ? s + L : s;
 }
 
-// where sub-list entry e = (d - 1) * kSubLists + q starts in spk, for the
-// step whose slot is s0
-__device__ inline int64_t entry_base(const DeliverArgs& a, int32_t s0, int32_t e)
+// Delivery entries: entry e < (D - 1) kSubLists is sub-list e % kSubLists of the
+// step that spiked e / kSubLists + 1 steps ago (delay e / kSubLists + 2), the
+// last kSubLists entries are the step's own (delay 1).  The counts of the
+// earlier steps are final before the step begins, so one extra workgroup of
+// the neuron kernel turns them into prefix sums, which every workgroup of the
+// delivery then reads contiguously: read from the counters they are a line
+// each, 1,280 lines and a scan for each of 1,024 workgroups with 40 delays.
+// The extra workgroup itself keeps a contiguous copy of the counts (cc, by
+// spike-list slot): in a batch's first step it reads all of them from the
+// counters, later only those of the step before.
+__device__ inline void earlier_entries(const NeuronArgs& a, int32_t k, int32_t slot, uint32_t* wtot)
 {
-    const int32_t d = e / kSubLists + 1, q = e % kSubLists;
-    return ((int64_t)delay_slot(s0, d, a.L) * kSubLists + q) * a.spk_cap;
+    const int32_t E = (a.D - 1) * kSubLists;
+    constexpr int kPer = kMaxEntries / 256;
+    static_assert(kSubLists % kPer == 0, "a lane's entries belong to one step");
+    uint32_t c[kPer];
+    uint32_t sum = 0;
+    const int32_t e0 = threadIdx.x * kPer;
+    if (e0 < E) {
+        const int32_t x0 = delay_slot(slot, e0 / kSubLists + 2, a.L) * kSubLists + e0 % kSubLists;
+        const bool counters = k == 0 || e0 < kSubLists;
+#pragma unroll
+        for (int x = 0; x < kPer; ++x) c[x] = counters ? a.spk_cnt[(int64_t)(x0 + x) * kCntStride] : a.cc[x0 + x];
+#pragma unroll
+        for (int x = 0; x < kPer; ++x) {
+            c[x] = min(c[x], (uint32_t)a.spk_cap);
+            if (counters) a.cc[x0 + x] = c[x];
+            sum += c[x];
+        }
+    }
+    uint32_t run = block_inclusive_scan_256(sum, wtot) - sum;
+    if (threadIdx.x == 0) a.pcum[0] = 0;
+    if (e0 < E) {
+#pragma unroll
+        for (int x = 0; x < kPer; ++x) {
+            run += c[x];
+            a.pcum[e0 + x + 1] = run;
+        }
+    }
 }
 
-// Segments to deliver at batch step k: entry e = (d - 1) * kSubLists + q holds
-// sub-list q of the step that spiked d - 1 steps ago; cum[e + 1] = segments in
-// entries <= e.  Workgroups of 256 threads; returns the number of entries.
-// Every counter load is issued before the first is waited for (entries past
-// E read entry E - 1's counter and are then dropped).
-__device__ inline int32_t delivery_entries(const DeliverArgs& a, int32_t k, uint32_t* cum, uint32_t* wtot)
+template <bool PAIR, bool PSET>
+__global__ __launch_bounds__(256) void neuron_step_kernel(NeuronArgs a, int32_t k)
 {
+    __shared__ uint32_t s_wcnt[4];
+    __shared__ uint32_t s_base;
+    __shared__ StatsLds<4> s_stats;
+    __shared__ float s_tab[kMaxPsets * 16];
+    if (PSET) {
+        for (int x = threadIdx.x; x < a.npsets * 16; x += 256) s_tab[x] = a.ptab[x];
+        __syncthreads();
+    }
+    const uint32_t wg = a.pcum ? blockIdx.x - 1u : blockIdx.x;
+    const int64_t i = (int64_t)wg * 256 + threadIdx.x;
     const int64_t step = a.ctl->nbase + k + 1;
-    const int32_t s0 = (int32_t)(step % a.L);
+    const double t = a.ttab[k];
+    const int32_t slot = (int32_t)(step % a.L);
+    if (a.pcum && blockIdx.x == 0) { // the extra workgroup, ahead of the others
+        earlier_entries(a, k, slot, s_wcnt);
+        return;
+    }
+    // the list of step+1 reuses the slot of step+1-L, whose last delivery was step
+    if (wg == 0 && threadIdx.x < kSubLists)
+        a.spk_cnt[((int64_t)((step + 1) % a.L) * kSubLists + threadIdx.x) * kCntStride] = 0;
+
+    bool act = false, spike = false;
+    float vout = 0.0f;
+    int32_t p = -1;
+    if (i < a.n) {
+        p = a.pop[i];
+        neuron_update<PAIR, PSET, true>(a, i, step, t, k, make_float4(0.f, 0.f, 0.f, 0.f), s_tab, act, spike, vout);
+    }
+
+    // spike compaction: ballot + per-wave prefix, one global atomic per workgroup
+    const uint32_t lane = __lane_id();
+    const uint32_t wid = threadIdx.x >> 6;
+    const uint64_t m = __ballot(spike);
+    const uint32_t pre = (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    if (lane == 0) s_wcnt[wid] = (uint32_t)__popcll(m);
+    const bool stats = a.rec_freq || a.rec_vsum;
+    if (stats) wave_stats<4>(a, k, p, act, vout, wid, s_stats);
+    __syncthreads();
+    if (stats && threadIdx.x >= 64 && threadIdx.x < 68) group_stats<4>(a, k, (int)threadIdx.x - 64, s_stats);
+    const int64_t sl = (int64_t)slot * kSubLists + wg % kSubLists;
+    if (threadIdx.x == 0) {
+        const uint32_t tot = s_wcnt[0] + s_wcnt[1] + s_wcnt[2] + s_wcnt[3];
+        s_base = tot ? atomicAdd(&a.spk_cnt[sl * kCntStride], tot) : 0u;
+    }
+    __syncthreads();
+    if (spike) {
+        uint32_t off = s_base;
+        for (uint32_t w = 0; w < wid; ++w) off += s_wcnt[w];
+        a.spk[sl * a.spk_cap + off + pre] = (int32_t)i;
+    }
+}
+
+struct DeliverArgs {
+    int64_t n;
+    int32_t D, L;
+    SynPack pk;
+    const int64_t* __restrict__ rowptr;
+    const uint16_t* __restrict__ dend; // [n][D] end of each delay segment, relative to the row start
+    const uint32_t* __restrict__ col;
+    const float* __restrict__ w;
+    const float2* __restrict__ w2;
+    void* __restrict__ acc;
+    const int32_t* __restrict__ spk;
+    const uint32_t* __restrict__ spk_cnt;
+    const uint32_t* __restrict__ pcum;
+    int64_t spk_cap;
+    const StepCtl* __restrict__ ctl;
+    uint64_t* __restrict__ rec_events;
+    uint32_t* __restrict__ rec_nspk;
+};
+
+// Inclusive scan over the W wavefronts of a workgroup (W * 64 lanes).
+template <int W>
+__device__ inline uint32_t block_inclusive_scan_n(uint32_t v, uint32_t* wtot)
+{
+    const uint32_t lane = __lane_id();
+    const uint32_t wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t y = __shfl_up(v, off);
+        if (lane >= (uint32_t)off) v += y;
+    }
+    if (lane == kWave - 1) wtot[wid] = v;
+    __syncthreads();
+    uint32_t add = 0;
+    for (uint32_t w = 0; w < wid; ++w) add += wtot[w];
+    __syncthreads();
+    return v + add;
+}
+
+// the delay of delivery entry e
+__device__ inline int32_t entry_delay(int32_t D, int32_t e)
+{
+    const int32_t d = e / kSubLists + 2;
+    return d > D ? 1 : d;
+}
+
+// where the sub-list of entry e (of delay d) starts in spk, for the step whose slot is s0
+__device__ inline int64_t entry_base(const DeliverArgs& a, int32_t s0, int32_t e, int32_t d)
+{
+    return ((int64_t)delay_slot(s0, d, a.L) * kSubLists + e % kSubLists) * a.spk_cap;
+}
+
+// Segments to deliver at batch step k, from the counters: cum[e + 1] =
+// segments in entries <= e.  Workgroups of 256 threads; returns the number of
+// entries.  Every counter load is issued before the first is waited for
+// (entries past E read entry E - 1's counter and are then dropped).
+__device__ inline int32_t delivery_entries(const DeliverArgs& a, int32_t s0, uint32_t* cum, uint32_t* wtot)
+{
     const int32_t E = a.D * kSubLists;
     constexpr int kPer = kMaxEntries / 256;
     uint32_t c[kPer];
@@ -514,8 +570,7 @@ __device__ inline int32_t delivery_entries(const DeliverArgs& a, int32_t k, uint
 #pragma unroll
     for (int x = 0; x < kPer; ++x) {
         const int32_t e = min(e0 + x, E - 1);
-        const int32_t d = e / kSubLists + 1, q = e % kSubLists;
-        c[x] = a.spk_cnt[((int64_t)delay_slot(s0, d, a.L) * kSubLists + q) * kCntStride];
+        c[x] = a.spk_cnt[((int64_t)delay_slot(s0, entry_delay(a.D, e), a.L) * kSubLists + e % kSubLists) * kCntStride];
     }
 #pragma unroll
     for (int x = 0; x < kPer; ++x) {
@@ -531,6 +586,53 @@ __device__ inline int32_t delivery_entries(const DeliverArgs& a, int32_t k, uint
     }
     __syncthreads();
     return E;
+}
+
+// The same from the prefix sums of the earlier entries (earlier_entries), in
+// two parts: the loads, all in flight together -- the step's own counts (the
+// first kSubLists lanes of every wavefront), the earlier entries' total and
+// this lane's share of their sums -- and the LDS copy.
+struct EntryCounts {
+    uint32_t own, earlier, total;
+    uint32_t pre[kMaxEntries / 256];
+};
+
+__device__ inline void load_entry_counts(const DeliverArgs& a, int32_t s0, EntryCounts& c)
+{
+    const uint32_t lane = __lane_id();
+    const int32_t E0 = (a.D - 1) * kSubLists;
+    c.own = lane < kSubLists ? a.spk_cnt[((int64_t)s0 * kSubLists + lane) * kCntStride] : 0u;
+    c.earlier = 0u;
+    if (E0 > 0) { // uniform
+        c.earlier = a.pcum[E0];
+#pragma unroll
+        for (int x = 0; x < kMaxEntries / 256; ++x)
+            if (x * 256 < E0) c.pre[x] = a.pcum[min(x * 256 + (int32_t)threadIdx.x, E0)]; // uniform
+    }
+    c.own = min(c.own, (uint32_t)a.spk_cap);
+    uint32_t v = c.own;
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    c.total = c.earlier + v;
+}
+
+__device__ inline int32_t delivery_entries(const DeliverArgs& a, const EntryCounts& c, uint32_t* cum)
+{
+    const int32_t E0 = (a.D - 1) * kSubLists;
+#pragma unroll
+    for (int x = 0; x < kMaxEntries / 256; ++x)
+        if (x * 256 + (int32_t)threadIdx.x < E0) cum[x * 256 + threadIdx.x] = c.pre[x];
+    if (threadIdx.x < kWave) {
+        uint32_t v = c.own;
+#pragma unroll
+        for (int off = 1; off < kSubLists; off <<= 1) {
+            const uint32_t y = __shfl_up(v, off);
+            if (threadIdx.x >= off) v += y;
+        }
+        if (threadIdx.x < kSubLists) cum[E0 + 1 + threadIdx.x] = c.earlier + v;
+        if (threadIdx.x == 0) cum[E0] = c.earlier;
+    }
+    __syncthreads();
+    return E0 + kSubLists;
 }
 
 // entry holding segment g (cum[E] > g): the last e with cum[e] <= g
@@ -553,20 +655,20 @@ __global__ __launch_bounds__(256) void deliver_kernel(DeliverArgs a, int32_t k)
     __shared__ uint32_t cum[kMaxEntries + 1];
     __shared__ uint32_t wtot[4];
     const int32_t s0 = (int32_t)((a.ctl->nbase + k + 1) % a.L);
-    const int32_t E = delivery_entries(a, k, cum, wtot);
+    const int32_t E = delivery_entries(a, s0, cum, wtot);
     const uint32_t total = cum[E];
     const uint32_t lane = __lane_id();
     const uint32_t sub = lane % G;
     constexpr uint32_t kGroups = kWave / G;
     const uint32_t gid = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kGroups + lane / G;
     const uint32_t ngroups = ((gridDim.x * blockDim.x) >> 6) * kGroups;
-    if (gid == 0 && sub == 0 && a.rec_nspk) a.rec_nspk[k] = cum[kSubLists];
+    if (gid == 0 && sub == 0 && a.rec_nspk) a.rec_nspk[k] = total - cum[E - kSubLists];
     uint64_t ev = 0;
     int32_t e = 0;
     for (uint32_t r = gid; r < total; r += ngroups) {
         while (r >= cum[e + 1]) ++e; // r only grows, so e only moves forward
-        const int32_t d = e / kSubLists + 1;
-        const int32_t j = a.spk[entry_base(a, s0, e) + (r - cum[e])];
+        const int32_t d = entry_delay(a.D, e);
+        const int32_t j = a.spk[entry_base(a, s0, e, d) + (r - cum[e])];
         const int64_t row = a.rowptr[j];
         int64_t beg, end;
         if (a.D == 1) {
@@ -665,6 +767,7 @@ struct StageArgs {
     uint32_t* ovf;    // [nbk] overflow flags
     SegArgs sg;       // segment lists
     int32_t k;        // batch step (the accumulation kernel clears the step's segment list)
+    uint32_t min_segs; // segments that a workgroup takes at least
     uint64_t* evp;    // [kEvParts][kEvStride] events counted by the stage kernel's workgroups
 };
 
@@ -762,7 +865,8 @@ __device__ inline void stage_put(const StageArgs& s, int32_t part, uint32_t bk, 
 //      targets, then a second pass that stores (targets read twice);
 //   2  one reservation per (round, bucket), the round's events first sorted
 //      by bucket in LDS so that consecutive lanes store each bucket's run
-//      contiguously (whole cache lines instead of scattered 8-byte stores).
+//      contiguously (whole cache lines instead of scattered 8-byte stores);
+//   3  as 2, but chunks of few events as in 0, one event per lane.
 // Four workgroups per CU at 16 events per lane: registers are capped at 128
 // per lane and the dynamic LDS holds only what the block needs (entries of
 // its delays, its buckets, the sorted round), so a launch of up to 4 x CUs
@@ -789,7 +893,7 @@ __global__ __launch_bounds__(256, EPT <= 16 ? 4 : 2) void deliver_stage_kernel(S
     bool use_seg = false;
     uint32_t total = 0;
     int64_t seg0 = 0;
-    if (s.sg.seg) {
+    if (VAR != 3 && s.sg.seg) {
         const int64_t step = a.ctl->nbase + k + 1;
         const int32_t ls = (int32_t)(step % a.D);
         const uint32_t* c = s.sg.cnt + (int64_t)ls * kCursorStride;
@@ -798,22 +902,33 @@ __global__ __launch_bounds__(256, EPT <= 16 ? 4 : 2) void deliver_stage_kernel(S
         seg0 = (int64_t)ls * s.sg.cap;
     }
     int32_t NE = 0;
-    if (!use_seg) {
-        NE = delivery_entries(a, k, cum, wtot);
+    uint64_t G = gridDim.x;
+    if constexpr (VAR == 3) {
+        EntryCounts ec;
+        load_entry_counts(a, s0, ec);
+        total = __builtin_amdgcn_readfirstlane(ec.total); // the same in every lane
+        if (blockIdx.x == 0 && t == 0 && a.rec_nspk) a.rec_nspk[k] = ec.total - ec.earlier;
+        // Workgroups that would get a handful of events leave the work to the
+        // others: what a workgroup spends before and after its events (and its
+        // reservations, an atomic per event when the events are few) is the
+        // same for any number of them.
+        G = min((uint32_t)gridDim.x, max(1u, total / s.min_segs));
+        if (blockIdx.x >= G) return;
+        NE = delivery_entries(a, ec, cum);
+    } else if (!use_seg) {
+        NE = delivery_entries(a, s0, cum, wtot);
         total = cum[NE];
-        if (blockIdx.x == 0 && t == 0 && a.rec_nspk) a.rec_nspk[k] = cum[kSubLists];
+        if (blockIdx.x == 0 && t == 0 && a.rec_nspk) a.rec_nspk[k] = total - cum[NE - kSubLists];
     } else if (blockIdx.x == 0 && t < 64 && a.rec_nspk) {
         // the step's spikes: the sum of its sub-list counts
-        const int32_t slot = (int32_t)((a.ctl->nbase + k + 1) % a.L);
-        uint32_t c = t < kSubLists ? min(a.spk_cnt[((int64_t)slot * kSubLists + t) * kCntStride], (uint32_t)a.spk_cap)
+        uint32_t c = t < kSubLists ? min(a.spk_cnt[((int64_t)s0 * kSubLists + t) * kCntStride], (uint32_t)a.spk_cap)
                                    : 0u;
         for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o);
         if (t == 0) a.rec_nspk[k] = c;
     }
-    // The step's segments in kper * gridDim chunks of equal size (at most
+    // The step's segments in kper * G chunks of equal size (at most
     // SEG), dealt round-robin: every workgroup gets kper chunks, and each
     // gets chunks from all delays (segment lengths vary with the delay).
-    const uint64_t G = gridDim.x;
     const uint64_t kper = ((uint64_t)total + G * SEG - 1) / (G * SEG);
     const uint64_t nch = G * kper;
     const uint64_t cs = nch ? ((uint64_t)total + nch - 1) / nch : 0;
@@ -831,8 +946,8 @@ __global__ __launch_bounds__(256, EPT <= 16 ? 4 : 2) void deliver_stage_kernel(S
             len = (uint32_t)(v & 0xffffffu);
         } else if (t < SEG && g < g_end) {
             const int32_t e = entry_of(cum, NE, g);
-            const int32_t d = e / kSubLists + 1;
-            const int32_t j = a.spk[entry_base(a, s0, e) + (g - cum[e])];
+            const int32_t d = entry_delay(a.D, e);
+            const int32_t j = a.spk[entry_base(a, s0, e, d) + (g - cum[e])];
             const int64_t row = a.rowptr[j];
             int64_t end;
             if (a.D == 1) {
@@ -855,6 +970,34 @@ __global__ __launch_bounds__(256, EPT <= 16 ? 4 : 2) void deliver_stage_kernel(S
         __syncthreads();
         const uint32_t E = segpre[SEG];
         ev_wg += E;
+        if constexpr (VAR == 3) {
+            // a chunk of at most 256 events: one event per lane, stored as it
+            // lies (a round of EPT events a lane costs its address arithmetic
+            // and LDS reads whether they are there or not)
+            if (E <= 256) {
+                uint32_t loc[1], cw[1];
+                float w0[1], w1[1];
+                stage_locate<SEG, 1>(segpre, 0, E, t, loc);
+                stage_load<PAIR, 1>(a, segbeg, loc, cw, w0, w1);
+                const bool ok = loc[0] != 0xffffffffu;
+                const uint32_t post = cw[0] & a.pk.idx_mask;
+                const uint32_t bk = (uint32_t)(((uint64_t)post * s.bmagic) >> s.bshift);
+                const uint32_t rank = ok ? atomicAdd(&hist[bk], 1u) : 0u;
+                __syncthreads();
+                for (int b = t; b < s.nbk; b += 256) {
+                    const uint32_t h = hist[b];
+                    hist[b] = h ? atomicAdd(&s.cursor[((size_t)b * kStageParts + part) * kCursorStride], h) : 0u;
+                }
+                __syncthreads();
+                if (ok)
+                    stage_put<PAIR>(s, part, bk, (uint64_t)hist[bk] + rank,
+                                    (post - bk * (uint32_t)s.bsize) | (cw[0] & 0x80000000u), w0[0], w1[0]);
+                __syncthreads();
+                for (int b = t; b < s.nbk; b += 256) hist[b] = 0;
+                __syncthreads();
+                continue;
+            }
+        }
         if constexpr (VAR == 0) {
             for (uint32_t r0 = 0; r0 < E; r0 += 256 * EPT) {
                 uint32_t br[EPT], pk_[EPT]; // br = bucket << kRankBits | rank
@@ -895,7 +1038,7 @@ __global__ __launch_bounds__(256, EPT <= 16 ? 4 : 2) void deliver_stage_kernel(S
                 for (int b = t; b < s.nbk; b += 256) hist[b] = 0;
                 __syncthreads();
             }
-        } else if constexpr (VAR == 2) {
+        } else if constexpr (VAR >= 2) {
             uint32_t* pre = hist + s.nbk; // [nbk] first LDS slot of each bucket in the round
             // [nbk] staging index of the round's slot 0 for that bucket when the
             // bucket's whole reservation fits its partition, else kPartial
@@ -1150,6 +1293,20 @@ __global__ void segment_reset_kernel(uint32_t* cnt, int32_t D, int64_t from)
     if (threadIdx.x == 0) *reinterpret_cast<int64_t*>(cnt + (int64_t)D * kCursorStride) = from;
 }
 
+// Whether the stage kernel is the one for steps of few events (variant 3):
+// segments of up to 16 synapses, of which a small chunk has few events, and so
+// few synapses that at some 30 Hz a step's events (1 in 300) leave most of the
+// 1,024 workgroups fewer than 256.  Others, and blocks with segment lists, do
+// without its counts, its limit of workgroups and its second path, whose
+// registers cost them 2 to 5%.  us a step, without and with: 4 M synapses, 40
+// delays 34.6 and 20.8; 16 M 38.3 and 25.5; 40 M 44.0 and 38.8; 60 M 49.2 and
+// 46.0, with 10 delays 37.6 and 36.7.
+static bool short_segments(const Block* b)
+{
+    return b->deliver_mode >= 1 && b->stage_variant == 2 && !(b->seg && b->seg_cap > 0 && b->D > 1) &&
+           b->nnz <= 16 * b->n * b->D && b->nnz <= kFewEventsNnz;
+}
+
 // dynamic LDS of the stage kernel: the delivery entries and the bucket
 // histogram, plus for the sorted variant the round's bucket offsets,
 // reservations and sorted events
@@ -1157,7 +1314,7 @@ static size_t stage_lds(const Block* b, int ept, int var)
 {
     size_t words = (size_t)b->D * kSubLists + 1 + (size_t)b->nbk;
     // + pre, off, one word of alignment, the round with a spare slot
-    if (var == 2) words += 2 * (size_t)b->nbk + 1 + ((size_t)256 * ept + 1) * (b->pair ? 3 : 2);
+    if (var >= 2) words += 2 * (size_t)b->nbk + 1 + ((size_t)256 * ept + 1) * (b->pair ? 3 : 2);
     return sizeof(uint32_t) * words;
 }
 
@@ -1177,7 +1334,10 @@ template <bool PAIR>
 static void launch_stage(const Block* b, const StageArgs& sa, int32_t k)
 {
     switch (b->stage_variant) {
-    case 2: launch_stage_ept<PAIR, 16, 2>(b, sa, k); break; // sorted rounds use 16 events per lane
+    case 2: // sorted rounds use 16 events per lane
+        if (short_segments(b)) launch_stage_ept<PAIR, 16, 3>(b, sa, k);
+        else launch_stage_ept<PAIR, 16, 2>(b, sa, k);
+        break;
     case 1:
         if (b->stage_ept == 16) launch_stage_ept<PAIR, 16, 1>(b, sa, k);
         else launch_stage_ept<PAIR, 32, 1>(b, sa, k);
@@ -1452,14 +1612,14 @@ static int update_jexp(Block* b, bool with_state)
     return DTB_OK;
 }
 
-template <bool PAIR>
+template <bool PAIR, int VAR>
 static int allow_sorted_stage_lds(int bytes)
 {
-    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 64, 16, 2>,
+    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 64, 16, VAR>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 128, 16, 2>,
+    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 128, 16, VAR>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 256, 16, 2>,
+    DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_stage_kernel<PAIR, 256, 16, VAR>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     return DTB_OK;
 }
@@ -2520,6 +2680,8 @@ static int alloc_state(Block* b)
     b->spk_cap = spk_cap_of(n);
     DTB_TRY(alloc_n(b, &b->spk, (int64_t)(b->D + 1) * kSubLists * b->spk_cap));
     DTB_TRY(alloc_n(b, &b->spk_cnt, (int64_t)(b->D + 1) * kSubLists * kCntStride));
+    DTB_TRY(alloc_n(b, &b->spk_cc, (int64_t)(b->D + 1) * kSubLists));
+    DTB_TRY(alloc_n(b, &b->pcum, (int64_t)(b->D - 1) * kSubLists + 1));
     DTB_TRY(alloc_n(b, &b->ctl, 1));
     b->kmax = 1000;
     DTB_TRY(alloc_n(b, &b->ttab, b->kmax));
@@ -2664,8 +2826,10 @@ static int ensure_bucketed(Block* b)
                                     hipFuncAttributeMaxDynamicSharedMemorySize, b->lds_max - kAccumStaticLds));
     DTB_TRY_HIP(hipFuncSetAttribute((const void*)deliver_accum_kernel<false, 16, false>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, b->lds_max - kAccumStaticLds));
-    DTB_TRY(allow_sorted_stage_lds<true>(b->lds_max - kStageStaticLds));
-    DTB_TRY(allow_sorted_stage_lds<false>(b->lds_max - kStageStaticLds));
+    DTB_TRY((allow_sorted_stage_lds<true, 2>(b->lds_max - kStageStaticLds)));
+    DTB_TRY((allow_sorted_stage_lds<false, 2>(b->lds_max - kStageStaticLds)));
+    DTB_TRY((allow_sorted_stage_lds<true, 3>(b->lds_max - kStageStaticLds)));
+    DTB_TRY((allow_sorted_stage_lds<false, 3>(b->lds_max - kStageStaticLds)));
     int64_t nbk_max = 0, events_max = 0;
     for (int occ = 1; occ <= 2; ++occ) {
         const BucketGeom g = bucket_geom(b, occ);
@@ -2917,7 +3081,7 @@ static NeuronArgs neuron_args(Block* b, const dtb_run_args* a, const float* unif
     x.src = b->src;
     x.pset = b->pset; x.ptab = b->ptab; x.npsets = b->npsets;
     x.V = b->V; x.Jp = b->Jp; x.ref_end = b->ref_end; x.last_step = b->last_step; x.t_last = b->t_last;
-    x.flags = b->flags; x.acc = b->acc; x.spk = b->spk; x.spk_cnt = b->spk_cnt; x.spk_cap = b->spk_cap;
+    x.flags = b->flags; x.acc = b->acc; x.spk = b->spk; x.spk_cnt = b->spk_cnt; x.cc = b->spk_cc; x.pcum = b->D > 1 && short_segments(b) ? b->pcum : nullptr; x.spk_cap = b->spk_cap;
     x.L = b->D + 1; x.ctl = b->ctl;
     x.clear_acc = b->deliver_mode == 0;
     x.ttab = b->ttab;
@@ -2934,7 +3098,7 @@ static DeliverArgs deliver_args(Block* b)
     DeliverArgs x;
     x.n = b->n; x.D = b->D; x.L = b->D + 1; x.pk = b->pk; x.rowptr = b->rowptr; x.dend = b->dend; x.col = b->col;
     x.w = b->w; x.w2 = b->w2;
-    x.acc = b->acc; x.spk = b->spk; x.spk_cnt = b->spk_cnt; x.spk_cap = b->spk_cap; x.ctl = b->ctl;
+    x.acc = b->acc; x.spk = b->spk; x.spk_cnt = b->spk_cnt; x.pcum = b->pcum; x.spk_cap = b->spk_cap; x.ctl = b->ctl;
     x.rec_events = b->rec_events;
     x.rec_nspk = b->rec_nspk;
     return x;
@@ -3012,7 +3176,7 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
                        b->rec_nspk, b->pbar);
     const NeuronArgs na = neuron_args(b, a, uniforms, w.freq, w.vsum);
     const DeliverArgs da = deliver_args(b);
-    const unsigned ng = grid_for(b->n, 256);
+    const unsigned ng = grid_for(b->n, 256) + (na.pcum ? 1 : 0); // one more for the earlier entries
     if (persist_batch(b, a, w)) {
         PersistArgs pa;
         pa.na = na;
@@ -3054,8 +3218,11 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
         if (w.timing) DTB_TRY_HIP(hipEventRecord(b->events[(size_t)(3 * k + 1)], b->stream));
         if (b->deliver_mode >= 1) {
             const SegArgs sg = seg_args(b);
+            // about kMinEvents events, by the mean length of a segment
+            const uint32_t min_segs = (uint32_t)std::min<int64_t>(
+                64, std::max<int64_t>(1, kMinEvents * b->n * b->D / std::max<int64_t>(b->nnz, 1)));
             StageArgs sa{da, b->nbk, b->bsize, b->bmagic, b->bshift, b->stage_cap, b->cursor, b->stage, b->acc2,
-                         b->ovf, sg, k, b->ev_part};
+                         b->ovf, sg, k, min_segs, b->ev_part};
             if (sg.seg)
                 hipLaunchKernelGGL(segment_emit_kernel, dim3((unsigned)std::min<int64_t>(1024, (b->n + 255) / 256)),
                                    dim3(256), 0, b->stream, da, sg, k);
@@ -3074,9 +3241,9 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
         if (w.timing) DTB_TRY_HIP(hipEventRecord(b->events[(size_t)(3 * k + 2)], b->stream));
         if (w.isum) {
             if (b->pair)
-                hipLaunchKernelGGL(isum_kernel<true>, dim3(ng), dim3(256), 0, b->stream, na, k, b->rec_isum);
+                hipLaunchKernelGGL(isum_kernel<true>, dim3(grid_for(b->n, 256)), dim3(256), 0, b->stream, na, k, b->rec_isum);
             else
-                hipLaunchKernelGGL(isum_kernel<false>, dim3(ng), dim3(256), 0, b->stream, na, k, b->rec_isum);
+                hipLaunchKernelGGL(isum_kernel<false>, dim3(grid_for(b->n, 256)), dim3(256), 0, b->stream, na, k, b->rec_isum);
         }
         if (w.bold && (k + 1) % b->bold_sps == 0)
             hipLaunchKernelGGL(bold_counts_kernel, dim3(grid_for(b->nvox, 256)), dim3(256), 0, b->stream, b->S,

@@ -62,6 +62,8 @@ struct Block {
     // spike lists of the last D+1 steps (slot = step mod (D+1))
     int32_t* spk = nullptr;      // [D+1][sub-lists][spk_cap]
     uint32_t* spk_cnt = nullptr; // [D+1][sub-lists], padded
+    uint32_t* spk_cc = nullptr;  // [D+1][sub-lists] counts of the earlier steps of a batch, contiguous
+    uint32_t* pcum = nullptr;    // [(D-1) sub-lists + 1] prefix sums of the earlier steps' counts
     int64_t spk_cap = 0;         // entries per sub-list
 
     StepCtl* ctl = nullptr;

@@ -480,6 +480,36 @@ def test_bucketed_delivery_matches_atomics_including_overflow(pair):
     assert outs[0][2][:20].max() > 3 * 8192 * 3  # some bucket saw more events than its staging room
 
 
+# the stage kernel for steps of few events (segments of at most 16 synapses): a workgroup or
+# none at work, chunks of up to 256 events and larger ones, one delay and the most, across batches
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("n,K,D", [(300, 10, 1), (5000, 60, 4), (20001, 100, 40), (4000, 64, 64)])
+def test_short_segment_delivery_matches_atomics(n, K, D, pair):
+    from digital_twin_brain_amd import NativeBlock
+
+    rng = np.random.default_rng(n + D)
+    props = _plain_like_props(n, n * 4 // 5, rng, g_scale=0.2)
+    ref = orc.gen_fixed_indegree(n, n * 4 // 5, K, D, 0.0, 1.0, pair, seed=n)
+    for key in ("w0", "w1"):
+        if ref.get(key) is not None:
+            ref[key] = (np.floor(ref[key] * 64) / 64).astype(np.float32)
+    outs = []
+    for mode, segs in ((0, 128), (1, 64), (1, 256)):
+        nb = NativeBlock.from_csr(props, ref["rowptr"], ref["post"], ref["kind"], ref["w0"], ref["w1"] if pair else None,
+                                  ref["delay"], dt=0.1, noise_seed=4)
+        nb.set_launch(deliver_mode=mode, deliver_grid=200, stage_segs=segs, stage_ept=16, stage_variant=2)
+        ev, sp = np.zeros(90, np.uint64), np.zeros(90, np.uint32)
+        # silence, single spikes, light and heavy noise, silence again
+        for i, rate in enumerate((0.0, 2.0 / n, 0.003, 0.25, 0.02, 0.0)):
+            nb.run(15, noise_rate=rate, graph=i % 2 == 0, events=ev[15 * i:15 * i + 15], spikes=sp[15 * i:15 * i + 15])
+        outs.append((nb.get("V"), nb.get("J"), ev, sp))
+        nb.close()
+    assert outs[0][2].max() > 0
+    for o in outs[1:]:
+        for x, y in zip(outs[0], o):
+            assert np.array_equal(x, y)
+
+
 def test_large_block_full_size_event_identity():
     """The benchmark's single large block at full size (5e6 neurons, 5e9
     synapses, delays 1-10): with noise-only spikes during 4 steps and then
