@@ -144,9 +144,12 @@ class block:
         self._freq = np.zeros(self._nb.S, np.uint32)
         self._vmean = np.zeros(self._nb.S, np.float32)
 
-    # The persistent launch (deliver mode 2) takes blocks without sources whose
-    # sums fit its fixed point; steps with injected uniforms, and those soon
-    # after a weight change, run on the kernels the block was created with.
+    # The persistent launch takes blocks without sources; steps with injected
+    # uniforms, and those soon after a weight change, run on the kernels the
+    # block was created with.  It adds the FP32 weights as they are, in 64-bit
+    # sums (deliver mode 3): the fixed point of deliver mode 2 would round them
+    # to about 2^-30 of their channel's sum.
+    # _mode: 2 in the persistent launch, else the kernels' mode (0 or 1).
     def _choose_launch(self, hold=0):
         self._base_mode = self._mode = self._nb.get_launch()["deliver_mode"]
         self._persist = self.src is None and PERSIST_N[0] <= self.N <= PERSIST_N[1]
@@ -161,12 +164,12 @@ class block:
                 mode = 2
         if mode != self._mode:
             try:
-                self._nb.set_launch(deliver_mode=mode)
+                self._nb.set_launch(deliver_mode=3 if mode == 2 else mode)
                 self._mode = mode
             except nat.DTBError as e:
                 if e.code != nat.DTB_INVALID_PARAMETER:
                     raise
-                self._persist = False  # no fixed point for these weights
+                self._persist = False  # it does not hold this block, or not all of its weights' bits
 
     def _apply_sources(self, nb):
         k, t = np.nonzero(self._sched)

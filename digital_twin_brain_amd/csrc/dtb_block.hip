@@ -1364,7 +1364,7 @@ static void launch_accum_f(const Block* b, const StageArgs& sa)
 template <bool PAIR>
 static void launch_accum(const Block* b, const StageArgs& sa)
 {
-    if (b->accum_fixed) launch_accum_f<PAIR, true>(b, sa);
+    if (b->accum_fixed && b->deliver_mode != 3) launch_accum_f<PAIR, true>(b, sa);
     else launch_accum_f<PAIR, false>(b, sa);
 }
 
@@ -1513,6 +1513,28 @@ __global__ void weight_out_kernel(int64_t nnz, const uint32_t* __restrict__ col,
     }
 }
 
+// out = 1 if some scaled weight is no multiple of 2^-32
+template <bool PAIR>
+__global__ void inexact_kernel(int64_t nnz, const float* __restrict__ w, const float2* __restrict__ w2,
+                               uint32_t* __restrict__ out)
+{
+    bool bad = false;
+    auto whole = [](float v) {
+        const float x = v * 0x1p32f;
+        return rintf(x) == x;
+    };
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz; e += stride) {
+        if (PAIR) {
+            const float2 v = w2[e];
+            bad |= !whole(v.x) || !whole(v.y);
+        } else {
+            bad |= !whole(w[e]);
+        }
+    }
+    if (__any(bad) && __lane_id() == 0) atomicOr(out, 1u);
+}
+
 static inline unsigned grid_syn(int64_t nnz);
 static inline unsigned grid_for(int64_t n, int bs);
 
@@ -1608,7 +1630,7 @@ static int update_jexp(Block* b, bool with_state)
     DTB_TRY_HIP(e);
     if (!b->fixed_ok) b->accum_fixed = false;
     b->persist_dirty = true; // the grouped copy holds the rounded scaled weights
-    if (!b->fixed_ok && b->deliver_mode == 2) b->deliver_mode = 1;
+    if (!b->fixed_ok && b->deliver_mode >= 2) b->deliver_mode = 1;
     return DTB_OK;
 }
 
@@ -1759,7 +1781,7 @@ __global__ __launch_bounds__(1024) void deliver_accum_kernel(StageArgs s)
 }
 
 // ---------------------------------------------------------------------------
-// Persistent delivery (deliver_mode 2) for blocks small enough that every
+// Persistent delivery (deliver_mode 2 and 3) for blocks small enough that every
 // workgroup of one launch is resident: one launch runs all K steps of a
 // batch, so a step costs one grid barrier instead of two or three kernel
 // launches.  Workgroup p (p < G <= kSubLists) owns the neurons
@@ -1767,16 +1789,23 @@ __global__ __launch_bounds__(1024) void deliver_accum_kernel(StageArgs s)
 // same share: it updates them, writes their spikes into spike sub-list p
 // (per never exceeds a sub-list's capacity; its only writer, so in the standard list
 // format without reservation atomics), and after the barrier accumulates
-// every arrival for its own neurons into an int32 LDS slice.  The synapses
+// every arrival for its own neurons into an LDS slice.  The synapses
 // are a copy of the CSR grouped by owning workgroup: each workgroup's
 // synapses are contiguous, in (row, delay) segment order (one record per
-// synapse: slice index and kind, then the weights pre-rounded to the same
-// int32 fixed point as bucketed delivery, so one load fetches both), and so
-// are its segment bounds.  The records and bounds that the workgroups of one
+// synapse: slice index and kind, then the weights, so one load fetches both),
+// and so are its segment bounds.  The records and bounds that the workgroups of one
 // XCD read then share no cache line with other workgroups', and that XCD's
 // L2 holds only its own workgroups' share of the block (an eighth of it on
-// 32 workgroups over 8 XCDs, instead of most of its lines).  The results
-// equal bucketed delivery bit for bit.
+// 32 workgroups over 8 XCDs, instead of most of its lines).
+// Mode 2 adds weights pre-rounded to the int32 fixed point of bucketed
+// delivery, and the results equal bucketed delivery bit for bit.  Mode 3
+// (WIDE) adds FP32 weights in 64-bit fixed point, 32 bits below that of mode
+// 2, for blocks none of whose weights it rounds (fixed_exact): those of at
+// least 2^-38 of their channel's sum of |w|, whose last bit is then no
+// smaller than its step.  The sums are exact, where direct delivery (mode 0)
+// rounds each add to FP32.  (FP32 LDS adds instead: ds_add_f32 takes several
+// times as long as the integer ones, 20 steps of the 10,000-neuron drop-in
+// block 290 us against 249.)
 constexpr int kPersistMaxLds = 64 * 1024; // LDS slice bytes per workgroup
 constexpr uint32_t kBarrierSpinLimit = 1u << 22;
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima), gfx9 encoding
@@ -1789,7 +1818,7 @@ struct PersistArgs {
     NeuronArgs na;
     const int32_t* __restrict__ bptr;  // [G][n*D+1]: start of workgroup g's synapses of each (row, delay) segment
     // grouped synapses, one record each: compact (local index | kind << 31,
-    // round(scaled weight)) as 8 bytes, pair (index | kind, w0, w1, 0) as 16
+    // scaled weight) as 8 bytes, pair (index | kind, w0, w1, 0) as 16
     const uint32_t* __restrict__ pcw;
     int32_t G;                         // workgroups
     int32_t m;                         // blocks per workgroup (the LDS slice holds m*256 neurons)
@@ -1820,6 +1849,39 @@ __device__ __forceinline__ void persist_record(const uint32_t* __restrict__ pcw,
     }
 }
 
+// The arrivals of a workgroup's neurons: sums of int32, or of 2^-32 in 64 bits.
+template <bool WIDE>
+struct PersistSum {
+    typedef int32_t T;
+    static __device__ __forceinline__ T of(int w) { return w; }
+    static __device__ __forceinline__ void add(T* p, T v) { atomicAdd(p, v); }
+    static __device__ __forceinline__ float value(T s) { return (float)s; }
+};
+template <>
+struct PersistSum<true> {
+    typedef long long T;
+    // w 2^32, a whole number, from the bits of w (|w| <= 2^30); both parts of |w| are exact
+    static __device__ __forceinline__ T of(int w)
+    {
+        const float a = fabsf(__int_as_float(w)), hi = truncf(a);
+        const T m = (T)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)((a - hi) * 4294967296.0f));
+        return w < 0 ? -m : m;
+    }
+    static __device__ __forceinline__ void add(T* p, T v)
+    {
+        atomicAdd(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
+    }
+    static __device__ __forceinline__ float value(T s) { return (float)s * 0x1p-32f; }
+};
+
+// add one record's weight(s) at slice element o
+template <bool PAIR, bool WIDE>
+__device__ __forceinline__ void persist_add(typename PersistSum<WIDE>::T* s_acc, int32_t o, int2 v)
+{
+    PersistSum<WIDE>::add(&s_acc[o], PersistSum<WIDE>::of(v.x));
+    if (PAIR) PersistSum<WIDE>::add(&s_acc[o + 1], PersistSum<WIDE>::of(v.y));
+}
+
 __device__ inline int32_t ld_coherent(const int32_t* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1830,12 +1892,14 @@ __device__ inline int32_t ld_coherent(const int32_t* p)
 // pass), whose state (V, J, refractory end, flags) and constants stay in
 // registers for the whole batch; it is read before the first step and written
 // back after the last.  The per-step arithmetic is the neuron kernel's own.
-template <bool PAIR, bool PSET, int MB, bool RES>
+template <bool PAIR, bool PSET, int MB, bool RES, bool WIDE>
 __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
 {
     constexpr int C = PAIR ? 4 : 2;
     constexpr int NT = 256 * MB;
-    extern __shared__ int s_acc[]; // [m*256][C] arrivals of the workgroup's neurons, int32 fixed point
+    extern __shared__ long long s_dyn[];
+    typedef typename PersistSum<WIDE>::T Sum;
+    Sum* s_acc = reinterpret_cast<Sum*>(s_dyn); // [m*256][C] arrivals of the workgroup's neurons
     __shared__ uint32_t s_wcnt[4 * MB];
     __shared__ float s_tab[kMaxPsets * 16];
     __shared__ uint32_t cum[kMaxEntries + 1];
@@ -1851,6 +1915,7 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
     const int32_t G = P.G;
     const uint32_t lane = __lane_id();
     const uint32_t wid = threadIdx.x >> 6;
+    auto arrived = [&](int32_t o) { return PersistSum<WIDE>::value(s_acc[o]); };
     if (PSET)
         for (int x = threadIdx.x; x < a.npsets * 16; x += NT) s_tab[x] = a.ptab[x];
     for (int x = threadIdx.x; x < P.m * 256 * C; x += NT) s_acc[x] = 0;
@@ -1910,10 +1975,9 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
                             d = make_float4(d2.x, d2.x, d2.y, d2.y);
                         }
                     } else if (PAIR) {
-                        d = make_float4((float)s_acc[4 * li], (float)s_acc[4 * li + 1], (float)s_acc[4 * li + 2],
-                                        (float)s_acc[4 * li + 3]);
+                        d = make_float4(arrived(4 * li), arrived(4 * li + 1), arrived(4 * li + 2), arrived(4 * li + 3));
                     } else {
-                        const float e = (float)s_acc[2 * li], f = (float)s_acc[2 * li + 1];
+                        const float e = arrived(2 * li), f = arrived(2 * li + 1);
                         d = make_float4(e, e, f, f);
                     }
 #pragma unroll
@@ -1944,10 +2008,9 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
                         d = make_float4(d2.x, d2.x, d2.y, d2.y);
                     }
                 } else if (PAIR) {
-                    d = make_float4((float)s_acc[4 * li], (float)s_acc[4 * li + 1], (float)s_acc[4 * li + 2],
-                                    (float)s_acc[4 * li + 3]);
+                    d = make_float4(arrived(4 * li), arrived(4 * li + 1), arrived(4 * li + 2), arrived(4 * li + 3));
                 } else {
-                    const float e = (float)s_acc[2 * li], f = (float)s_acc[2 * li + 1];
+                    const float e = arrived(2 * li), f = arrived(2 * li + 1);
                     d = make_float4(e, e, f, f);
                 }
 #pragma unroll
@@ -2071,8 +2134,7 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
                     for (int u = 0; u < 8; ++u) {
                         if (x0 + u >= hi) continue;
                         const int32_t o = (int32_t)(cc[u] & 0x7fffffffu) * C + (int32_t)(cc[u] >> 31) * (C / 2);
-                        atomicAdd(&s_acc[o], vv[u].x);
-                        if (PAIR) atomicAdd(&s_acc[o + 1], vv[u].y);
+                        persist_add<PAIR, WIDE>(s_acc, o, vv[u]);
                     }
                 }
                 continue;
@@ -2111,8 +2173,7 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
                 for (int u = 0; u < U; ++u) {
                     if (pos[u] < 0) continue;
                     const int32_t o = (int32_t)(cc[u] & 0x7fffffffu) * C + (int32_t)(cc[u] >> 31) * (C / 2);
-                    atomicAdd(&s_acc[o], vv[u].x);
-                    if (PAIR) atomicAdd(&s_acc[o + 1], vv[u].y);
+                    persist_add<PAIR, WIDE>(s_acc, o, vv[u]);
                 }
             }
             __syncthreads();
@@ -2138,10 +2199,10 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
         const int64_t i = (int64_t)p * P.per + li;
         if (i >= a.n) continue;
         if (PAIR)
-            reinterpret_cast<float4*>(a.acc)[i] = make_float4((float)s_acc[4 * li], (float)s_acc[4 * li + 1],
-                                                              (float)s_acc[4 * li + 2], (float)s_acc[4 * li + 3]);
+            reinterpret_cast<float4*>(a.acc)[i] = make_float4(arrived(4 * li), arrived(4 * li + 1), arrived(4 * li + 2),
+                                                              arrived(4 * li + 3));
         else
-            reinterpret_cast<float2*>(a.acc)[i] = make_float2((float)s_acc[2 * li], (float)s_acc[2 * li + 1]);
+            reinterpret_cast<float2*>(a.acc)[i] = make_float2(arrived(2 * li), arrived(2 * li + 1));
     }
 }
 
@@ -3059,8 +3120,31 @@ static int create_from_csr(Block* b, const dtb_block_desc* d)
 }
 
 // ------------------------------------------------------------- the run loop
-static int ensure_persist(Block* b);
-static bool persist_fits(const Block* b, int32_t* G = nullptr, int32_t* m = nullptr, int32_t* per = nullptr);
+// Whether 64-bit fixed point holds every weight exactly.
+static int fixed_exact(Block* b, int32_t* exact)
+{
+    *exact = 0;
+    if (!b->fixed_ok) return DTB_OK;
+    if (!b->inexact) DTB_TRY(alloc_n(b, &b->inexact, 1));
+    uint32_t bad = 0;
+    DTB_TRY_HIP(hipMemsetAsync(b->inexact, 0, sizeof(uint32_t), b->stream));
+    if (b->nnz > 0) {
+        if (b->pair)
+            hipLaunchKernelGGL(inexact_kernel<true>, dim3(grid_syn(b->nnz)), dim3(256), 0, b->stream, b->nnz, b->w,
+                               b->w2, b->inexact);
+        else
+            hipLaunchKernelGGL(inexact_kernel<false>, dim3(grid_syn(b->nnz)), dim3(256), 0, b->stream, b->nnz, b->w,
+                               b->w2, b->inexact);
+        DTB_TRY_HIP(hipGetLastError());
+    }
+    DTB_TRY_HIP(hipMemcpyAsync(&bad, b->inexact, sizeof(bad), hipMemcpyDeviceToHost, b->stream));
+    DTB_TRY_HIP(hipStreamSynchronize(b->stream));
+    *exact = bad ? 0 : 1;
+    return DTB_OK;
+}
+
+static int ensure_persist(Block* b, bool wide);
+static bool persist_fits(const Block* b, bool wide, int32_t* G = nullptr, int32_t* m = nullptr, int32_t* per = nullptr);
 
 static SegArgs seg_args(const Block* b)
 {
@@ -3109,42 +3193,44 @@ struct Want {
 };
 
 
-template <bool PAIR, bool PSET>
+template <bool PAIR, bool PSET, bool WIDE>
 static void launch_persist_t(const Block* b, const PersistArgs& pa, int mb, size_t lds)
 {
     // every thread holds at most one neuron when the workgroup's blocks fit one pass
     const bool res = b->pm <= mb;
+    const dim3 g(b->pG), t(256 * mb);
     if (mb == 4) {
-        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 4, true>), dim3(b->pG), dim3(1024), lds, b->stream, pa);
-        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 4, false>), dim3(b->pG), dim3(1024), lds, b->stream, pa);
+        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 4, true, WIDE>), g, t, lds, b->stream, pa);
+        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 4, false, WIDE>), g, t, lds, b->stream, pa);
     } else if (mb == 2) {
-        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 2, true>), dim3(b->pG), dim3(512), lds, b->stream, pa);
-        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 2, false>), dim3(b->pG), dim3(512), lds, b->stream, pa);
+        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 2, true, WIDE>), g, t, lds, b->stream, pa);
+        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 2, false, WIDE>), g, t, lds, b->stream, pa);
     } else {
-        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 1, true>), dim3(b->pG), dim3(256), lds, b->stream, pa);
-        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 1, false>), dim3(b->pG), dim3(256), lds, b->stream, pa);
+        if (res) hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 1, true, WIDE>), g, t, lds, b->stream, pa);
+        else hipLaunchKernelGGL((persist_step_kernel<PAIR, PSET, 1, false, WIDE>), g, t, lds, b->stream, pa);
     }
 }
 
+template <bool WIDE>
 static void launch_persist(const Block* b, const PersistArgs& pa, int mb, size_t lds)
 {
     if (b->pair) {
-        if (b->npsets) launch_persist_t<true, true>(b, pa, mb, lds);
-        else launch_persist_t<true, false>(b, pa, mb, lds);
+        if (b->npsets) launch_persist_t<true, true, WIDE>(b, pa, mb, lds);
+        else launch_persist_t<true, false, WIDE>(b, pa, mb, lds);
     } else {
-        if (b->npsets) launch_persist_t<false, true>(b, pa, mb, lds);
-        else launch_persist_t<false, false>(b, pa, mb, lds);
+        if (b->npsets) launch_persist_t<false, true, WIDE>(b, pa, mb, lds);
+        else launch_persist_t<false, false, WIDE>(b, pa, mb, lds);
     }
 }
 
 // A batch runs as one persistent launch when the block is set to deliver_mode
-// 2 and the batch needs nothing that launch does not produce (injected
+// 2 or 3 and the batch needs nothing that launch does not produce (injected
 // uniforms, sources, the external drive, I_syn means, samples, per-kernel
-// times); otherwise it runs on the bucketed kernels, whose fixed-point sums
-// give the same results.
+// times); otherwise it runs on the bucketed kernels, with fixed-point sums in
+// mode 2 (the same results) and FP32 sums in mode 3 (the same up to their roundings).
 static bool persist_batch(const Block* b, const dtb_run_args* a, const Want& w)
 {
-    return b->deliver_mode == 2 && b->pcol && !b->persist_dirty && a->noise_mode != DTB_NOISE_UNIFORMS &&
+    return b->deliver_mode >= 2 && b->pcol && !b->persist_dirty && a->noise_mode != DTB_NOISE_UNIFORMS &&
            b->src_nts == 0 && !b->src && b->ext.n == 0 && !w.isum && !w.sample && !w.timing;
 }
 
@@ -3186,9 +3272,10 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
         pa.seg_loop = b->nnz <= 8 * b->n * (int64_t)b->D * b->pG ? 1 : 0;
         pa.pub = b->pbar;
         pa.rec_events = b->rec_events; pa.rec_nspk = b->rec_nspk;
-        const size_t lds = sizeof(int) * (size_t)b->pm * 256 * (b->pair ? 4 : 2);
+        const size_t lds = (b->pwide ? 8 : 4) * (size_t)b->pm * 256 * (b->pair ? 4 : 2);
         const int mb = b->pm >= 4 ? 4 : b->pm >= 2 ? 2 : 1;
-        launch_persist(b, pa, mb, lds);
+        if (b->pwide) launch_persist<true>(b, pa, mb, lds);
+        else launch_persist<false>(b, pa, mb, lds);
         if (w.bold)
             for (int32_t k = b->bold_sps - 1; k < K; k += b->bold_sps)
                 hipLaunchKernelGGL(bold_counts_kernel, dim3(grid_for(b->nvox, 256)), dim3(256), 0, b->stream, b->S,
@@ -3296,10 +3383,13 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
         return DTB_UNSET_SAMPLE_FAILURE;
     }
     DTB_TRY_HIP(hipSetDevice(b->device));
-    if (b->deliver_mode == 2 && b->persist_dirty) {
+    if (b->deliver_mode >= 2 && b->persist_dirty) {
         // weights or layout changed since the grouped copy was built
-        if (persist_fits(b)) DTB_TRY(ensure_persist(b));
-        else b->deliver_mode = 1;
+        const bool wide = b->deliver_mode == 3;
+        int32_t exact = 1;
+        if (wide) DTB_TRY(fixed_exact(b, &exact));
+        if (exact && persist_fits(b, wide)) DTB_TRY(ensure_persist(b, wide));
+        else b->deliver_mode = wide ? 0 : 1;
     }
     // segment lists: written only by bucketed batches; restarted after any
     // batch that did not write them (or a state load)
@@ -3909,7 +3999,7 @@ namespace dtb {
 // Persistent delivery fits when at most kSubLists workgroups of 256 threads
 // cover the neurons with an LDS slice of at most kPersistMaxLds bytes, the
 // synapse positions fit int32 and the fixed-point sums cannot overflow.
-static bool persist_fits(const Block* b, int32_t* G, int32_t* m, int32_t* per)
+static bool persist_fits(const Block* b, bool wide, int32_t* G, int32_t* m, int32_t* per)
 {
     // G workgroups own consecutive, equal ranges of ceil(n / G) neurons (at most
     // a sub-list's capacity), each held in an LDS slice of m 256-neuron blocks
@@ -3917,7 +4007,7 @@ static bool persist_fits(const Block* b, int32_t* G, int32_t* m, int32_t* per)
     const int64_t g = std::min<int64_t>(kSubLists, nblk);
     const int64_t pp = g > 0 ? (b->n + g - 1) / g : 0;
     const int64_t mm = (pp + 255) / 256;
-    const int64_t lds = mm * 256 * (b->pair ? 4 : 2) * 4;
+    const int64_t lds = mm * 256 * (b->pair ? 4 : 2) * (wide ? 8 : 4);
     if (G) *G = (int32_t)g;
     if (m) *m = (int32_t)mm;
     if (per) *per = (int32_t)pp;
@@ -3929,15 +4019,20 @@ static bool persist_fits(const Block* b, int32_t* G, int32_t* m, int32_t* per)
 // each owning workgroup (post / per) back to back, workgroup after
 // workgroup, in (row, delay) segment order inside each, each stored as its
 // index in that workgroup's LDS slice (post - owner * per) with the kind bit,
-// and its weight rounded to the int32 the bucketed accumulation adds
-// (__float2int_rn of the scaled weight).
-static int ensure_persist(Block* b)
+// and its scaled weight: rounded to the int32 the bucketed accumulation adds
+// or as it is (wide).
+static int ensure_persist(Block* b, bool wide)
 {
-    if (!b->persist_dirty && b->pcol) return DTB_OK;
+    if (!b->persist_dirty && b->pcol && b->pwide == wide) return DTB_OK;
     int32_t G = 0, m = 0, per = 0;
-    DTB_REQUIRE(persist_fits(b, &G, &m, &per),
+    DTB_REQUIRE(persist_fits(b, wide, &G, &m, &per),
                 "persistent delivery needs at most %d x 256 x %d neurons, fixed-point sums and fewer than 2^31 "
-                "synapses", kSubLists, kPersistMaxLds / (256 * 4 * (b->pair ? 4 : 2)), kSubLists);
+                "synapses", kSubLists, kPersistMaxLds / (256 * (wide ? 8 : 4) * (b->pair ? 4 : 2)));
+    if (wide) {
+        int32_t exact = 0;
+        DTB_TRY(fixed_exact(b, &exact));
+        DTB_REQUIRE(exact, "64-bit fixed point would round some weights (less than 2^-38 of their channel's sum)");
+    }
     DTB_TRY_HIP(hipSetDevice(b->device));
     DTB_TRY_HIP(hipStreamSynchronize(b->stream));
     const int64_t n = b->n, nnz = b->nnz, D = b->D;
@@ -3953,7 +4048,7 @@ static int ensure_persist(Block* b)
     DTB_REQUIRE(rp[(size_t)n] == nnz, "the CSR row pointer does not end at nnz");
     GroupedCsr gc;
     const std::string err = group_by_owner(n, D, G, per, b->pk.idx_bits, b->pk.dmask, b->pk.idx_mask, b->pair,
-                                           rp.data(), col.data(), w.data(), gc);
+                                           rp.data(), col.data(), w.data(), gc, wide);
     DTB_REQUIRE(err.empty(), "persistent delivery: %s", err.c_str());
     const std::vector<int32_t>& bptr = gc.bptr;
     const std::vector<uint32_t>& rec = gc.rec;
@@ -3976,6 +4071,7 @@ static int ensure_persist(Block* b)
     b->pG = G;
     b->pm = m;
     b->pper = per;
+    b->pwide = wide;
     b->persist_dirty = false;
     for (auto& kv : b->graphs) hipGraphExecDestroy(kv.second);
     b->graphs.clear();
@@ -4602,13 +4698,11 @@ int dtb_block_set_launch(dtb_block* b, int32_t what, int32_t value)
         b->seg_cap = value == 0 ? 0 : value == 1 ? b->seg_alloc : std::min<int64_t>(value, b->seg_alloc);
         b->seg_dirty = true;
     } else if (what == DTB_LAUNCH_DELIVER_MODE) {
-        DTB_REQUIRE(value >= 0 && value <= 2,
-                    "delivery mode must be 0 (atomics), 1 (bucketed) or 2 (persistent, small blocks)");
+        DTB_REQUIRE(value >= 0 && value <= 3,
+                    "delivery mode must be 0 (atomics), 1 (bucketed), 2 or 3 (persistent, small blocks)");
         if (value >= 1) DTB_TRY(ensure_bucketed(b));
-        if (value == 2) {
-            DTB_TRY(ensure_persist(b));
-            b->accum_fixed = true; // batches that fall back to bucketed kernels sum as the persistent launch does
-        }
+        if (value >= 2) DTB_TRY(ensure_persist(b, value == 3));
+        if (value == 2) b->accum_fixed = true; // batches that fall back to bucketed kernels sum as the persistent launch does
         b->deliver_mode = value;
     } else {
         set_error("unknown launch parameter %d", what);

@@ -114,7 +114,7 @@ struct Block {
     double t_host = 0.0;
     int32_t deliver_grid = 64;  // workgroups of the delivery kernel
     int32_t deliver_lanes = 64; // lanes per (row, delay) segment
-    int32_t deliver_mode = 0;   // 0: global atomics, 1: bucketed (staged + LDS accumulation)
+    int32_t deliver_mode = 0;   // 0: global atomics, 1: bucketed (staged + LDS accumulation), 2, 3: persistent
     int32_t stage_segs = 256;   // bucketed: (row, delay) segments per staging chunk
     int32_t stage_ept = 32;     // bucketed: events per lane per staging round
     int32_t stage_variant = 0;  // bucketed: 0 scattered stores, 1 two passes per chunk, 2 LDS-sorted rounds
@@ -152,11 +152,13 @@ struct Block {
     int64_t seg_cap = 0;          // entries used per list (0: segment lists off)
     bool seg_dirty = true;        // the lists must be restarted before the next bucketed batch
 
-    // persistent delivery (deliver_mode 2): the CSR grouped by owning
+    // persistent delivery (deliver_mode 2 and 3): the CSR grouped by owning
     // workgroup (each workgroup's synapses contiguous, in (row, delay) segment
     // order), rebuilt when the weights change
     int32_t* pbptr = nullptr;   // [pG][n*D+1] start of workgroup g's synapses of each segment
-    uint32_t* pcol = nullptr;   // [nnz] records: local index | kind << 31, round(scaled weight) (x2 pair, + pad)
+    uint32_t* pcol = nullptr;   // [nnz] records: local index | kind << 31, scaled weight (x2 pair, + pad)
+    bool pwide = false;         // the weights in pcol are FP32 (mode 3), else rounded to int32 (mode 2)
+    uint32_t* inexact = nullptr; // flag of fixed_exact
     void* pin = nullptr;        // pinned host buffer for small records (kPinBytes)
     uint32_t* pbar = nullptr;   // [0] barrier counter, [64] abort flag
     int32_t pG = 0, pm = 0;     // workgroups, 256-neuron blocks of LDS slice per workgroup

@@ -11,12 +11,14 @@
 // so workgroup g reads segment q's records [bptr[g][q], bptr[g][q + 1]).
 // A record is R = 2 words (compact weights) or 4 (pair weights):
 //   word 0: post - g * per (the index in the workgroup's LDS slice) | kind << 31,
-//   word 1 (and 2): the weight(s) rounded to the nearest int32, ties to even.
+//   word 1 (and 2): the weight(s), rounded to the nearest int32, ties to even,
+//   or with `given` the bits of the float32 as they are.
 #pragma once
 
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -33,7 +35,7 @@ struct GroupedCsr {
 // is wrong with the input.
 inline std::string group_by_owner(int64_t n, int64_t D, int32_t G, int64_t per, uint32_t idx_bits, uint32_t dmask,
                                   uint32_t idx_mask, bool pair, const int64_t* rp, const uint32_t* col,
-                                  const float* w, GroupedCsr& out)
+                                  const float* w, GroupedCsr& out, bool given = false)
 {
     char msg[160];
     if (n <= 0 || D <= 0 || G <= 0 || per <= 0 || (int64_t)G * per < n) return "bad sizes";
@@ -89,8 +91,11 @@ inline std::string group_by_owner(int64_t n, int64_t D, int32_t G, int64_t per, 
             const int64_t g = post / per;
             const int32_t to = pos[(size_t)g]++;
             out.rec[(size_t)to * R] = (uint32_t)(post - g * per) | (c & 0x80000000u);
-            for (int y = 0; y < W; ++y)
-                out.rec[(size_t)to * R + 1 + y] = (uint32_t)(int32_t)std::nearbyint(w[x * W + y]);
+            for (int y = 0; y < W; ++y) {
+                uint32_t& r = out.rec[(size_t)to * R + 1 + y];
+                if (given) std::memcpy(&r, &w[x * W + y], sizeof(r));
+                else r = (uint32_t)(int32_t)std::nearbyint(w[x * W + y]);
+            }
         }
     }
     return std::string();

@@ -304,7 +304,9 @@ int dtb_block_set_external(dtb_block* b, int32_t n_thresholds, const uint32_t* t
                                       blocks: one launch per step batch with a grid barrier per step, at most
                                       32 workgroups; fixed-point sums, results equal to mode 1; batches that
                                       need injected uniforms, sources, the external drive, I_syn means, samples
-                                      or kernel times run on the mode-1 kernels) */
+                                      or kernel times run on the mode-1 kernels), 3: as 2 with 64-bit sums of the
+                                      FP32 weights as they are, exact where mode 0 rounds each add (refused if
+                                      some weight is not a multiple of 2^-62 of its channel's sum of |w|) */
 #define DTB_LAUNCH_NEURON_PSETS 3  /* set: 0 per-neuron constants, 1 shared parameter sets when <= 64
                                       distinct; get: number of sets in use (0 = per-neuron) */
 #define DTB_LAUNCH_STAGE_SEGS 4    /* bucketed delivery: at most 64, 128 or 256 (row, delay) segments per chunk (the

@@ -448,3 +448,49 @@ def test_dropin_persistent_launch_equals_per_step_kernels(n, npop):
     both(lambda x: x.run_steps(3, noise_rate=2.0 ** -6))
     assert np.array_equal(a.V_i.numpy(), b.V_i.numpy())
     assert np.array_equal(a.J_ui.numpy(), b.J_ui.numpy())
+
+
+# weights over several decades, which a fixed point of 30 bits does not hold: J in the
+# persistent launch (or out of it, where not even its 62 bits hold them) against the FP64
+# oracle.
+# J is a sum of positive terms; each step rounds it three times (the addition, the decay,
+# the decay constant) and once more for each of at most a channel's `most` arrivals, so
+# that k steps are within (3 + most) k 2^-24 relative.
+@pytest.mark.parametrize("n,decades,mode", [(2000, 6, 2), (5000, 5, 2), (2000, 14, 0)])
+def test_dropin_keeps_weights_of_several_decades(n, decades, mode):
+    from digital_twin_brain_amd import block as block_class
+
+    rng = np.random.default_rng(n)
+    csr = orc.gen_fixed_indegree(n, n * 4 // 5, 40, 1, 0.0, 1.0, False, seed=n)
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    _, first = np.unique(pre * n + csr["post"], return_index=True)
+    keep = np.zeros(pre.shape[0], bool)
+    keep[first] = True
+    csr = _keep_synapses(n, csr, keep)
+    csr["w0"] = (10.0 ** rng.uniform(-decades + 1, 1, csr["post"].shape[0])).astype(np.float32)
+    csr["w1"] = csr["w0"].copy()
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    p = _lif_props(n, rng, g_scale=1.5)
+    idx = torch.from_numpy(np.stack([csr["kind"].astype(np.int64) * 2, csr["post"], pre]))
+    idx = torch.cat([idx, idx + torch.tensor([[1], [0], [0]])], dim=1)
+    W = torch.sparse_coo_tensor(idx, torch.from_numpy(np.concatenate([csr["w0"], csr["w1"]])), (4, n, n))
+    b = block_class(torch.from_numpy(p), W, delta_t=0.1, seed=5)
+    o = orc.OracleBlock(p, csr, 0.1)
+    # silent steps (a program's worth), then noise spikes alone: what arrives does not depend on V
+    b.run_steps(3000, noise_rate=0.0, isolated=True)
+    for _ in range(3000):
+        o.run(noise_rate=0.0, isolated=True, seed=5)
+    assert not b.J_ui.numpy().any()
+    most = int(np.bincount(csr["post"] * 2 + csr["kind"]).max())
+    for k in range(1, 13):
+        if k % 4:
+            b.run(noise_rate=2.0 ** -6, isolated=True)
+        else:
+            b.run_steps(1, noise_rate=2.0 ** -6, isolated=True)
+            assert b._mode == mode
+        o.run(noise_rate=2.0 ** -6, isolated=True, seed=5)
+        J, Jo = b.J_ui.numpy(), o.get("J")
+        assert np.array_equal(J > 0, Jo > 0)
+        np.testing.assert_allclose(J, Jo, rtol=(3 + most) * k * 2.0 ** -24, atol=0)
+    assert (Jo > 0).sum() > n
+
