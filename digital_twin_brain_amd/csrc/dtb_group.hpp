@@ -1,11 +1,15 @@
-// Host-side grouping of a block's CSR for persistent delivery.  Plain C++
-// (no HIP), so it also builds with g++ alone.
+// Layout of a block's CSR grouped for persistent delivery.  group_slot,
+// group_target and group_weight say where a synapse goes and what its record
+// holds; the device builds the copy with them, and group_by_owner lays it out
+// on the host, the plain form that the CPU suite checks.  No HIP calls, so it
+// also builds with g++ alone.
 //
 // The CSR rows are sorted by delay: segment q = j * D + d - 1 of row j and
 // delay d is the run of row j whose delay field is d - 1.  Workgroup g of
 // the persistent launch owns the neurons [g * per, (g + 1) * per).  The
 // grouped copy stores every workgroup's synapses back to back, workgroup
-// after workgroup, in segment order inside each (stable within a segment):
+// after workgroup, in segment order inside each (group_by_owner: in CSR order
+// within a segment; the device: in any order, the sums being of integers):
 //   bptr[g * (n * D + 1) + q]  first record of workgroup g's part of segment q,
 //   bptr[g * (n * D + 1) + n * D] = bptr[(g + 1) * (n * D + 1)]  (the end of g's run),
 // so workgroup g reads segment q's records [bptr[g][q], bptr[g][q + 1]).
@@ -22,7 +26,40 @@
 #include <string>
 #include <vector>
 
+#ifdef __HIPCC__
+#define DTB_GROUP_FN __host__ __device__ inline
+#else
+#define DTB_GROUP_FN inline
+#endif
+
 namespace dtb {
+
+struct GroupShape {
+    int64_t n, D, per;
+    uint32_t idx_bits, dmask, idx_mask;
+};
+
+// element of bptr of a synapse of row j with packed target c: its owner's part of segment (j, delay)
+DTB_GROUP_FN int64_t group_slot(const GroupShape& s, int64_t j, uint32_t c)
+{
+    const int64_t owner = (int64_t)(c & s.idx_mask) / s.per;
+    return owner * (s.n * s.D + 1) + j * s.D + (int64_t)(((c & 0x7fffffffu) >> s.idx_bits) & s.dmask);
+}
+
+// word 0 of its record
+DTB_GROUP_FN uint32_t group_target(const GroupShape& s, uint32_t c)
+{
+    return (uint32_t)((int64_t)(c & s.idx_mask) % s.per) | (c & 0x80000000u);
+}
+
+// word 1 (and 2)
+DTB_GROUP_FN uint32_t group_weight(float w, bool given)
+{
+    if (!given) return (uint32_t)(int32_t)rintf(w);
+    uint32_t r;
+    memcpy(&r, &w, sizeof(r));
+    return r;
+}
 
 struct GroupedCsr {
     std::vector<int32_t> bptr; // [G][n * D + 1]
@@ -42,6 +79,7 @@ inline std::string group_by_owner(int64_t n, int64_t D, int32_t G, int64_t per, 
     const int64_t nnz = rp[n];
     if (nnz < 0 || nnz >= (1ll << 31)) return "nnz out of range";
     const int64_t NS = n * D;
+    const GroupShape s{n, D, per, idx_bits, dmask, idx_mask};
     std::vector<int64_t> sb((size_t)NS + 1); // CSR start of every segment
     for (int64_t j = 0; j < n; ++j) {
         int64_t e = rp[j];
@@ -69,7 +107,7 @@ inline std::string group_by_owner(int64_t n, int64_t D, int32_t G, int64_t per, 
     }
     for (int64_t q = 0; q < NS; ++q)
         for (int64_t x = sb[(size_t)q]; x < sb[(size_t)q + 1]; ++x)
-            ++bptr[(size_t)((int64_t)(col[x] & idx_mask) / per) * BS + (size_t)q + 1];
+            ++bptr[(size_t)group_slot(s, q / D, col[x]) + 1];
     int64_t run = 0;
     for (int32_t g = 0; g < G; ++g) {
         int32_t* bp = &bptr[(size_t)g * BS];
@@ -87,15 +125,10 @@ inline std::string group_by_owner(int64_t n, int64_t D, int32_t G, int64_t per, 
         for (int32_t g = 0; g < G; ++g) pos[(size_t)g] = bptr[(size_t)g * BS + (size_t)q];
         for (int64_t x = sb[(size_t)q]; x < sb[(size_t)q + 1]; ++x) {
             const uint32_t c = col[x];
-            const int64_t post = (int64_t)(c & idx_mask);
-            const int64_t g = post / per;
+            const int64_t g = (int64_t)(c & idx_mask) / per;
             const int32_t to = pos[(size_t)g]++;
-            out.rec[(size_t)to * R] = (uint32_t)(post - g * per) | (c & 0x80000000u);
-            for (int y = 0; y < W; ++y) {
-                uint32_t& r = out.rec[(size_t)to * R + 1 + y];
-                if (given) std::memcpy(&r, &w[x * W + y], sizeof(r));
-                else r = (uint32_t)(int32_t)std::nearbyint(w[x * W + y]);
-            }
+            out.rec[(size_t)to * R] = group_target(s, c);
+            for (int y = 0; y < W; ++y) out.rec[(size_t)to * R + 1 + y] = group_weight(w[x * W + y], given);
         }
     }
     return std::string();

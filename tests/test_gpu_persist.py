@@ -7,6 +7,8 @@ within 1e-5) -- across batch sizes, graph
 replay, delays, pair weights and switches between the modes mid-run.
 Parity with the FP64 oracle then carries over from the bucketed path's
 tests; the plain-block test runs the oracle comparison in this mode too."""
+import time
+
 import numpy as np
 import pytest
 
@@ -150,4 +152,21 @@ def test_persistent_refuses_blocks_it_cannot_hold():
     with pytest.raises(nat.DTBError):
         nb.set_launch(deliver_mode=2)
     assert nb.get_launch()["deliver_mode"] != 2
+    nb.close()
+
+
+def test_grouped_copy_costs_no_host_work_per_synapse():
+    """The switch to persistent delivery must not walk the synapses on the
+    host: 16 M of them cost a host thread about 20 ns each (0.3 s), a few
+    kernels and allocations some milliseconds."""
+    from digital_twin_brain_amd import NativeBlock
+
+    n, K = 16_000, 1000
+    nb = NativeBlock.fixed_indegree(_props(n, 12_800, np.random.default_rng(4)), 12_800, K, conn_seed=2, noise_seed=3)
+    nb.run(1, noise_mode=1)
+    for mode in (2, 3):
+        nb.set_launch(deliver_mode=0)
+        t0 = time.process_time()
+        nb.set_launch(deliver_mode=mode)
+        assert time.process_time() - t0 < 0.1
     nb.close()
