@@ -170,3 +170,37 @@ def test_grouped_copy_costs_no_host_work_per_synapse():
         nb.set_launch(deliver_mode=mode)
         assert time.process_time() - t0 < 0.1
     nb.close()
+
+
+# weights of whole 1/256, which every way of adding sums exactly: the bucketed kernels, the
+# persistent launch on int32 and the one on 64-bit sums agree bit for bit, for one to four
+# 256-neuron blocks a workgroup (8,192 neurons each; three do not fit one pass), delays,
+# and both record sizes
+@pytest.mark.parametrize("n,K,D,pair", [(300, 40, 1, True), (8_192, 30, 1, True), (8_193, 30, 1, True),
+                                        (9_000, 30, 4, False), (20_000, 20, 1, True), (24_577, 20, 2, True),
+                                        (32_768, 20, 1, True), (32_768, 20, 1, False), (2_000, 400, 1, True)])
+def test_persistent_sums_agree_on_dyadic_weights(n, K, D, pair):
+    from digital_twin_brain_amd import NativeBlock
+
+    ne = n * 4 // 5
+    csr = orc.gen_fixed_indegree(n, ne, K, D, 0.0, 1.0, pair, seed=n + D)
+    w = [None if csr[k] is None else (np.floor(csr[k] * 256) / 256).astype(np.float32) for k in ("w0", "w1")]
+    props = _props(n, ne, np.random.default_rng(n))
+    blocks = []
+    for mode in (1, 2, 3):
+        nb = NativeBlock.from_csr(props, csr["rowptr"], csr["post"], csr["kind"], w[0], w[1], delay=csr["delay"],
+                                  dt=0.1, noise_seed=7)
+        nb.set_launch(deliver_mode=1, accum_fixed=1)
+        nb.set_launch(deliver_mode=mode)
+        assert nb.get_launch()["deliver_mode"] == mode
+        blocks.append(nb)
+    tot = 0
+    for steps, graph in ((1, False), (30, True), (7, False)):
+        for nb in blocks[1:]:
+            snap = blocks[0].save_state()
+            tot += int(_run_both(blocks[0], nb, steps, graph=graph)["events"].sum())
+            if nb is not blocks[-1]:
+                blocks[0].load_state(snap)
+    assert tot > 0
+    for nb in blocks:
+        nb.close()
