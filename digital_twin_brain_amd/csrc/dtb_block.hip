@@ -1813,7 +1813,39 @@ constexpr uint32_t kBarrierSpinLimit = 1u << 22;
 constexpr unsigned kWaitVmcnt0 = 0x0F70;
 constexpr int kPubStride = 16;                 // words between publication words (one 64-byte line each)
 constexpr int kPubAbort = kSubLists * kPubStride; // word index of the abort flag
+constexpr int kPubArrive = kPubAbort + 32;        // word index of the arrivals (on a line of its own)
 constexpr int kPubWords = kPubAbort + 64;
+constexpr uint32_t kGone = 1u << 31;              // in the arrivals: a workgroup gave up waiting, nobody runs
+
+// Whether all G workgroups of the launch are on the device, by one lane of
+// each after persist_arrive: the barriers of the steps need them all at once.
+// Either all of them get true or all get false, before any has written
+// anything, so that a batch for which a busy device has no room can run on
+// the per-step kernels instead.  A workgroup gives up only by setting kGone
+// while the count is short of G; once it is G, all will see it.
+__device__ inline void persist_arrive(uint32_t* pub, uint32_t wait)
+{
+    if (wait > 0) __hip_atomic_fetch_add(pub + kPubArrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else __hip_atomic_fetch_or(pub + kPubArrive, kGone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ inline bool persist_all_here(uint32_t* pub, uint32_t G, uint32_t wait)
+{
+    uint32_t* w = pub + kPubArrive;
+    uint32_t v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t spins = 0;;) {
+        if (v & kGone) return false;
+        if (v >= G) return true;
+        if (spins < wait) {
+            ++spins;
+            __builtin_amdgcn_s_sleep(1);
+            v = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else if (__hip_atomic_compare_exchange_strong(w, &v, v | kGone, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_AGENT)) {
+            return false;
+        } // else v is the count now: it can only have grown
+    }
+}
 
 struct PersistArgs {
     NeuronArgs na;
@@ -1826,7 +1858,9 @@ struct PersistArgs {
     int32_t per;                       // neurons per workgroup: workgroup p owns [p * per, (p + 1) * per)
     int32_t K;                         // steps of the batch
     int32_t seg_loop;                  // 1: each thread walks its own (short) segment; 0: scan-balanced chunks
-    uint32_t* pub;                     // [kSubLists] 64-bit words (step << 32 | spikes), kPubStride apart; abort flag
+    uint32_t wait;                     // looks for the workgroups to be on the device
+    uint32_t* pub;                     // [kSubLists] 64-bit words (step << 32 | spikes), kPubStride apart; abort
+                                       // flag; arrivals
     uint64_t* __restrict__ rec_events;
     uint32_t* __restrict__ rec_nspk;
 };
@@ -1917,12 +1951,12 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
     const uint32_t lane = __lane_id();
     const uint32_t wid = threadIdx.x >> 6;
     auto arrived = [&](int32_t o) { return PersistSum<WIDE>::value(s_acc[o]); };
+    if (threadIdx.x == 0) persist_arrive(P.pub, P.wait); // looked at once the state is loaded
     if (PSET)
         for (int x = threadIdx.x; x < a.npsets * 16; x += NT) s_tab[x] = a.ptab[x];
     for (int x = threadIdx.x; x < P.m * 256 * C; x += NT) s_acc[x] = 0;
     // counts of the earlier steps' lists (written before this launch)
     for (int x = threadIdx.x; x < a.L * kSubLists; x += NT) s_cnt[x] = a.spk_cnt[(int64_t)x * kCntStride];
-    if (threadIdx.x == 0) s_ok = 1;
     __syncthreads();
     const int32_t E = a.D * kSubLists;
     // register-resident neuron (RES): block sb = threadIdx / 256 of this workgroup
@@ -1952,6 +1986,9 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
             rgL = a.gL[ri]; rvL = a.vL[ri]; rdtC = a.dtC[ri]; rvth = a.vth[ri]; rvrst = a.vrst[ri]; riext = a.iext[ri];
         }
     }
+    if (threadIdx.x == 0) s_ok = persist_all_here(P.pub, (uint32_t)G, P.wait) ? 1 : 0;
+    __syncthreads();
+    if (!s_ok) return;
     for (int32_t k = 0; k < P.K; ++k) {
         const int64_t step = a.ctl->nbase + k + 1;
         const double t = a.ttab[k];
@@ -2214,22 +2251,34 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
 // wants in host memory are stored straight into the block's pinned buffer: a
 // one-step call otherwise pays a copy each through pageable memory and a
 // blocking read of the abort word, more than its kernels (72 -> 51 us a call
-// on the 10,000-neuron block).
+// on the 10,000-neuron block).  A persistent batch that its launch did not
+// run (kGone) leaves the step counter and the time as they were before it.
 struct HostRecords { // in the pinned buffer (NULL: not wanted)
-    uint32_t* abort;
+    uint32_t* abort;  // of a persistent batch: 1 gave up in a step, kGone did not begin
     uint32_t* freq;   // [K][S]
     float* vmean;     // [K][S]
     uint64_t* events; // [K]
     uint32_t* nspk;   // [K]
 };
-__global__ void finish_kernel(const StepCtl* __restrict__ ctl, int32_t L, uint32_t* spk_cnt, int32_t K, int32_t S,
+__global__ void finish_kernel(StepCtl* ctl, int32_t L, uint32_t* spk_cnt, int32_t K, int32_t S,
                               const uint32_t* __restrict__ rec_freq, const double* __restrict__ rec_vsum,
                               const float* __restrict__ inv, float* __restrict__ rec_vmean,
                               const uint64_t* __restrict__ rec_events, const uint32_t* __restrict__ rec_nspk,
-                              const uint32_t* __restrict__ abort, HostRecords h)
+                              const uint32_t* __restrict__ pub, HostRecords h)
 {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    if (h.abort) { // persistent
+        const uint32_t gone = pub[kPubArrive] & kGone;
+        if (tid == 0) *h.abort = gone ? gone : pub[kPubAbort];
+        if (gone) {
+            if (tid == 0) {
+                ctl->nsteps = ctl->nbase;
+                ctl->t = ctl->tbase;
+            }
+            return;
+        }
+    }
     if (spk_cnt && tid < kSubLists) {
         const int64_t next = ctl->nsteps + 1;
         spk_cnt[((int64_t)(next % L) * kSubLists + tid) * kCntStride] = 0;
@@ -2246,7 +2295,6 @@ __global__ void finish_kernel(const StepCtl* __restrict__ ctl, int32_t L, uint32
         if (h.events) h.events[x] = rec_events[x];
         if (h.nspk) h.nspk[x] = rec_nspk[x];
     }
-    if (tid == 0 && h.abort) *h.abort = *abort;
 }
 
 // Forced spikes of batch step k: the sources listed for the step's 0-based
@@ -2276,10 +2324,13 @@ __global__ void prologue_kernel(StepCtl* ctl, double* ttab, int32_t K, double dt
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     if (tid == 0) {
-        if (bar)
+        if (bar) {
             for (int q = 0; q < kSubLists; ++q) *reinterpret_cast<uint64_t*>(bar + kPubStride * q) = 0ull;
+            bar[kPubArrive] = 0u;
+        }
         const int64_t n0 = ctl->nsteps;
         double t = ctl->t;
+        ctl->tbase = t;
         for (int32_t k = 0; k < K; ++k) {
             t += dt;
             ttab[k] = t;
@@ -2353,10 +2404,12 @@ __global__ void sample_kernel(int64_t ns, const uint32_t* __restrict__ idx, cons
 __global__ void bold_counts_kernel(int32_t S, int32_t V, int32_t k, int32_t sps, const uint32_t* __restrict__ rec_freq,
                                    const int32_t* __restrict__ vptr, const int32_t* __restrict__ vpops,
                                    const double* __restrict__ size, const double* __restrict__ par,
-                                   double* __restrict__ st, double* __restrict__ rec_bold)
+                                   double* __restrict__ st, double* __restrict__ rec_bold,
+                                   const uint32_t* __restrict__ pub)
 {
     const int32_t v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
+    if (pub && (pub[kPubArrive] & kGone)) return; // a persistent batch that did not run
     uint64_t c = 0;
     for (int32_t x = vptr[v]; x < vptr[v + 1]; ++x) {
         const int32_t p = vpops[x];
@@ -3243,11 +3296,11 @@ static void launch_finish(const Block* b, int32_t K, const Want& w, bool persist
     hipLaunchKernelGGL(finish_kernel, dim3(grid_for(std::min<int64_t>(std::max<int64_t>(nrec, K), 1 << 20), 256)),
                        dim3(256), 0, b->stream, b->ctl, b->D + 1, persist ? b->spk_cnt : nullptr, K,
                        nrec ? b->S : 0, b->rec_freq, w.vsum ? b->rec_vsum : nullptr, b->pop_inv, b->rec_vmean, b->rec_events,
-                       b->rec_nspk, b->pbar ? b->pbar + kPubAbort : nullptr, h);
+                       b->rec_nspk, b->pbar, h);
 }
 
 static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float* uniforms, Want w,
-                         const HostRecords& hr)
+                         const HostRecords& hr, bool persist)
 {
     if (w.timing && (int64_t)b->events.size() < 3ll * K) {
         for (size_t e = b->events.size(); e < (size_t)(3 * K); ++e) {
@@ -3264,7 +3317,7 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
     const NeuronArgs na = neuron_args(b, a, uniforms, w.freq, w.vsum);
     const DeliverArgs da = deliver_args(b);
     const unsigned ng = grid_for(b->n, 256) + (na.pcum ? 1 : 0); // one more for the earlier entries
-    if (persist_batch(b, a, w)) {
+    if (persist) {
         PersistArgs pa;
         pa.na = na;
         pa.bptr = b->pbptr; pa.pcw = b->pcol;
@@ -3272,6 +3325,7 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
         // a thread per (row, delay, workgroup) segment when they average at most 8 synapses
         pa.seg_loop = b->nnz <= 8 * b->n * (int64_t)b->D * b->pG ? 1 : 0;
         pa.pub = b->pbar;
+        pa.wait = (uint32_t)b->persist_wait;
         pa.rec_events = b->rec_events; pa.rec_nspk = b->rec_nspk;
         const size_t lds = (b->pwide ? 8 : 4) * (size_t)b->pm * 256 * (b->pair ? 4 : 2);
         const int mb = b->pm >= 4 ? 4 : b->pm >= 2 ? 2 : 1;
@@ -3281,7 +3335,7 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
             for (int32_t k = b->bold_sps - 1; k < K; k += b->bold_sps)
                 hipLaunchKernelGGL(bold_counts_kernel, dim3(grid_for(b->nvox, 256)), dim3(256), 0, b->stream, b->S,
                                    b->nvox, k, b->bold_sps, b->rec_freq, b->vox_ptr, b->vox_pops, b->vox_size,
-                                   b->bold_state + 6 * (int64_t)b->nvox, b->bold_state, b->rec_bold);
+                                   b->bold_state + 6 * (int64_t)b->nvox, b->bold_state, b->rec_bold, b->pbar);
         launch_finish(b, K, w, true, hr);
         DTB_TRY_HIP(hipGetLastError());
         return DTB_OK;
@@ -3336,7 +3390,7 @@ static int enqueue_batch(Block* b, int32_t K, const dtb_run_args* a, const float
         if (w.bold && (k + 1) % b->bold_sps == 0)
             hipLaunchKernelGGL(bold_counts_kernel, dim3(grid_for(b->nvox, 256)), dim3(256), 0, b->stream, b->S,
                                b->nvox, k, b->bold_sps, b->rec_freq, b->vox_ptr, b->vox_pops, b->vox_size,
-                               b->bold_state + 6 * (int64_t)b->nvox, b->bold_state, b->rec_bold);
+                               b->bold_state + 6 * (int64_t)b->nvox, b->bold_state, b->rec_bold, nullptr);
         if (w.sample)
             hipLaunchKernelGGL(sample_kernel, dim3(grid_for(b->ns, 256)), dim3(256), 0, b->stream, b->ns, b->samples,
                                b->V, b->flags, k, b->rec_sspk, b->rec_sv);
@@ -3405,7 +3459,7 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
     // small records wanted in host memory come back through the pinned buffer,
     // larger ones (and those wanted on the device) by copies
     const int64_t S = b->S, kbig = std::min<int64_t>(nsteps, b->kmax);
-    const bool persist = persist_batch(b, a, w);
+    bool persist = persist_batch(b, a, w); // until a batch finds the device taken
     const bool small = kbig * (8 * S + 12) + 64 <= kPinBytes;
     const bool pin_freq = small && a->freqs && !is_device_ptr(a->freqs);
     const bool pin_vmean = small && a->vmeans && !is_device_ptr(a->vmeans);
@@ -3438,6 +3492,62 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
     if (uhost) DTB_TRY_HIP(hipMalloc(&ustage, sizeof(float) * (size_t)b->n * (size_t)std::min<int64_t>(nsteps, b->kmax)));
     int st = DTB_OK;
     int64_t done = 0, last = 0; // steps enqueued; of them, in the last batch
+    // one batch and the copies of its records
+    auto enqueue = [&](int32_t K, const float* u) -> int {
+        const bool graph = a->use_graph && a->noise_mode != DTB_NOISE_UNIFORMS && !w.timing;
+        if (graph) {
+            uint32_t nr;
+            std::memcpy(&nr, &a->noise_rate, 4);
+            std::vector<uint64_t> key{(uint64_t)K, (uint64_t)a->noise_mode, (uint64_t)a->isolated, nr,
+                                      (uint64_t)w.freq, (uint64_t)w.vsum, (uint64_t)w.isum, (uint64_t)w.sample,
+                                      (uint64_t)b->ns, (uint64_t)b->bold_sps, (uint64_t)(uintptr_t)hr.abort,
+                                      (uint64_t)(uintptr_t)hr.freq, (uint64_t)(uintptr_t)hr.vmean,
+                                      (uint64_t)(uintptr_t)hr.events, (uint64_t)(uintptr_t)hr.nspk, (uint64_t)persist};
+            auto it = b->graphs.find(key);
+            if (it == b->graphs.end()) {
+                hipGraph_t g;
+                if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+                    set_error("hipStreamBeginCapture failed");
+                    return DTB_RUNTIME_ERROR;
+                }
+                int s2 = enqueue_batch(b, K, a, nullptr, w, hr, persist);
+                hipError_t e2 = hipStreamEndCapture(b->stream, &g);
+                if (s2 || e2 != hipSuccess) {
+                    if (!s2) set_error("hipStreamEndCapture failed: %s", hipGetErrorString(e2));
+                    return s2 ? s2 : DTB_RUNTIME_ERROR;
+                }
+                hipGraphExec_t ge;
+                e2 = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+                hipGraphDestroy(g);
+                if (e2 != hipSuccess) {
+                    set_error("hipGraphInstantiate failed: %s", hipGetErrorString(e2));
+                    return DTB_RUNTIME_ERROR;
+                }
+                it = b->graphs.emplace(key, ge).first;
+            }
+            if (hipGraphLaunch(it->second, b->stream) != hipSuccess) {
+                set_error("hipGraphLaunch failed");
+                return DTB_RUNTIME_ERROR;
+            }
+        } else {
+            DTB_TRY(enqueue_batch(b, K, a, u, w, hr, persist));
+        }
+        DTB_TRY(copy_out(b, a->freqs && !pin_freq ? a->freqs + done * S : nullptr, b->rec_freq,
+                           sizeof(uint32_t) * (size_t)(S * K)));
+        DTB_TRY(copy_out(b, a->vmeans && !pin_vmean ? a->vmeans + done * S : nullptr, b->rec_vmean,
+                           sizeof(float) * (size_t)(S * K)));
+        DTB_TRY(copy_out(b, a->imeans ? a->imeans + done * S : nullptr, b->rec_isum, sizeof(float) * (size_t)(S * K)));
+        DTB_TRY(copy_out(b, a->sample_spike ? a->sample_spike + done * b->ns : nullptr, b->rec_sspk,
+                           (size_t)b->ns * K));
+        DTB_TRY(copy_out(b, a->sample_v ? a->sample_v + done * b->ns : nullptr, b->rec_sv,
+                           sizeof(float) * (size_t)b->ns * K));
+        DTB_TRY(copy_out(b, a->events && !pin_events ? a->events + done : nullptr, b->rec_events, sizeof(uint64_t) * K));
+        DTB_TRY(copy_out(b, a->spikes && !pin_spikes ? a->spikes + done : nullptr, b->rec_nspk, sizeof(uint32_t) * K));
+        if (bold)
+            DTB_TRY(copy_out(b, a->bold ? a->bold + (done / b->bold_sps) * b->nvox : nullptr, b->rec_bold,
+                             sizeof(double) * (size_t)b->nvox * (size_t)(K / b->bold_sps)));
+        return DTB_OK;
+    };
     while (done < nsteps && st == DTB_OK) {
         int64_t kcap = b->kmax;
         if (bold) kcap -= kcap % b->bold_sps;
@@ -3452,66 +3562,33 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
                 u = src;
             }
         }
-        const bool graph = a->use_graph && a->noise_mode != DTB_NOISE_UNIFORMS && !w.timing;
-        if (graph) {
-            uint32_t nr;
-            std::memcpy(&nr, &a->noise_rate, 4);
-            std::vector<uint64_t> key{(uint64_t)K, (uint64_t)a->noise_mode, (uint64_t)a->isolated, nr,
-                                      (uint64_t)w.freq, (uint64_t)w.vsum, (uint64_t)w.isum, (uint64_t)w.sample,
-                                      (uint64_t)b->ns, (uint64_t)b->bold_sps, (uint64_t)(uintptr_t)hr.abort,
-                                      (uint64_t)(uintptr_t)hr.freq, (uint64_t)(uintptr_t)hr.vmean,
-                                      (uint64_t)(uintptr_t)hr.events, (uint64_t)(uintptr_t)hr.nspk};
-            auto it = b->graphs.find(key);
-            if (it == b->graphs.end()) {
-                hipGraph_t g;
-                if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-                    set_error("hipStreamBeginCapture failed");
-                    st = DTB_RUNTIME_ERROR;
-                    break;
-                }
-                int s2 = enqueue_batch(b, K, a, nullptr, w, hr);
-                hipError_t e2 = hipStreamEndCapture(b->stream, &g);
-                if (s2 || e2 != hipSuccess) {
-                    if (!s2) set_error("hipStreamEndCapture failed: %s", hipGetErrorString(e2));
-                    st = s2 ? s2 : DTB_RUNTIME_ERROR;
-                    break;
-                }
-                hipGraphExec_t ge;
-                e2 = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-                hipGraphDestroy(g);
-                if (e2 != hipSuccess) {
-                    set_error("hipGraphInstantiate failed: %s", hipGetErrorString(e2));
-                    st = DTB_RUNTIME_ERROR;
-                    break;
-                }
-                it = b->graphs.emplace(key, ge).first;
-            }
-            if (hipGraphLaunch(it->second, b->stream) != hipSuccess) {
-                set_error("hipGraphLaunch failed");
+        if ((st = enqueue(K, u))) break;
+        if (persist) {
+            if (hipStreamSynchronize(b->stream) != hipSuccess) {
+                set_error("step batch failed: %s", hipGetErrorString(hipGetLastError()));
                 st = DTB_RUNTIME_ERROR;
                 break;
             }
-        } else {
-            if ((st = enqueue_batch(b, K, a, u, w, hr))) break;
+            const uint32_t how = *reinterpret_cast<volatile uint32_t*>(b->pin);
+            if (how == kGone) {
+                // other work holds the device: the batch has not begun, and the
+                // rest of the call runs on kernels that need not be resident
+                persist = false;
+                hr.abort = nullptr;
+                if (seg_args(b).seg) {
+                    hipLaunchKernelGGL(segment_reset_kernel, dim3(1), dim3(64), 0, b->stream, b->seg_cnt, b->D,
+                                       (int64_t)(b->steps_done + b->D));
+                    b->seg_dirty = false;
+                }
+                if ((st = enqueue(K, u))) break;
+            } else if (how) {
+                DTB_TRY_HIP(hipMemset(b->pbar + kPubAbort, 0, 4));
+                set_error("persistent step launch: a workgroup waited past the barrier limit; the block state is "
+                          "undefined");
+                st = DTB_RUNTIME_ERROR;
+                break;
+            }
         }
-        if ((st = copy_out(b, a->freqs && !pin_freq ? a->freqs + done * S : nullptr, b->rec_freq,
-                           sizeof(uint32_t) * (size_t)(S * K))))
-            break;
-        if ((st = copy_out(b, a->vmeans && !pin_vmean ? a->vmeans + done * S : nullptr, b->rec_vmean,
-                           sizeof(float) * (size_t)(S * K))))
-            break;
-        if ((st = copy_out(b, a->imeans ? a->imeans + done * S : nullptr, b->rec_isum, sizeof(float) * (size_t)(S * K)))) break;
-        if ((st = copy_out(b, a->sample_spike ? a->sample_spike + done * b->ns : nullptr, b->rec_sspk,
-                           (size_t)b->ns * K)))
-            break;
-        if ((st = copy_out(b, a->sample_v ? a->sample_v + done * b->ns : nullptr, b->rec_sv,
-                           sizeof(float) * (size_t)b->ns * K)))
-            break;
-        if ((st = copy_out(b, a->events && !pin_events ? a->events + done : nullptr, b->rec_events, sizeof(uint64_t) * K))) break;
-        if ((st = copy_out(b, a->spikes && !pin_spikes ? a->spikes + done : nullptr, b->rec_nspk, sizeof(uint32_t) * K))) break;
-        if (bold && (st = copy_out(b, a->bold ? a->bold + (done / b->bold_sps) * b->nvox : nullptr, b->rec_bold,
-                                   sizeof(double) * (size_t)b->nvox * (size_t)(K / b->bold_sps))))
-            break;
         if (w.timing) {
             if (hipStreamSynchronize(b->stream) != hipSuccess) {
                 set_error("step batch failed: %s", hipGetErrorString(hipGetLastError()));
@@ -3551,14 +3628,6 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
         return DTB_RUNTIME_ERROR;
     }
     from_pin(done - last, last);
-    if (persist && nsteps > 0) {
-        if (*reinterpret_cast<volatile uint32_t*>(b->pin)) {
-            DTB_TRY_HIP(hipMemset(b->pbar + kPubAbort, 0, 4));
-            set_error("persistent step launch: a workgroup waited past the barrier limit (not all workgroups "
-                      "resident); the block state is undefined");
-            return DTB_RUNTIME_ERROR;
-        }
-    }
     return DTB_OK;
 }
 
@@ -4786,6 +4855,9 @@ int dtb_block_set_launch(dtb_block* b, int32_t what, int32_t value)
         if (value > 0) DTB_TRY(ensure_segments(b));
         b->seg_cap = value == 0 ? 0 : value == 1 ? b->seg_alloc : std::min<int64_t>(value, b->seg_alloc);
         b->seg_dirty = true;
+    } else if (what == DTB_LAUNCH_PERSIST_WAIT) {
+        DTB_REQUIRE(value >= 0, "looks for a persistent launch's workgroups must be >= 0");
+        b->persist_wait = value;
     } else if (what == DTB_LAUNCH_DELIVER_MODE) {
         DTB_REQUIRE(value >= 0 && value <= 3,
                     "delivery mode must be 0 (atomics), 1 (bucketed), 2 or 3 (persistent, small blocks)");
@@ -4809,6 +4881,7 @@ int dtb_block_get_launch(dtb_block* b, int32_t what, int32_t* value)
     else if (what == DTB_LAUNCH_DELIVER_LANES) *value = b->deliver_lanes;
     else if (what == DTB_LAUNCH_DELIVER_MODE) *value = b->deliver_mode;
     else if (what == DTB_LAUNCH_NEURON_PSETS) *value = b->npsets;
+    else if (what == DTB_LAUNCH_PERSIST_WAIT) *value = b->persist_wait;
     else if (what == DTB_LAUNCH_STAGE_SEGS) *value = b->stage_segs;
     else if (what == DTB_LAUNCH_STAGE_EPT) *value = b->stage_ept;
     else if (what == DTB_LAUNCH_STAGE_VARIANT) *value = b->stage_variant;

@@ -15,7 +15,7 @@ struct StepCtl {
     int64_t nsteps;
     int64_t nbase;
     double t;
-    double pad;
+    double tbase; // t before the batch
 };
 
 struct Block {
@@ -160,7 +160,8 @@ struct Block {
     bool pwide = false;         // the weights in pcol are FP32 (mode 3), else rounded to int32 (mode 2)
     uint32_t* inexact = nullptr; // flag of fixed_exact
     void* pin = nullptr;        // pinned host buffer for small records (kPinBytes)
-    uint32_t* pbar = nullptr;   // [0] barrier counter, [64] abort flag
+    uint32_t* pbar = nullptr;   // [kPubWords]: publication words, abort flag, arrivals
+    int32_t persist_wait = 1 << 16; // looks that a persistent launch waits for its workgroups to be on the device
     int32_t pG = 0, pm = 0;     // workgroups, 256-neuron blocks of LDS slice per workgroup
     int32_t pper = 0;           // neurons per workgroup (consecutive ranges)
     bool persist_dirty = true;

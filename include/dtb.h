@@ -328,6 +328,9 @@ int dtb_block_set_external(dtb_block* b, int32_t n_thresholds, const uint32_t* t
                                        instead of the CSR's row pointer and segment ends at every delay; 0 turns
                                        this off; a value > 1 caps the entries per list (a step whose list is full
                                        reads the spike lists instead); get returns the cap in use, 0 when off */
+#define DTB_LAUNCH_PERSIST_WAIT 11 /* persistent delivery needs all its workgroups on the device at once: how many
+                                      times (about a microsecond each, default 65536) one looks for the others
+                                      before the batch runs on the mode-1 kernels instead; 0: at once */
 int dtb_block_set_launch(dtb_block* b, int32_t what, int32_t value);
 int dtb_block_get_launch(dtb_block* b, int32_t what, int32_t* value);
 

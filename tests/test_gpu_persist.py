@@ -204,3 +204,23 @@ def test_persistent_sums_agree_on_dyadic_weights(n, K, D, pair):
     assert tot > 0
     for nb in blocks:
         nb.close()
+
+
+def test_persistent_batch_runs_on_the_per_step_kernels_when_its_workgroups_do_not_arrive():
+    """A device that other work holds may not have room for all workgroups of
+    the launch at once.  With no looks for them (persist_wait=0) every launch
+    gives up before its first step; the call must then run its batches on the
+    bucketed kernels and leave state, records, BOLD and time as if it had
+    begun there, over batch ends, graph replays and delays, and the next call
+    finds the launch as it was."""
+    a, b = _pair(9_000, 7_200, 60, 5, False, seed=5, mode=2, bold=True)
+    assert b.get_launch()["persist_wait"] > 0
+    _run_both(a, b, 40, graph=True)
+    for wait in (0, 1 << 16):
+        b.set_launch(persist_wait=wait)
+        assert b.get_launch()["persist_wait"] == wait
+        for steps, graph in ((10, False), (1_030, True), (10, True), (10, True)):
+            r = _run_both(a, b, steps, graph=graph)
+            assert a.t == b.t and a.steps == b.steps
+    assert int(r["events"].sum()) > 0
+    a.close(); b.close()
