@@ -93,16 +93,35 @@ def csr_from_w(w_uij):
                 w1=None if np.array_equal(w0, w1) else w1)
 
 
-# Blocks of these sizes run their steps in the persistent launch.  Above, its 32
-# workgroups no longer keep a neuron per thread in registers; below, a step is
-# all launch cost either way.  us, persistent against direct delivery: 20 steps
-# in one call 229 and 238 (1,000 neurons), 205 and 234 (2,000), 195 and 343
-# (10,000), 314 and 497 (32,768); a one-step call 34.6 and 31.4, 33.7 and 31.7,
-# 33.3 and 36.9, 41.2 and 37.2.
+# Which calls of run and run_steps take the persistent launch.  Its (at most)
+# 32 workgroups of a neuron per thread hold 32,768 neurons.  us, per-step
+# kernels against persistent launch, for networks at rest (noise spikes at 10
+# Hz) and, after the slash, at 460 Hz:
+#   20 steps in a call:
+#     synapses per neuron        20                100               1,000
+#      2,000 neurons    174:145 / 228:190  185:160 / 248:245  280:165 / 613:898
+#      6,000            196:157 / 251:204  220:172 / 298:244  410:181 / 988:1048
+#     10,000            211:154 / 267:193  227:159 / 352:214  467:180 / 1319:694
+#     32,768            254:220 / 338:286  267:230 / 618:363  574:267 / 3445:1368
+#   so below 10,000 neurons, where fewer workgroups share the events of a
+#   volley, up to one synapse per neuron for every 20 neurons of the block
+#   (6,000 x 400: 310:173 / 539:543).
+#   one step in a call:
+#     synapses per neuron        100               400               1,000
+#      2,000 neurons     28:31 / 31:34      30:31 / 34:38      33:31 / 42:45
+#     10,000             29:31 / 34:33      35:32 / 40:37      42:32 / 51:42
+#     16,000             30:31 / 36:34      35:32 / 48:41      43:32 / 61:47
+#     32,768             32:38 / 41:42      38:39 / 71:52      47:40 / 85:58
+#   The launch, and its set-up of 6 us more above 16,384 neurons, are paid back
+#   by 8 steps of any of these blocks; shorter calls need the denser ones (the
+#   plain block of 10,000 x 100, which fires at the higher rate, among them).
+# Building its copy of the synapses takes 0.3 to 1 ms up to 4 M synapses and
+# 5 ms for 32 M, so larger blocks run 200 steps first.
 PERSIST_N = (2000, 32 * 1024)
-# Steps after a weight change that run on the per-step kernels: the persistent
-# launch keeps a copy of the synapses grouped on the host, which a program that
-# changes weights between steps should not pay for each time.
+PERSIST_CALL = 8
+PERSIST_NNZ, PERSIST_STEPS = 4_000_000, 200
+# Steps after a weight change that run on the per-step kernels: a program that
+# changes weights between steps should not pay for that copy each time.
 PERSIST_HOLD = 1000
 
 
@@ -152,24 +171,33 @@ class block:
     # _mode: 2 in the persistent launch, else the kernels' mode (0 or 1).
     def _choose_launch(self, hold=0):
         self._base_mode = self._mode = self._nb.get_launch()["deliver_mode"]
+        self._nnz = self._nb.nnz
         self._persist = self.src is None and PERSIST_N[0] <= self.N <= PERSIST_N[1]
-        self._hold = hold
+        self._weights_changed(hold)
+
+    def _weights_changed(self, hold):
+        self._seen = 0  # steps run with these weights
+        self._wait = max(hold, 0 if self._nnz <= PERSIST_NNZ else PERSIST_STEPS)
+
+    def _persist_pays(self, steps):
+        per = self._nnz / self.N
+        if steps < PERSIST_CALL:
+            return self.N >= 10_000 and per >= (100 if self.N <= 16 * 1024 else 1000)
+        return self.N >= 10_000 or 20 * per <= self.N
 
     def _set_mode(self, steps, persist=True):
         mode = self._base_mode
-        if persist and self._persist:
-            if self._hold > 0:
-                self._hold -= steps
-            else:
-                mode = 2
+        if persist and self._persist and self._seen >= self._wait and self._persist_pays(steps):
+            mode = 2
+        self._seen += steps
         if mode != self._mode:
             try:
                 self._nb.set_launch(deliver_mode=3 if mode == 2 else mode)
                 self._mode = mode
             except nat.DTBError as e:
-                if e.code != nat.DTB_INVALID_PARAMETER:
+                if mode != 2 or e.code not in (nat.DTB_INVALID_PARAMETER, nat.DTB_OUT_OF_MEMORY):
                     raise
-                self._persist = False  # it does not hold this block, or not all of its weights' bits
+                self._persist = False  # it does not hold this block, or all bits of its weights, or has no room
 
     def _apply_sources(self, nb):
         k, t = np.nonzero(self._sched)
@@ -217,7 +245,7 @@ class block:
             raise IndexError("conn_idx out of range")
         if self._mode != self._base_mode:
             self._set_mode(0, persist=False)
-        self._hold = PERSIST_HOLD
+        self._weights_changed(PERSIST_HOLD)
         try:
             self._nb.set_weights(pre, post, ch, w)
         except nat.DTBError as e:

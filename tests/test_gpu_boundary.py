@@ -482,15 +482,54 @@ def test_dropin_keeps_weights_of_several_decades(n, decades, mode):
         o.run(noise_rate=0.0, isolated=True, seed=5)
     assert not b.J_ui.numpy().any()
     most = int(np.bincount(csr["post"] * 2 + csr["kind"]).max())
-    for k in range(1, 13):
-        if k % 4:
-            b.run(noise_rate=2.0 ** -6, isolated=True)
-        else:
-            b.run_steps(1, noise_rate=2.0 ** -6, isolated=True)
-            assert b._mode == mode
-        o.run(noise_rate=2.0 ** -6, isolated=True, seed=5)
+    for k in (8, 16, 24):
+        b.run_steps(8, noise_rate=2.0 ** -6, isolated=True)
+        assert b._mode == mode
+        for _ in range(8):
+            o.run(noise_rate=2.0 ** -6, isolated=True, seed=5)
         J, Jo = b.J_ui.numpy(), o.get("J")
         assert np.array_equal(J > 0, Jo > 0)
         np.testing.assert_allclose(J, Jo, rtol=(3 + most) * k * 2.0 ** -24, atol=0)
     assert (Jo > 0).sum() > n
 
+
+def test_dropin_returns_to_the_persistent_launch_after_a_weight_change():
+    """Once the steps after a weight change are over, the launch's copy of the
+    synapses is built again: from the new weights, one of them large enough to
+    give its channels other exponents.  Short and long calls alternate, on
+    both sides of the switch (dyadic weights: every order gives the same sums)."""
+    from digital_twin_brain_amd import block as block_class
+
+    n = 2300
+    rng = np.random.default_rng(n)
+    csr = orc.gen_fixed_indegree(n, n * 4 // 5, 40, 1, 0.0, 1.0, False, seed=n)
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    _, first = np.unique(pre * n + csr["post"], return_index=True)
+    keep = np.zeros(pre.shape[0], bool)
+    keep[first] = True
+    csr = _keep_synapses(n, csr, keep)
+    w = (np.floor(csr["w0"] * 256) / 256).astype(np.float32)
+    pre = np.repeat(np.arange(n), np.diff(csr["rowptr"]))
+    p = _lif_props(n, rng, g_scale=1.5)
+    idx = torch.from_numpy(np.stack([csr["kind"].astype(np.int64) * 2, csr["post"], pre]))
+    idx = torch.cat([idx, idx + torch.tensor([[1], [0], [0]])], dim=1)
+    W = torch.sparse_coo_tensor(idx, torch.from_numpy(np.concatenate([w, w])), (4, n, n))
+    a = block_class(torch.from_numpy(p), W, delta_t=0.1, seed=5)
+    b = block_class(torch.from_numpy(p), W, delta_t=0.1, seed=5)
+    b._persist = False
+    ch, post, src = (x[:200].numpy() for x in idx)
+
+    def both(f):
+        for x, y in zip(f(a), f(b)):
+            np.testing.assert_allclose(x.numpy(), y.numpy(), rtol=2.0 ** -23, atol=0)
+
+    modes = []
+    for value in (64.0, 0.25):
+        for steps in (30, 1, 30, 1000, 30, 1, 30):
+            both(lambda x: x.run_steps(steps, noise_rate=2.0 ** -6) if steps > 1 else x.run(noise_rate=2.0 ** -6))
+            modes.append(a._mode)
+        assert np.array_equal(a.V_i.numpy(), b.V_i.numpy())
+        assert np.array_equal(a.J_ui.numpy(), b.J_ui.numpy())
+        for x in (a, b):
+            x.update_conn_weight((ch, post, src), np.full(200, value, np.float32))
+    assert modes == [2, 0, 2, 2, 2, 0, 2] + [0, 0, 0, 0, 2, 0, 2]
