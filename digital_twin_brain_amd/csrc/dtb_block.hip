@@ -2822,8 +2822,6 @@ static int alloc_ring_and_records(Block* b)
     DTB_TRY(block_alloc(b, &b->acc, esz * (size_t)b->n));
     DTB_TRY_HIP(hipMemsetAsync(b->acc, 0, esz * (size_t)b->n, b->stream));
     DTB_TRY(alloc_n(b, &b->rec_freq, b->kmax * b->S));
-    DTB_TRY(alloc_n(b, &b->rec_vsum, b->kmax * b->S));
-    DTB_TRY(alloc_n(b, &b->rec_vmean, b->kmax * b->S));
     DTB_TRY(alloc_n(b, &b->rec_isum, b->kmax * b->S));
     // delivery launch shape: about one segment per lane group at ~20 Hz of
     // spikes (an autotuner may replace it, dtb_block_set_launch)
@@ -3460,6 +3458,9 @@ static int run_impl(Block* b, int64_t nsteps, const dtb_run_args* a)
     const bool pin_vmean = small && a->vmeans && !is_device_ptr(a->vmeans);
     const bool pin_events = small && a->events && !is_device_ptr(a->events);
     const bool pin_spikes = small && a->spikes && !is_device_ptr(a->spikes);
+    // 12 bytes a population and step, for the runs that ask for means
+    if (w.vsum && !b->rec_vsum) DTB_TRY(alloc_n(b, &b->rec_vsum, b->kmax * S));
+    if (w.vsum && !pin_vmean && !b->rec_vmean) DTB_TRY(alloc_n(b, &b->rec_vmean, b->kmax * S));
     HostRecords hr{};
     if (persist || pin_freq || pin_vmean || pin_events || pin_spikes) {
         if (!b->pin) DTB_TRY_HIP(hipHostMalloc(&b->pin, kPinBytes, hipHostMallocDefault));

@@ -72,8 +72,8 @@ struct Block {
 
     // per-step records of the current batch
     uint32_t* rec_freq = nullptr; // [kmax][S]
-    double* rec_vsum = nullptr;   // [kmax][S]
-    float* rec_vmean = nullptr;   // [kmax][S]
+    double* rec_vsum = nullptr;   // [kmax][S], on first use
+    float* rec_vmean = nullptr;   // [kmax][S], on first use
     float* rec_isum = nullptr;    // [kmax][S]
     uint64_t* rec_events = nullptr; // [kmax]
     uint64_t* ev_part = nullptr;    // partial event counters of a step (zero between steps)

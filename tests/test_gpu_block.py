@@ -874,3 +874,29 @@ def test_fixed_point_per_neuron_scale_on_heterogeneous_inputs(mode):
     assert scale[got].min() < 3e-3 and scale[got].max() > 0.3 and k_of[got].min() < 30
     print(f"mode {mode}: worst J error {worst:.3g} x tolerance, launch {nb.get_launch()}")
     nb.close()
+
+
+def test_mean_records_take_memory_only_when_means_are_asked_for():
+    """Per-step records of a block of many populations: counts and I_syn sums
+    (4 bytes a population and step each, 1,000 steps) from the start, the FP64
+    V sums and the means once a run asks for them."""
+    from digital_twin_brain_amd import NativeBlock
+
+    n = 40_000
+    p = np.zeros((n, 22), np.float32)
+    p[:, 3] = np.arange(n)
+    p[:, 4] = 1; p[:, 5] = 2; p[:, 6] = 0.03; p[:, 7] = -75; p[:, 8] = -50; p[:, 9] = -65
+    p[:, 18:22] = (2, 40, 10, 50)
+    warm = NativeBlock.fixed_indegree(p[:1000], 800, 10, noise_seed=1)
+    warm.run(1, noise_mode=0, noise_rate=0.0, freqs=np.zeros((1, 1000), np.uint32))
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    nb = NativeBlock.fixed_indegree(p, 32_000, 10, noise_seed=1)
+    assert nb.S == n
+    f = np.zeros((1, n), np.uint32)
+    nb.run(1, noise_mode=0, noise_rate=0.0, freqs=f)
+    assert free0 - torch.cuda.mem_get_info()[0] < 1000 * n * 12 + (64 << 20)
+    vm = np.zeros((2, n), np.float32)
+    nb.run(2, noise_mode=0, noise_rate=0.0, freqs=np.zeros((2, n), np.uint32), vmeans=vm)
+    np.testing.assert_allclose(vm[1], nb.get("V"), rtol=1e-6)  # a neuron a population
+    warm.close(); nb.close()
