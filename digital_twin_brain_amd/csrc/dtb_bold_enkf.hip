@@ -318,12 +318,12 @@ __global__ __launch_bounds__(256) void enkf_update_kernel(int32_t E, int32_t V, 
 }
 
 // The analysis on a caller-chosen scratch of enkf_scratch_doubles doubles:
-// wd [E*V*S], the gains and innovations of each voxel [V*E] and gsum [V*S],
-// with room left over.  Every scratch element is written before it is read.
+// wd [E*V*S], the gains and innovations of each voxel [V*E] and gsum [V*S].
+// Every scratch element is written before it is read.
 static size_t enkf_scratch_doubles(int32_t E, int32_t V, int32_t S)
 {
-    const size_t EVS = (size_t)E * V * S, VS = (size_t)V * S, EV = (size_t)E * V, EE = (size_t)E * E;
-    return VS + EVS + 2 * EV + VS + EE;
+    const size_t EVS = (size_t)E * V * S, VS = (size_t)V * S, EV = (size_t)E * V;
+    return EVS + 2 * EV + VS;
 }
 
 static int enkf_launch(int32_t E, int32_t V, int32_t S, double* w, double sigma, const double* y, double rho,
@@ -396,7 +396,7 @@ static int enkf(int32_t E, int32_t V, int32_t S, double* w, double sigma, const 
 // address, so each device's address comes from hipGetSymbolAddress, taken
 // once per device with that device current, and only that address is handed
 // to the kernels.
-constexpr size_t kEnkfScratchMax = (size_t)1 << 19; // doubles (4 MiB): E = 256, V = 90, S = 10 needs 343,816
+constexpr size_t kEnkfScratchMax = (size_t)1 << 19; // doubles (4 MiB): E = 256, V = 90, S = 10 needs 277,380
 static __device__ __align__(256) double scratch[kEnkfScratchMax];
 static std::mutex g_scratch_mu;
 static double* g_scratch_ptr[64] = {nullptr};
@@ -409,9 +409,10 @@ static int enkf_noalloc(int32_t E, int32_t V, int32_t S, double* w, double sigma
     DTB_REQUIRE((size_t)E <= kEnkfScratchMax && (size_t)V <= kEnkfScratchMax && (size_t)S <= kEnkfScratchMax,
                 "allocation-free EnKF: E=%d, V=%d, S=%d exceeds the fixed scratch of %zu doubles "
                 "(use dtb_enkf_analysis_f64)", E, V, S, kEnkfScratchMax);
-    const size_t need = enkf_scratch_doubles(E, V, S);
+    // the documented limit, which also counts a mean [V*S] and a matrix [E*E]
+    const size_t need = enkf_scratch_doubles(E, V, S) + (size_t)V * S + (size_t)E * E;
     DTB_REQUIRE(need <= kEnkfScratchMax,
-                "allocation-free EnKF: E=%d, V=%d, S=%d needs %zu scratch doubles, the fixed scratch holds %zu "
+                "allocation-free EnKF: E=%d, V=%d, S=%d counts %zu scratch doubles, the fixed scratch holds %zu "
                 "(use dtb_enkf_analysis_f64)", E, V, S, need, kEnkfScratchMax);
     int dev = 0;
     DTB_TRY_HIP(hipGetDevice(&dev));

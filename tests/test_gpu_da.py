@@ -376,3 +376,18 @@ def test_enkf_tile_and_chunk_edges(E, V, S, rho):
     want, bound = _enkf_reference(w, 1e-2, y, rho, xi)
     err = np.abs(d[0].cpu().numpy() - want)
     assert (err <= bound).all(), float((err / bound).max())
+
+
+def test_enkf_scratch_grows_with_what_the_analysis_stores():
+    """8,000 members of one voxel and state need 32,000 doubles of scratch; an
+    E x E matrix, which the analysis does not store, would be 512 MB."""
+    from digital_twin_brain_amd.enkf import diffusion_enkf
+
+    E = 8000
+    w = torch.randn((E, 1, 1), dtype=torch.float64, device="cuda")
+    y = torch.zeros((1, 1), dtype=torch.float64, device="cuda")
+    xi = torch.zeros((E, 1), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    diffusion_enkf(w, 1e-4, y, 0.5, xi=xi)
+    assert free0 - torch.cuda.mem_get_info()[0] < 256 << 20
