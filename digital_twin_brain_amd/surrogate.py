@@ -30,6 +30,15 @@ def _params(rows):
     return np.array([(r, c, *(0 if x is None else x.data_ptr() for x in ts)) for r, c, *ts in rows], dtype=np.int64)
 
 
+def _broadcast(x, shape, dev):
+    """x as contiguous FP32 on the device, broadcast to `shape` as an assignment
+    to a tensor of that shape broadcasts it (leading ones beyond its rank go)."""
+    x = torch.as_tensor(x).to(dev, torch.float32)
+    while x.dim() > len(shape) and x.shape[0] == 1:
+        x = x[0]
+    return x.expand(shape).contiguous()
+
+
 class MLPSurrogate:
     def __init__(self, n_in, n_out, hidden=(512, 512, 512), max_batch=256, device=0, seed=0, lr=1e-3,
                  betas=(0.9, 0.999), eps=1e-8):
@@ -411,9 +420,8 @@ class GRUSurrogate:
         T, r, B = self._forward(X, h0)
         H, I, O = self.H, self.I, self.O
         TB = T * B
-        Yd = torch.as_tensor(Y).to(self.dev, torch.float32).expand(T, r, self.n_out).contiguous()
-        Md = None if mask is None else \
-            torch.as_tensor(mask).to(self.dev, torch.float32).expand(T, r, self.n_out).contiguous()
+        Yd = _broadcast(Y, (T, r, self.n_out), self.dev)
+        Md = None if mask is None else _broadcast(mask, (T, r, self.n_out), self.dev)
         nat.check(self.lib.dtb_mlp_sequence_loss(T, B, O, r, self.n_out, self.Y.data_ptr(), Yd.data_ptr(),
                                                  self.y_scale.data_ptr(), self.y_shift.data_ptr(), nat.ptr(Md),
                                                  1.0 / (T * r), self.Gy.data_ptr(), self.Gyb.data_ptr(),

@@ -436,3 +436,24 @@ def test_gru_beyond_the_sequence_kernels():
     for k in g:
         if k in sur.grad:
             assert _rel(sur.grad[k].cpu().double().numpy(), g[k]) < 5e-3, k
+
+
+def test_gru_targets_and_masks_broadcast_as_in_an_assignment():
+    from digital_twin_brain_amd.surrogate import GRUSurrogate
+
+    T, r = 3, 5
+    g = torch.Generator().manual_seed(1)
+    m = GRUSurrogate(4, 6, hidden=32, max_batch=8, max_steps=T)
+    X, Y = torch.randn((T, r, 4), generator=g), torch.randn((T, r, 6), generator=g)
+    mask = (torch.rand((r, 1), generator=g) > 0.4).float()
+
+    def grads(y, k):
+        loss = m.gradients(X, y, mask=k).clone()
+        return [loss] + [v.clone() for v in m.grad.values()]
+
+    want = grads(Y, mask.expand(T, r, 6))
+    for y, k in ((Y[None], mask), (Y, mask[None, None]), (Y[None, None], mask.expand(1, 1, T, r, 6))):
+        for a, b in zip(grads(y, k), want):
+            assert torch.equal(a, b)
+    with pytest.raises(RuntimeError):
+        m.gradients(X, Y[None].expand(2, T, r, 6))
