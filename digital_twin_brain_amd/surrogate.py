@@ -108,6 +108,41 @@ class MLPSurrogate:
         self.T = torch.empty((B, self.sizes[-1]), **f32)
         self.M = torch.empty((B, self.sizes[-1]), **f32)
 
+    def _chain_pays(self, rows, train=False):
+        """Whether the whole-network kernel is the faster way to take `rows` rows
+        (else a launch per product, the same results bit for bit).
+
+        It is, by far, for many rows.  But up to max_batch rows of a wide
+        network leave most of the device idle while each workgroup streams
+        every weight (10.5 us a MB) and walks wide inputs and outputs, where
+        the launches cost 4.5 us each more than its layers and spread over the
+        device.  us, launches : whole network, four layers with hidden widths h:
+            18 -> h -> 6, 90 rows         h = 512 52:39, 768 56:50, 1,024 59:74
+            18 -> h -> 1,000, 256 rows    h = 128 47:57, 512 48:71; 2,048 rows 55:58, 78:73
+            720 -> h -> 540, 256 rows     h = 128 49:61, 512 50:74; 2,048 rows 54:61, 86:77
+            1,100 -> h -> 900, 256 rows   h = 128 48:77, 1,024 59:164; 8,192 rows 104:97, 302:170
+        and 18 -> 768 x 6 -> 6, 90 rows 81:98.  Training has more to gain
+        (43 launches) and loses only for a single tile of rows of the widest:
+        32 rows of 1,100 -> 1,024 x 3 -> 900 224:304, of 720 -> 1,024 x 3 -> 540
+        214:252, but of 18 -> 1,024 x 3 -> 6 199:156."""
+        n_in, n_out = self.sizes[0], self.sizes[-1]
+        mb = 2e-6 * sum(w.numel() for w in self.W)  # bf16
+        if train:
+            return rows > 32 or mb < 6 or n_in + n_out < 1000
+        if rows > self.max_batch:
+            return True
+        return 10.5 * mb + 0.02 * n_in + 0.03 * n_out <= 11 + 4.5 * len(self.W) + 0.006 * rows * mb
+
+    def _use_chain(self, rows, train=False):
+        if not (self.chain_train if train else self.chain):
+            return False
+        if self._chain_pays(rows, train):
+            return True
+        if self.Wb is None:
+            self._alloc_layers()
+            self._refresh_bf16()
+        return False
+
     def _table(self):
         """dtb_mlp_layer [layers] (ten 8-byte fields each) of the current buffers."""
         return np.array([(w.shape[1], w.shape[0], wf.data_ptr(), wt.data_ptr(), b.data_ptr(), dw.data_ptr(),
@@ -160,7 +195,7 @@ class MLPSurrogate:
         X = torch.as_tensor(X)
         n = X.shape[0]
         out = torch.empty((n, self.n_out), dtype=torch.float32, device=self.dev)
-        if self.chain:
+        if self._use_chain(n):
             X = X.to(self.dev, torch.float32).contiguous()
             table = self._table()
             nat.check(self.lib.dtb_mlp_predict(len(self.W), table.ctypes.data, n, self.max_batch, X.data_ptr(),
@@ -192,7 +227,7 @@ class MLPSurrogate:
         B = _pad(r)
         no = self.sizes[-1]
         Yd = torch.as_tensor(Y).to(self.dev, torch.float32).contiguous()
-        if self.chain_train:
+        if self._use_chain(r, train=True):
             X = X.to(self.dev, torch.float32).contiguous()
             Md = None if mask is None else \
                 torch.as_tensor(mask).to(self.dev, torch.float32).expand(r, self.n_out).contiguous()

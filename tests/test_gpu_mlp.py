@@ -457,3 +457,34 @@ def test_gru_targets_and_masks_broadcast_as_in_an_assignment():
             assert torch.equal(a, b)
     with pytest.raises(RuntimeError):
         m.gradients(X, Y[None].expand(2, T, r, 6))
+
+
+# wide networks on both sides of the rule that sends few rows to a launch per product
+@pytest.mark.parametrize("n_in,n_out,hidden,rows,chain,chain_train", [
+    (18, 6, (512, 512, 512), 90, True, True), (18, 6, (1024, 1024, 1024), 90, False, True),
+    (720, 540, (512, 512, 512), 40, False, True), (720, 540, (512, 512, 512), 2048, True, True),
+    (720, 540, (1024, 1024, 1024), 32, False, False), (1100, 900, (1024, 1024, 1024), 33, False, True)])
+def test_few_rows_of_wide_networks_go_layer_by_layer(n_in, n_out, hidden, rows, chain, chain_train):
+    """The same predictions and weight gradients bit for bit, before and after
+    an update, and with a first layer-by-layer call after it."""
+    from digital_twin_brain_amd.surrogate import MLPSurrogate
+
+    g = torch.Generator().manual_seed(rows + n_in)
+    X, Y = torch.randn((rows, n_in), generator=g), torch.randn((rows, n_out), generator=g)
+    a, b, late = (MLPSurrogate(n_in, n_out, hidden=hidden, max_batch=max(rows, 64), seed=4) for _ in range(3))
+    assert a.chain and a.chain_train
+    assert a._chain_pays(rows) == chain and a._chain_pays(rows, train=True) == chain_train
+    assert a._chain_pays(a.max_batch + 1)
+    b._chain_pays = lambda rows, train=False: True
+    for _ in range(2):
+        assert torch.equal(a.predict(X), b.predict(X))
+        for s in (a, b, late):
+            s.gradients(X, Y)
+        for l in range(len(hidden) + 1):
+            assert torch.equal(a.dW[l], b.dW[l]), l
+            for s in (a, late):  # FP32 sums in another order
+                s.db[l].copy_(b.db[l])
+        for s in (a, b, late):
+            s.step()
+    assert torch.equal(a.predict(X), b.predict(X)) and torch.equal(late.predict(X), b.predict(X))
+    assert (a.Wb is not None) == (not chain or not chain_train)
