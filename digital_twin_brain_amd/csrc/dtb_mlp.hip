@@ -1612,18 +1612,26 @@ using GruBwdWeights = GruWeights<(2 * G + kGruBwdWaves - 1) / kGruBwdWaves, 3 * 
 //   128 or more 64x64 tiles: split-K's 32x32 tiles read each operand row twice
 //     as often, in 32-byte pieces (768^2 K = 768: 13.5 split, 7.1 tiles; 96 x
 //     6144 K = 3008: 38.3, 21.1); up to 64 its workgroups are the only ones
-//     that fill the CUs (512^2 K = 512: 4.7, 6.0);
+//     that fill the CUs (512^2 K = 512: 4.7, 6.0), and so they are up to 256
+//     32x32 tiles, a round of one a CU, where a 64x64 tile is half padding (32 x
+//     8192 K = 4096: 22.0, 29.0; 32 x 12000, 375 tiles: 36.9, 30.1);
 //   128x128 tiles once every CU gets one (2048^2: 64x64 29.4, 128x128 23.8;
 //     1536^2 K = 1536, 144 tiles: 15.5, 17.0);
 //   256x256 tiles, one a CU and 1.75 times the time of a round of 128x128
 //     tiles, two a CU, where that many fewer rounds do (8192^3: 808 against
 //     1033; 5024 x 1632 K = 2000: 51 against 59; 6144^3, 2.25 rounds: 426
-//     against 416).
-static int gemm_tile(int32_t M, int32_t N)
+//     against 416);
+//   a short K is bound by the stores of C, which several workgroups a CU
+//     overlap and one does not: 64x64 tiles up to K = 256, or 192 past 2,304
+//     tiles of 256 (8192^2, tiles of 64, 128 and 256: K = 64 48, 52, 62; 128 53,
+//     57, 67; 256 77, 73, 82; 384 101, 88, 95.  8192 x 12288: 128 84, 114, 106;
+//     256 113, 137, 125; 384 144, 185, 149.  4096^2 K = 256: 22.0, 22.3, 23.5.
+//     16384^2: 128 278, 281, 309; 256 397, 373, 362).
+static int gemm_tile(int32_t M, int32_t N, int32_t K)
 {
     auto tiles = [&](int32_t t) { return (int64_t)((M + t - 1) / t) * ((N + t - 1) / t); };
-    if (!gemm_one_chain(M, N)) return tiles(64) >= 128 ? -1 : 0;
-    if (tiles(128) < 256) return 1;
+    if (!gemm_one_chain(M, N)) return tiles(64) >= 128 && tiles(32) > 256 ? -1 : 0;
+    if (tiles(128) < 256 || K <= 192 || (K <= 256 && tiles(256) <= 2304)) return 1;
     const int64_t r4 = (tiles(256) + 255) / 256, r2 = (tiles(128) + 511) / 512;
     return 7 * r4 <= 4 * r2 ? 4 : 2;
 }
@@ -1661,7 +1669,7 @@ int dtb_mlp_gemm_bf16_nt(int32_t M, int32_t N, int32_t K, const void* A, int64_t
     DTB_REQUIRE(act == 0 || act == 1, "act must be 0 (identity) or 1 (ReLU)");
     DTB_REQUIRE((reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0,
                 "A and B must be 16-byte aligned");
-    switch (gemm_tile(M, N)) {
+    switch (gemm_tile(M, N, K)) {
     case 4: DTB_TRY((launch_gemm_tile<4, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
     case 2: DTB_TRY((launch_gemm_tile<2, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;
     case 1: DTB_TRY((launch_gemm_tile<1, false>(M, N, K, A, lda, B, ldb, bias, act, C, ldc, Cb, ldcb, stream))); break;

@@ -541,17 +541,18 @@ class GRUSurrogate:
 def gemm_kernel_name(M, N, K):
     """The kernel dtb_mlp_gemm_bf16_nt dispatches an M x N x K product to:
     LDS-staged square tiles of 256, 128 or 64 (the fewest rounds of
-    workgroups, weighed by a round's time; 64 with K in four ranges where
-    there are fewer than 256 such tiles), or below 128 tiles of 64 the
-    32x32 tiles with K split over the four wavefronts."""
+    workgroups, weighed by a round's time, and smaller ones for a short K; 64
+    with K in four ranges where there are fewer than 256 such tiles), or below
+    128 tiles of 64, or up to 256 of 32, the 32x32 tiles with K split over the
+    four wavefronts."""
     def tiles(t):
         return -(-M // t) * -(-N // t)
 
-    if tiles(64) < 128:
+    if tiles(64) < 128 or (tiles(64) < 256 and tiles(32) <= 256):
         return "gemm_nt_splitk_kernel (32x32 tiles, K split over 4 wavefronts, bf16 MFMA, FP32 accumulate)"
     if tiles(64) < 256:
         return "gemm_nt_tile_kernel<1> (64x64 LDS-staged tiles, K in 4 ranges, bf16 MFMA, FP32 accumulate)"
-    if tiles(128) < 256:
+    if tiles(128) < 256 or K <= 192 or (K <= 256 and tiles(256) <= 2304):
         t = 1
     else:
         t = 4 if 7 * -(-tiles(256) // 256) <= 4 * -(-tiles(128) // 512) else 2

@@ -85,6 +85,25 @@ def test_gemm_tile_edges(M, N, K):
     assert torch.equal(C, want)
 
 
+# both sides of the rules that choose by K and by the number of 32x32 tiles (256: one a CU)
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (4096, 4128, 192, "tile_kernel<1>"), (4096, 4128, 256, "tile_kernel<1>"), (4096, 4128, 272, "tile_kernel<2>"),
+    (4096, 4064, 272, "tile_kernel<4>"), (12320, 12288, 192, "tile_kernel<1>"), (12320, 12288, 208, "tile_kernel<4>"),
+    (32, 8192, 1040, "splitk"), (8192, 32, 1040, "splitk"), (32, 8224, 1040, "tile_kernel<1>"),
+    (64, 8192, 1040, "tile_kernel<1>")])
+def test_gemm_on_both_sides_of_the_tile_rules(M, N, K, kernel):
+    from digital_twin_brain_amd.surrogate import gemm_kernel_name
+
+    assert kernel in gemm_kernel_name(M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randint(-4, 5, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+    B = torch.randint(-4, 5, (N, K), generator=g, device="cuda").to(torch.bfloat16)
+    C = torch.empty((M, N), device="cuda")
+    nat.check(nat.lib().dtb_mlp_gemm_bf16_nt(M, N, K, A.data_ptr(), K, B.data_ptr(), K, None, 0, C.data_ptr(), N, None,
+                                             0, ctypes_stream()))
+    assert torch.equal(C, A.float() @ B.float().T)
+
+
 def test_gemm_rejects_bad_shapes():
     L = nat.lib()
     A = torch.zeros((32, 16), dtype=torch.bfloat16, device="cuda")
