@@ -99,26 +99,29 @@ def csr_from_w(w_uij):
 # Hz) and, after the slash, at 460 Hz:
 #   20 steps in a call:
 #     synapses per neuron        20                100               1,000
-#      2,000 neurons    174:145 / 228:190  185:160 / 248:245  280:165 / 613:898
-#      6,000            196:157 / 251:204  220:172 / 298:244  410:181 / 988:1048
-#     10,000            211:154 / 267:193  227:159 / 352:214  467:180 / 1319:694
-#     32,768            254:220 / 338:286  267:230 / 618:363  574:267 / 3445:1368
+#      2,000 neurons    179:150 / 232:188  187:159 / 248:243  280:164 / 630:894
+#      6,000            188:156 / 249:203  217:172 / 305:246  412:179 / 998:1051
+#     10,000            196:155 / 258:193  222:162 / 354:214  466:184 / 1330:694
+#     18,000            214:211 / 282:255  231:220 / 441:298  518:253 / 1995:856
+#     32,768            243:215 / 340:286  258:229 / 624:359  573:266 / 3436:1368
 #   so below 10,000 neurons, where fewer workgroups share the events of a
 #   volley, up to one synapse per neuron for every 20 neurons of the block
-#   (6,000 x 400: 310:173 / 539:543).
+#   (6,000 x 400: 309:171 / 549:545).
 #   one step in a call:
 #     synapses per neuron        100               400               1,000
-#      2,000 neurons     28:31 / 31:34      30:31 / 34:38      33:31 / 42:45
+#      2,000 neurons     28:31 / 31:33      30:31 / 34:37      33:31 / 43:45
 #     10,000             29:31 / 34:33      35:32 / 40:37      42:32 / 51:42
-#     16,000             30:31 / 36:34      35:32 / 48:41      43:32 / 61:47
-#     32,768             32:38 / 41:42      38:39 / 71:52      47:40 / 85:58
-#   The launch, and its set-up of 6 us more above 16,384 neurons, are paid back
-#   by 8 steps of any of these blocks; shorter calls need the denser ones (the
-#   plain block of 10,000 x 100, which fires at the higher rate, among them).
+#     14,000             29:31 / 34:33      35:32 / 48:41      43:32 / 53:44
+#     18,000             30:37 / 35:40      36:38 / 49:44      44:39 / 71:49
+#     32,768             31:38 / 41:42      37:39 / 71:50      47:40 / 85:57
+#   The launch costs up to 3 us more than the per-step kernels' first step, 7
+#   above 16,384 neurons, which 8 and 16 steps of any of these blocks pay back;
+#   shorter calls need the denser ones (the plain block of 10,000 x 100, which
+#   fires at the higher rate, among them).
 # Building its copy of the synapses takes 0.3 to 1 ms up to 4 M synapses and
 # 5 ms for 32 M, so larger blocks run 200 steps first.
 PERSIST_N = (2000, 32 * 1024)
-PERSIST_CALL = 8
+PERSIST_CALL, PERSIST_CALL_LARGE = 8, 16
 PERSIST_NNZ, PERSIST_STEPS = 4_000_000, 200
 # Steps after a weight change that run on the per-step kernels: a program that
 # changes weights between steps should not pay for that copy each time.
@@ -181,8 +184,9 @@ class block:
 
     def _persist_pays(self, steps):
         per = self._nnz / self.N
-        if steps < PERSIST_CALL:
-            return self.N >= 10_000 and per >= (100 if self.N <= 16 * 1024 else 1000)
+        large = self.N > 16 * 1024
+        if steps < (PERSIST_CALL_LARGE if large else PERSIST_CALL):
+            return self.N >= 10_000 and per >= (1000 if large else 100)
         return self.N >= 10_000 or 20 * per <= self.N
 
     def _set_mode(self, steps, persist=True):

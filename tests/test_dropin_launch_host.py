@@ -41,7 +41,8 @@ def _block(n, per, refuse=None, src=None):
     (32_768, 100, 20, 3), (32_769, 100, 20, 0),
     # short calls: at the ends of the range the per-step kernels are the faster ones
     (2000, 20, 1, 0), (2000, 20, 7, 0), (2000, 20, 8, 3), (9_999, 400, 1, 0), (10_000, 100, 1, 3), (10_000, 99, 1, 0),
-    (16_384, 100, 1, 3), (16_385, 100, 1, 0), (32_768, 122, 1, 0),
+    (16_384, 100, 1, 3), (16_385, 100, 1, 0), (32_768, 122, 1, 0), (16_384, 20, 8, 3), (16_385, 20, 15, 0),
+    (16_385, 20, 16, 3),
 ])
 def test_calls_that_take_the_persistent_launch(n, per, steps, mode):
     b = _block(n, per)
