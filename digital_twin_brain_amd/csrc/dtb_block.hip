@@ -371,7 +371,7 @@ __device__ __forceinline__ void group_stats(const NeuronArgs& a, int32_t k, int 
     bool first = p >= 0;
     uint32_t c = 0;
     double v = 0.0;
-#pragma unroll
+#pragma unroll(W <= 4 ? W : 2)
     for (int x = 0; x < W; ++x) {
         const bool eq = s.pop[x] == p;
         if (x < w && eq) first = false;
@@ -2064,7 +2064,7 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
             const bool stats = a.rec_freq || a.rec_vsum;
             if (stats) wave_stats<4 * MB>(a, k, pp, act, vout, wid, s_stats);
             __syncthreads();
-            if (stats && threadIdx.x >= 64 && threadIdx.x < 64 + 4 * MB)
+            if (!RES && stats && threadIdx.x >= 64 && threadIdx.x < 64 + 4 * MB)
                 group_stats<4 * MB>(a, k, (int)threadIdx.x - 64, s_stats);
             uint32_t off = run, tot = 0;
             for (uint32_t w = 0; w < 4 * MB; ++w) {
@@ -2086,6 +2086,13 @@ __global__ __launch_bounds__(256 * MB) void persist_step_kernel(PersistArgs P)
             __hip_atomic_store(reinterpret_cast<uint64_t*>(P.pub + kPubStride * p),
                                ((uint64_t)step << 32) | run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+        // With one pass a step its statistics are added while wave 0 waits.
+        // Before the publication they were waited for, and unrolled over the
+        // 16 wavefronts of a workgroup they spilled up to 38 registers in
+        // batches without records too (100 steps of 30,000 x 100 at rest 741 us, now
+        // 616, with records 785 and 636).
+        if (RES && (a.rec_freq || a.rec_vsum) && threadIdx.x >= 64 && threadIdx.x < 64 + 4 * MB)
+            group_stats<4 * MB>(a, k, (int)threadIdx.x - 64, s_stats);
         // wait for every workgroup's word of this step (wave 0, one lane per
         // workgroup), then wave 0 builds the (delay, sub-list) entry prefix:
         // cum[e + 1] = spikes in entries <= e, e = (d - 1) * kSubLists + q
