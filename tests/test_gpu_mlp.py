@@ -334,6 +334,22 @@ def test_bias_grad_adds_in_row_order(M, N):
     assert float(db[N]) == 7.0
 
 
+# the kernel stages 256 rows at a time: one stage short of, at and past full, ragged ones
+# after full ones, beside column counts off its 64
+@pytest.mark.parametrize("M,N", [(255, 63), (256, 65), (257, 33), (300, 100), (511, 7), (512, 129), (513, 64)])
+def test_bias_grad_over_several_stages_of_rows(M, N):
+    g = torch.Generator().manual_seed(M * 3 + N)
+    dZ = torch.randn((M, N), generator=g)
+    d = dZ.cuda()
+    db = torch.full((N + 1,), 7.0, device="cuda")
+    nat.check(nat.lib().dtb_mlp_bias_grad(M, N, d.data_ptr(), db.data_ptr(), ctypes_stream()))
+    want = torch.zeros(N)
+    for row in dZ:
+        want += row
+    assert torch.equal(db[:N].cpu(), want)
+    assert float(db[N]) == 7.0
+
+
 # one layer; one 32-wide tile; widths of one, two and more tiles per wavefront; a batch whose
 # products are one chain over K (2048 x 512) beside ones split in four; wide inputs and outputs
 # (two output tiles a wavefront and a half-empty second round); rows at the edges of the 32-row tiles
