@@ -74,7 +74,7 @@ __device__ inline float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h <<
 // runs on XCD w mod 8): each XCD takes a contiguous run of tiles, ordered in
 // bands of GM tile rows, column by column, so that the tiles it has in flight
 // form a near-square block and share their slices in its L2.
-// 8192^3: 1136 -> 859 us (1.28 PFLOP/s; matrix pipe busy 74% of the cycles, no
+// 8192^3: 1110 -> 830 us a call (1.32 PFLOP/s; matrix pipe busy 74% of the cycles, no
 // LDS bank conflicts); 960 x 960 x 6144: 112 -> 39 us; 992 x 4160 x 3008 (no
 // multiples of 128): 181 -> 44 us.
 __device__ __forceinline__ void lds_dma16(const uint16_t* src, uint32_t lds_byte)
@@ -1618,7 +1618,8 @@ using GruBwdWeights = GruWeights<(2 * G + kGruBwdWaves - 1) / kGruBwdWaves, 3 * 
 //   128x128 tiles once every CU gets one (2048^2: 64x64 29.4, 128x128 23.8;
 //     1536^2 K = 1536, 144 tiles: 15.5, 17.0);
 //   256x256 tiles, one a CU and 1.75 times the time of a round of 128x128
-//     tiles, two a CU, where that many fewer rounds do (8192^3: 808 against
+//     tiles, two a CU, where that many fewer rounds do (best of several back
+//     to back, 8192^3: 808 against
 //     1033; 5024 x 1632 K = 2000: 51 against 59; 6144^3, 2.25 rounds: 426
 //     against 416);
 //   a short K is bound by the stores of C, which several workgroups a CU
