@@ -4869,7 +4869,8 @@ int dtb_block_set_launch(dtb_block* b, int32_t what, int32_t value)
                     "delivery mode must be 0 (atomics), 1 (bucketed), 2 or 3 (persistent, small blocks)");
         if (value >= 1) DTB_TRY(ensure_bucketed(b));
         if (value >= 2) DTB_TRY(ensure_persist(b, value == 3));
-        if (value == 2) b->accum_fixed = true; // batches that fall back to bucketed kernels sum as the persistent launch does
+        // batches that fall back to the bucketed kernels sum as the persistent launch does
+        if (value == 2) b->accum_fixed = true;
         b->deliver_mode = value;
         return DTB_OK; // part of the graphs' key: a program that switches back finds its graphs
     } else {
